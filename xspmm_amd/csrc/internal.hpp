@@ -120,6 +120,11 @@ public:
     TempArena& operator=(const TempArena&) = delete;
     bool fixed() const { return base_ != nullptr; }
     size_t capacity() const { return cap_; }
+    // whether take(bytes) has room for them
+    bool fits(size_t bytes) const {
+        const size_t at = (used_ + 255) & ~size_t(255);
+        return !base_ || (at <= cap_ && bytes <= cap_ - at);
+    }
     void* take(size_t bytes) {
         if (bytes == 0) return nullptr;
         if (!base_) {
@@ -285,12 +290,16 @@ bool spmm_f16_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, c
 
 // Tier-1 fp32 column-batch SpMM (spmm_f32.hip): covers N % 4 == 0 with B and
 // C 16-byte aligned, K * N * 4 <= 2^31 and Kb < 2^21 (XSPMM_F32_KERNEL=tile
-// declines it); order and row_map as for bcsr_spmm_ex.
+// declines it); order and row_map as for bcsr_spmm_ex.  With nc > 0, B is a
+// copy padded to N columns, C has nc (any alignment) and nonfinite holds the
+// copy's 256 bytes of Inf / NaN marks: when one is set, every column of a block
+// is multiplied, so that B meets each row as in the reference.
 bool spmm_f32_batch_covers(int64_t K, int64_t Kb, int64_t N, const void* B, const void* C);
 template <typename I>
 void bcsr_spmm_f32_batch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                          const float* bvals, const float* B, float* C, int64_t N,
-                         const int32_t* order, const I* row_map, hipStream_t s);
+                         const int32_t* order, const I* row_map, hipStream_t s, int64_t nc = 0,
+                         const uint32_t* nonfinite = nullptr);
 // Packed fp32 column batches (csr_pack_emit with V = uint32_t): strip br's
 // batches [offsets[br], offsets[br + 1]) (a multiple of 4), A' in a and row
 // indices in rows; order and row_map as for bcsr_spmm_ex.  Returns false
@@ -306,17 +315,19 @@ bool spmm_f32_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, c
 // its block-rows hold the canonical layout (block br * Kb + c has column c)
 // and otherwise multiplies its blocks in stored order, so any block order
 // gives the right C.  Returns false (and launches nothing) when the shape is
-// not covered; spmm_dense_f16_covers tells in advance.
+// not covered; spmm_dense_f16_covers tells in advance.  nc > 0: C has nc <= N
+// columns (B padded to N).
 bool spmm_dense_f16_covers(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N);
 template <typename I>
 bool bcsr_spmm_dense_f16(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb,
                          const I* brp, const I* bci, const uint16_t* bvals, const uint16_t* B,
-                         float* C, int64_t N, hipStream_t s, const I* row_map);
+                         float* C, int64_t N, hipStream_t s, const I* row_map, int64_t nc = 0);
 
 // Tier-1 fp16 SpMM for grids whose block-rows are contiguous runs of block
 // columns (banded grids): four neighbouring block-rows share each B tile.
 // Only correct when every block-row is contiguous; spmm_band_f16_covers tells
-// whether the shape is covered (false: nothing launched).
+// whether the shape is covered (false: nothing launched).  nc > 0: C has
+// nc <= N columns (B padded to N).
 bool spmm_band_f16_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N);
 // Tier-1 fp32 SpMM for banded grids (contiguous block-rows): four
 // neighbouring block-rows per workgroup share each B load in registers.
@@ -343,7 +354,7 @@ bool spmm_band_wanted(const I* brp, const I* bci, int64_t M, int64_t K, int64_t 
 template <typename I>
 bool bcsr_spmm_band_f16(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const uint16_t* bvals, const uint16_t* B, float* C, int64_t N,
-                        const I* row_map, hipStream_t s);
+                        const I* row_map, hipStream_t s, int64_t nc = 0);
 
 // CSR -> BCSR.  count writes brp[Mb+1] and returns nnzb (synchronizes `s`);
 // it throws std::invalid_argument on an out-of-range column index.

@@ -16,8 +16,11 @@
 //                           spmm_f16_packed_kernel (prepared products);
 //   spmm_f16_dense_kernel   (spmm_dense.hip) fully populated block grids;
 //   spmm_f16_gather_kernel  per-pair masked B-row gather (XSPMM_SPMM_KERNEL=gather);
-//   pack_b_panels + spmm_f16_kernel  any N: B repacked into 16-row panels laid
-//                           out [block_col][n][k16], two blocks per K = 32 operand.
+//   pack_b_panels + spmm_f16_kernel  B repacked into 16-row panels laid out
+//                           [block_col][n][k16], two blocks per K = 32 operand:
+//                           B beyond 2^31 bytes, or no room for a padded copy.
+// N % 8 != 0 (fp32: N % 4 != 0, or B or C off 16 bytes): the same kernels on a
+// copy of B with padded rows (pad_b_kernel).
 //
 // fp32 kernels.  v_mfma_f32_16x16x4f32 takes one k per lane, so B is read
 // row-major directly:
@@ -37,6 +40,7 @@
 #include <cstdlib>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "internal.hpp"
 #include "scan.hpp"
@@ -56,6 +60,47 @@ __device__ __forceinline__ half8_t load_h8(const uint16_t* p)
 {
     u32x4_t v = *reinterpret_cast<const u32x4_t*>(p);
     return __builtin_bit_cast(half8_t, v);
+}
+
+// ---------------------------------------------------------------------------
+// B (K x N) -> Bp (K x Np, Np = N rounded up to a 16-byte row multiple, the
+// added columns zero), for products whose rows do not start on 16 bytes: the
+// kernels that read B rows 16 bytes at a time then cover every N.  Bound by
+// memory (one read and one write of B): 3.2 us at 4999 x 31.
+// marks[0 .. 64) (256 bytes, all written): byte i is set when workgroup i of
+// the (at most 256) met an Inf or NaN.
+// ---------------------------------------------------------------------------
+constexpr int kPadMarks = 256;
+constexpr int kPadThreads = 256;
+template <typename U>
+__global__ __launch_bounds__(kPadThreads) void pad_b_kernel(const U* __restrict__ B, U* __restrict__ Bp,
+                                                            int64_t K, int64_t N, int64_t Np,
+                                                            unsigned char* __restrict__ marks)
+{
+    constexpr int V = 16 / (int)sizeof(U);
+    constexpr U kExp = sizeof(U) == 2 ? (U)0x7c00u : (U)0x7f800000u;
+    // K * Np * sizeof(U) <= 2^31: vector counts fit 32 bits
+    const uint32_t per_row = (uint32_t)(Np / V);
+    const uint32_t total = (uint32_t)K * per_row;
+    bool bad = false;
+    for (uint32_t t = blockIdx.x * kPadThreads + threadIdx.x; t < total; t += gridDim.x * kPadThreads) {
+        const uint32_t k = t / per_row;
+        const int64_t c = (int64_t)(t - k * per_row) * V;
+        const U* src = B + k * N + c;
+        typedef U vec_t __attribute__((ext_vector_type(V)));
+        vec_t v;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            v[e] = c + e < N ? src[e] : (U)0;
+            bad |= (v[e] & kExp) == kExp;
+        }
+        *reinterpret_cast<vec_t*>(Bp + (size_t)t * V) = v;
+    }
+    const int any = __syncthreads_or(bad ? 1 : 0);
+    if (threadIdx.x == 0) marks[blockIdx.x] = any ? 1 : 0;
+    // the bytes of workgroups that the grid does not have
+    if (blockIdx.x == 0)
+        for (int i = (int)gridDim.x + threadIdx.x; i < kPadMarks; i += kPadThreads) marks[i] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -651,6 +696,8 @@ struct BatchPack {
     const int64_t* offsets;   // kPack: first batch of (block-row, wave)
     u32x4_t* a;               // kPack: A' operands
     uint32_t* rows;           // kPack: B-row indices
+    int64_t nc = 0;                       // EX: columns of C (B is padded to N)
+    const uint32_t* nonfinite = nullptr;  // EX: pad_b_kernel's marks
 };
 
 // Sum the kBW waves' partial 16 x (16 NT) tiles through LDS (in wave order)
@@ -717,6 +764,46 @@ __device__ __forceinline__ constexpr uint32_t kslot(uint32_t k)
     return 16u * ((k >> 2) & 1u) + 4u * (k >> 3) + (k & 3u);
 }
 
+// The 16 x (16 NT) tile of block-row br from column n0 on, every block whole
+// and in stored order (reference src/common/spmm_math.hpp:68-114): wave w takes
+// column tiles w, w + kBW, ...  B has rows of N columns, C of nc.  Only
+// products with a non-finite value in A or B come here.
+template <typename I, int NT>
+__device__ void batch_row_exact(const I* __restrict__ brp, const I* __restrict__ bci,
+                                const uint16_t* __restrict__ vals, const uint16_t* __restrict__ B,
+                                float* __restrict__ C, int64_t M, int64_t K, int64_t N, int64_t nc,
+                                int64_t Kb, int64_t br, int64_t n0, const I* __restrict__ row_map)
+{
+    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & (kWave - 1);
+    const int li = lane & 15;
+    const int g = lane >> 4;
+    const _Float16* const Bh = reinterpret_cast<const _Float16*>(B);
+    for (int j = (int)(threadIdx.x / kWave); j < NT; j += kBW) {
+        const int64_t n = n0 + 16 * j + li;
+        float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
+        const int64_t be = (int64_t)brp[br + 1];
+        for (int64_t b = (int64_t)brp[br]; b < be; ++b) {
+            const int64_t col = (int64_t)bci[b];
+            if (col < 0 || col >= Kb) continue;
+            const half4_t a = *reinterpret_cast<const half4_t*>(vals + b * 256 + li * 16 + 4 * g);
+            half4_t bo;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int64_t k = 16 * col + 4 * g + s;
+                bo[s] = (k < K && n < N) ? Bh[k * N + n] : (_Float16)0.f;
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a, bo, acc, 0, 0, 0);
+        }
+        if (n >= nc) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t row = 16 * br + 4 * g + q;
+            if (row < M) C[(row_map ? (int64_t)row_map[row] : row) * nc + n] = acc[q];
+        }
+    }
+}
+
 // NC: 128-column chunks one workgroup multiplies each batch with (1, or 2
 // for N > 128: each pair is streamed and compacted once for 256 columns).
 // The chunks' products accumulate exactly as two NC = 1 workgroups would,
@@ -725,11 +812,19 @@ __device__ __forceinline__ constexpr uint32_t kslot(uint32_t k)
 // (HIP's second __launch_bounds__ argument is the minimum number of waves per
 // SIMD: kBW for four resident workgroups per CU, kBW / 2 for two.)
 //
+// EX (N % 8 != 0): B is pad_b_kernel's copy with rows of N columns, C has pk.nc
+// of them.  The reference multiplies every column of a block, so an Inf or NaN
+// in B reaches rows whose block only covers it, and an Inf in A keeps its
+// sign; skipping zero columns and compacting by one-hot products would lose
+// both.  A workgroup that meets a non-finite value (B: the pad kernel's marks;
+// A: 0 * A' is not 0 in some batch) discards its tile and multiplies the
+// block-row's blocks whole (batch_row_exact).
+//
 // XM (two 128-column chunks, Mb % 4 == 0, grid (2 Mb, 1)): workgroup l runs
 // chunk (l / 4) % 2 of block-row 4 (l / 8) + l % 4, so (workgroups going to
 // the 8 XCDs round-robin) XCDs 0-3 take the first chunk and XCDs 4-7 the
 // second, and each XCD's L2 holds half of B's columns instead of all of them.
-template <typename I, int NT, BatchMode MODE = BatchMode::kMultiply, int NC = 1, bool XM = false>
+template <typename I, int NT, BatchMode MODE = BatchMode::kMultiply, int NC = 1, bool XM = false, bool EX = false>
 __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_batch_kernel(
     const I* __restrict__ brp, const I* __restrict__ bci, const uint16_t* __restrict__ vals,
     const uint16_t* __restrict__ B, float* __restrict__ C, int64_t M, int64_t K, int64_t N,
@@ -762,6 +857,7 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
         return c == 0 ? W : W + kBatchWaveLds + (c - 1) * kBtBytes;
     };
 
+    static_assert(!EX || (NC == 1 && !XM && MODE == BatchMode::kMultiply), "padded B: one chunk per workgroup");
     static_assert(!XM || (NC == 1 && NT == 8 && MODE == BatchMode::kMultiply), "XCD chunk map: two 128-column chunks");
     const uint32_t bx = XM ? (((blockIdx.x >> 3) << 2) | (blockIdx.x & 3u)) : blockIdx.x;
     const uint32_t by = XM ? ((blockIdx.x >> 2) & 1u) : blockIdx.y;
@@ -852,6 +948,7 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
     half8_t aop{};
     bool started = false;
     uint32_t pending = 0;
+    float inexact = 0.f;  // EX: 0 while every A' value is finite, else NaN
 
     auto finish = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -906,6 +1003,10 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
             }
             ++nbatch;
             return;
+        }
+        if constexpr (EX) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) inexact = __builtin_fmaf((float)a[e], 0.f, inexact);
         }
         if (started) finish();
         aop = a;
@@ -1099,10 +1200,28 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
     } else if constexpr (MODE == BatchMode::kPack) {
         return;
     } else {
+        if constexpr (EX) {
+            // the waves' answers through smem, not __syncthreads_or: with a
+            // second LDS object in the kernel the compiler takes the tile's
+            // reads not to alias the direct-to-LDS loads and leaves out the
+            // wait between them
+            const uint64_t bad = __builtin_amdgcn_ballot_w64(pk.nonfinite[lane] != 0u || inexact != 0.f);
+            uint32_t* const ws = reinterpret_cast<uint32_t*>(smem);
+            __syncthreads();
+            if (lane == 0) ws[wave] = bad != 0u ? 1u : 0u;
+            __syncthreads();
+            uint32_t any = 0;
+#pragma unroll
+            for (int w = 0; w < kBW; ++w) any |= ws[w];
+            if (any) {
+                batch_row_exact<I, NT>(brp, bci, vals, B, C, M, K, N, pk.nc, Kb, br, n0, row_map);
+                return;
+            }
+        }
 #pragma unroll
         for (int c = 0; c < NC; ++c)
             if (n0 + 128 * c < N)
-                batch_tile_store<I, NT>(acc[c], smem, wave, g, li, br, n0 + 128 * c, M, N, C,
+                batch_tile_store<I, NT>(acc[c], smem, wave, g, li, br, n0 + 128 * c, M, EX ? pk.nc : N, C,
                                         row_map);
     }
 }
@@ -1735,6 +1854,43 @@ template bool spmm_dispatch_order_cols<int64_t>(const int64_t*, const int64_t*, 
 
 namespace {
 
+// B with rows of Np columns (N rounded up to 16 bytes) and its marks, made on
+// the stream by pad_b_kernel, and room for order_rows int32, all one piece of
+// the arena (an allocation costs the host about 15 us); bt null when a fixed
+// arena has no room for it.
+template <typename T>
+struct PaddedB {
+    const T* bt = nullptr;
+    const uint32_t* marks = nullptr;
+    int32_t* order = nullptr;
+    int64_t Np = 0;
+};
+
+template <typename T>
+PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena& arena, hipStream_t s)
+{
+    using U = std::conditional_t<sizeof(T) == 2, uint16_t, uint32_t>;
+    constexpr int64_t V = 16 / (int64_t)sizeof(T);
+    PaddedB<T> p;
+    p.Np = (N + V - 1) / V * V;
+    Carve cv;
+    const size_t o_marks = cv.take(kPadMarks);
+    const size_t o_bt = cv.take((size_t)(K > 0 ? K : 1) * (size_t)p.Np * sizeof(T));
+    const size_t o_order = cv.take((size_t)order_rows * sizeof(int32_t));
+    if (!arena.fits(cv.end)) return p;
+    char* const base = static_cast<char*>(arena.take(cv.end));
+    const int64_t vecs = K * (p.Np / V);
+    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads));
+    hipLaunchKernelGGL((pad_b_kernel<U>), dim3((unsigned)wgs), dim3(kPadThreads), 0, s,
+                       reinterpret_cast<const U*>(B), reinterpret_cast<U*>(base + o_bt), K, N, p.Np,
+                       reinterpret_cast<unsigned char*>(base + o_marks));
+    XSPMM_LAUNCH_CHECK();
+    p.bt = reinterpret_cast<const T*>(base + o_bt);
+    p.marks = reinterpret_cast<const uint32_t*>(base + o_marks);
+    p.order = reinterpret_cast<int32_t*>(base + o_order);
+    return p;
+}
+
 // The Tier-1 launcher: kernel choice as described at the top of this file;
 // temporaries (the dispatch order, repacked B panels) come from `arena`.
 template <typename T, typename I>
@@ -1799,6 +1955,47 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             XSPMM_LAUNCH_CHECK();
             return true;
         }
+        // N % 8 != 0: rows of B off 16 bytes.  The kernels above, on a padded
+        // copy of B, instead of the panel kernel below, which repacks B just
+        // the same and whose waves then walk whole block-rows alone.  Faster
+        // on every matrix and N tried (1 .. 127): 16384^2 templates, N = 17,
+        // 342 -> 77 us; 50000^2 power-law graph, N = 1, 867 -> 104 us;
+        // 5003 x 4999 at 2 %, N = 31, 96 -> 29 us; 8192^2 with 5 % of the
+        // blocks, N = 7, 24 -> 23 us.
+        const int64_t Np = (N + 7) / 8 * 8;
+        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && N % 8 != 0 &&
+            K * Np * 2 <= (int64_t(1) << 31) && Np < (int64_t(1) << 22) && Kb < (int64_t(1) << 20)) {
+            const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, Np);
+            const bool own_order = !full && !order_in && spmm_order_wanted(Mb);
+            const PaddedB<uint16_t> pb = pad_b<uint16_t>(b, K, N, own_order ? Mb : 0, arena, s);
+            if (pb.bt) {
+                if (full)
+                    return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
+                const int32_t* order = order_in;
+                if (own_order) {
+                    spmm_dispatch_order<I>(brp, Mb, pb.order, s);
+                    order = pb.order;
+                }
+                BatchPack pk{};
+                pk.nc = N;
+                pk.nonfinite = pb.marks;
+                auto launch = [&](auto nt) {
+                    hipLaunchKernelGGL((spmm_f16_batch_kernel<I, decltype(nt)::value, BatchMode::kMultiply, 1, false, true>),
+                                       ggrid, dim3(64 * kBW), 0, s, brp, bci, v, pb.bt, C, M, K, Np, Kb, order,
+                                       row_map, pk);
+                };
+                if (N <= 16)
+                    launch(std::integral_constant<int, 1>{});
+                else if (N <= 32)
+                    launch(std::integral_constant<int, 2>{});
+                else if (N <= 64)
+                    launch(std::integral_constant<int, 4>{});
+                else
+                    launch(std::integral_constant<int, 8>{});
+                XSPMM_LAUNCH_CHECK();
+                return true;
+            }
+        }
         if (row_map) return false;  // the other fp16 kernels store rows in place
         if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32) {
             if (N <= 64)
@@ -1810,26 +2007,26 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             XSPMM_LAUNCH_CHECK();
             return true;
         }
-        const int64_t Np = ntiles64 * 16;
-        uint16_t* bt = arena.take_as<uint16_t>((size_t)(Kb > 0 ? Kb : 1) * (size_t)Np * 16);
+        const int64_t Nw = ntiles64 * 16;
+        uint16_t* bt = arena.take_as<uint16_t>((size_t)(Kb > 0 ? Kb : 1) * (size_t)Nw * 16);
         if (Kb > 0) {
-            const int64_t per_kb = Np * 2;
+            const int64_t per_kb = Nw * 2;
             const dim3 pg((unsigned)((per_kb + 255) / 256), (unsigned)(Kb < 65535 ? Kb : 65535));
-            hipLaunchKernelGGL(pack_b_panels, pg, dim3(256), 0, s, b, bt, K, N, Kb, Np);
+            hipLaunchKernelGGL(pack_b_panels, pg, dim3(256), 0, s, b, bt, K, N, Kb, Nw);
             XSPMM_LAUNCH_CHECK();
         }
         switch (geo.ntw) {
         case 4:
             hipLaunchKernelGGL((spmm_f16_kernel<I, 4>), grid, block, 0, s, brp, bci, v, bt, C, M,
-                               N, Np, Kb, ntiles);
+                               N, Nw, Kb, ntiles);
             break;
         case 2:
             hipLaunchKernelGGL((spmm_f16_kernel<I, 2>), grid, block, 0, s, brp, bci, v, bt, C, M,
-                               N, Np, Kb, ntiles);
+                               N, Nw, Kb, ntiles);
             break;
         default:
             hipLaunchKernelGGL((spmm_f16_kernel<I, 1>), grid, block, 0, s, brp, bci, v, bt, C, M,
-                               N, Np, Kb, ntiles);
+                               N, Nw, Kb, ntiles);
             break;
         }
         XSPMM_LAUNCH_CHECK();
@@ -1848,6 +2045,28 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             }
             bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, b, C, N, order, row_map, s);
             return true;
+        }
+        // N % 4 != 0, or B or C off 16 bytes: the column batches on a padded
+        // copy of B, from 2^18 products of a block with a 16-column tile, where
+        // they make up for the copy (N = 17: 300980 blocks 123 -> 80 us, 97367
+        // blocks 43 -> 58 us; N = 33: 97367 blocks 71 -> 58, 14465 blocks
+        // 14 -> 24).  One tile (N <= 16) stays below, where a block costs one
+        // B load whatever its fill (N = 1: 367862 blocks of 5 columns 105 us,
+        // 151 in batches).
+        const int64_t Np = (N + 3) / 4 * 4;
+        if (spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr) &&
+            (f32_kernel_forced_batch() || (N > 16 && nnzb * ntiles64 >= (int64_t(1) << 18)))) {
+            const bool own_order = !order_in && spmm_order_wanted(Mb);
+            const PaddedB<float> pb = pad_b<float>(b, K, N, own_order ? Mb : 0, arena, s);
+            if (pb.bt) {
+                const int32_t* order = order_in;
+                if (own_order) {
+                    spmm_dispatch_order<I>(brp, Mb, pb.order, s);
+                    order = pb.order;
+                }
+                bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order, row_map, s, N, pb.marks);
+                return true;
+            }
         }
         if (row_map) return false;  // the fp32 tile kernel stores rows in place
         // 16-column tiles per wave: 4 (fewer B loads per block) unless that
@@ -1958,6 +2177,13 @@ void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
     check_alignment(bvals, B, sizeof(T) == 2);
     if constexpr (sizeof(T) == 2) {
         if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, s)) return;
+        // N % 8 != 0: on a padded copy of B
+        const int64_t Np = (N + 7) / 8 * 8;
+        if (spmm_band_f16_covers(K, Kb, Mb, Np)) {
+            TempArena arena(s);
+            const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K, N, 0, arena, s);
+            if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, pb.bt, C, Np, nullptr, s, N)) return;
+        }
     } else {
         if (bcsr_spmm_band_f32<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, nnzb, s)) return;
     }

@@ -123,13 +123,14 @@ __device__ __forceinline__ void band_barrier_writes()
     asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(R) : "memory");
 }
 
+// nc: columns of C (at most N; fewer when B is a copy with padded rows).
 // WPR: waves per block-row (1: a wave owns its row's 128 columns; 2: two
 // waves split them, 8 waves per workgroup, two per SIMD).
 template <typename I, int L, int WPR>
 __global__ __launch_bounds__(64 * kBandRows * WPR) void spmm_f16_band_kernel(
     const I* __restrict__ brp, const I* __restrict__ bci, const uint16_t* __restrict__ vals,
     const uint16_t* __restrict__ B, float* __restrict__ C, int64_t M, int64_t K, int64_t N,
-    int64_t Mb, const I* __restrict__ row_map)
+    int64_t Mb, const I* __restrict__ row_map, int64_t nc)
 {
     static_assert(WPR == 1 || WPR == 2, "one or two waves per block-row");
     static_assert(L % 6 == 0, "ring depth a multiple of 6 (ring slot, stage and operand set align)");
@@ -316,10 +317,10 @@ __global__ __launch_bounds__(64 * kBandRows * WPR) void spmm_f16_band_kernel(
             if (grow >= M) continue;
             const int64_t crow = row_map ? (int64_t)row_map[grow] : grow;
             const int64_t c0 = n0 + 16 * cs * NT + li;
-            float* dst = C + crow * N + c0;
+            float* dst = C + crow * nc + c0;
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                if (c0 + 16 * j < N) dst[16 * j] = acc[j][q];
+                if (c0 + 16 * j < nc) dst[16 * j] = acc[j][q];
         }
     }
 }
@@ -806,13 +807,13 @@ bool spmm_band_f16_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N)
 template <typename I>
 bool bcsr_spmm_band_f16(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const uint16_t* bvals, const uint16_t* B, float* C, int64_t N,
-                        const I* row_map, hipStream_t s)
+                        const I* row_map, hipStream_t s, int64_t nc)
 {
     if (!spmm_band_f16_covers(K, Kb, Mb, N)) return false;
     const dim3 grid((unsigned)((Mb + kBandRows - 1) / kBandRows), (unsigned)((N + 127) / 128));
     hipLaunchKernelGGL((spmm_f16_band_kernel<I, XSPMM_BAND_DEPTH, XSPMM_BAND_WPR>), grid,
                        dim3(64 * kBandRows * XSPMM_BAND_WPR), 0, s, brp, bci, bvals, B, C, M, K, N, Mb,
-                       row_map);
+                       row_map, nc > 0 ? nc : N);
     XSPMM_LAUNCH_CHECK();
     return true;
 }
@@ -931,10 +932,10 @@ template bool bcsr_spmm_band_f32<int64_t>(int64_t, int64_t, int64_t, int64_t, co
 
 template bool bcsr_spmm_band_f16<int32_t>(int64_t, int64_t, int64_t, int64_t, const int32_t*,
                                           const int32_t*, const uint16_t*, const uint16_t*, float*,
-                                          int64_t, const int32_t*, hipStream_t);
+                                          int64_t, const int32_t*, hipStream_t, int64_t);
 template bool bcsr_spmm_band_f16<int64_t>(int64_t, int64_t, int64_t, int64_t, const int64_t*,
                                           const int64_t*, const uint16_t*, const uint16_t*, float*,
-                                          int64_t, const int64_t*, hipStream_t);
+                                          int64_t, const int64_t*, hipStream_t, int64_t);
 
 }  // namespace detail
 }  // namespace xspmm

@@ -171,7 +171,7 @@ __device__ void dense_tile_generic(const I* __restrict__ brp, const I* __restric
                                    const uint16_t* __restrict__ vals, const uint16_t* __restrict__ B,
                                    float* __restrict__ C, int64_t M, int64_t K, int64_t N,
                                    int64_t Mb, int64_t Kb, int64_t br0, int rows, int64_t n0,
-                                   const I* __restrict__ row_map)
+                                   const I* __restrict__ row_map, int64_t nc)
 {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -205,13 +205,13 @@ __device__ void dense_tile_generic(const I* __restrict__ brp, const I* __restric
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int64_t n = n0 + 16 * j + li;
-            if (n >= N) continue;
+            if (n >= nc) continue;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int64_t row = 16 * br + 4 * g + q;
                 if (row >= M) continue;
                 const int64_t crow = row_map ? (int64_t)row_map[row] : row;
-                C[crow * N + n] = acc[j][q];
+                C[crow * nc + n] = acc[j][q];
             }
         }
     }
@@ -219,7 +219,7 @@ __device__ void dense_tile_generic(const I* __restrict__ brp, const I* __restric
 
 // RW: block-rows per wave (8: 256-row tiles; 7: 224-row tiles, whose A stage
 // rows 14 and 15 load as zeros).  I: index type of brp / bci and of the
-// optional output row map (C row row_map[r] receives product row r -- the
+// optional output row map (nc: columns of C, at most N; C row row_map[r] receives product row r -- the
 // clustered pipeline's un-permutation fused into the store; null stores rows
 // in place).
 template <int RW, typename I>
@@ -231,7 +231,8 @@ __global__ __launch_bounds__(kDThreads, XSPMM_DENSE_MINW) void spmm_f16_dense_ke
                                                                  int64_t M, int64_t K,
                                                                  int64_t N, int64_t Mb,
                                                                  int64_t Kb,
-                                                                 const I* __restrict__ row_map)
+                                                                 const I* __restrict__ row_map,
+                                                                 int64_t nc)
 {
     constexpr int NS = XSPMM_DENSE_STAGES;
     constexpr int kDR = kWR * RW;  // block-rows per workgroup
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(kDThreads, XSPMM_DENSE_MINW) void spmm_f16_dense_ke
     {
         const int rows = (int)(Mb - br0 < kDR ? Mb - br0 : kDR);
         if (!tile_is_canonical<I>(brp, bci, br0, rows, Kb)) {
-            dense_tile_generic<I>(brp, bci, vals, B, C, M, K, N, Mb, Kb, br0, rows, n0, row_map);
+            dense_tile_generic<I>(brp, bci, vals, B, C, M, K, N, Mb, Kb, br0, rows, n0, row_map, nc);
             return;
         }
     }
@@ -431,12 +432,12 @@ __global__ __launch_bounds__(kDThreads, XSPMM_DENSE_MINW) void spmm_f16_dense_ke
                 const int c = col_l + 4 * TPR * p;
                 const float4_t v = *reinterpret_cast<const float4_t*>(T + row_l * TS + c);
                 const int64_t col = n0 + c;
-                if (row < M && col < N) {
+                if (row < M && col < nc) {
                     // 16-byte stores only where C's rows stay 16-byte aligned
-                    if (col + 4 <= N && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0)
-                        __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(C + crow * N + col));
+                    if (col + 4 <= nc && (nc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0)
+                        __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(C + crow * nc + col));
                     else
-                        for (int e = 0; e < 4 && col + e < N; ++e) C[crow * N + col + e] = v[e];
+                        for (int e = 0; e < 4 && col + e < nc; ++e) C[crow * nc + col + e] = v[e];
                 }
             }
             __syncthreads();
@@ -448,15 +449,15 @@ __global__ __launch_bounds__(kDThreads, XSPMM_DENSE_MINW) void spmm_f16_dense_ke
 #pragma unroll
             for (int j = 0; j < kDTiles; ++j) {
                 const int64_t col = n0 + 16 * kDTiles * wc + 16 * j + li;
-                if (col >= N) continue;
+                if (col >= nc) continue;
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (row0 + q < M) {
                         const int64_t crow = row_map ? (int64_t)row_map[row0 + q] : row0 + q;
                         if constexpr (XSPMM_DENSE_EPI == 1)
-                            __builtin_nontemporal_store(acc[r][j][q], C + crow * N + col);
+                            __builtin_nontemporal_store(acc[r][j][q], C + crow * nc + col);
                         else
-                            C[crow * N + col] = acc[r][j][q];
+                            C[crow * nc + col] = acc[r][j][q];
                     }
             }
         }
@@ -522,17 +523,18 @@ bool spmm_dense_f16_covers(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t
 template <typename I>
 bool bcsr_spmm_dense_f16(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb,
                          const I* brp, const I* bci, const uint16_t* bvals, const uint16_t* B,
-                         float* C, int64_t N, hipStream_t s, const I* row_map)
+                         float* C, int64_t N, hipStream_t s, const I* row_map, int64_t nc)
 {
+    if (nc <= 0) nc = N;
     if (!spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, N)) return false;
     const int h = dense_tile_rows(Mb, N);
     const int64_t groups = dense_groups(Mb, N, h);
     if (h == 14)
         hipLaunchKernelGGL((spmm_f16_dense_kernel<7, I>), dim3((unsigned)groups), dim3(kDThreads), 0,
-                           s, brp, bci, bvals, B, C, M, K, N, Mb, Kb, row_map);
+                           s, brp, bci, bvals, B, C, M, K, N, Mb, Kb, row_map, nc);
     else
         hipLaunchKernelGGL((spmm_f16_dense_kernel<8, I>), dim3((unsigned)groups), dim3(kDThreads), 0,
-                           s, brp, bci, bvals, B, C, M, K, N, Mb, Kb, row_map);
+                           s, brp, bci, bvals, B, C, M, K, N, Mb, Kb, row_map, nc);
     XSPMM_LAUNCH_CHECK();
     return true;
 }
@@ -540,11 +542,11 @@ bool bcsr_spmm_dense_f16(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t n
 template bool bcsr_spmm_dense_f16<int32_t>(int64_t, int64_t, int64_t, int64_t, int64_t,
                                            const int32_t*, const int32_t*, const uint16_t*,
                                            const uint16_t*, float*, int64_t, hipStream_t,
-                                           const int32_t*);
+                                           const int32_t*, int64_t);
 template bool bcsr_spmm_dense_f16<int64_t>(int64_t, int64_t, int64_t, int64_t, int64_t,
                                            const int64_t*, const int64_t*, const uint16_t*,
                                            const uint16_t*, float*, int64_t, hipStream_t,
-                                           const int64_t*);
+                                           const int64_t*, int64_t);
 
 }  // namespace detail
 }  // namespace xspmm

@@ -128,11 +128,16 @@ __device__ __forceinline__ uint64_t columns_below(uint32_t lim)
 // NQ: 64-column quads per workgroup (one 16-byte B load per quad and batch
 // slot); W: waves per workgroup; D: blocks per ring pass (in flight per
 // wave); F: batches taken from the column queue per pass.
-template <typename I, int NQ, int W, int D, int F>
+// EX: B is a copy padded to N columns, C has nc (any alignment), and
+// nonfinite holds 256 bytes of marks: when one is set, an Inf or NaN of B must
+// reach every row whose block covers it (the reference multiplies whole
+// blocks), so no column is skipped.
+template <typename I, int NQ, int W, int D, int F, bool EX>
 __global__ __launch_bounds__(64 * W, (W <= 4 ? 16 / W : 1)) void spmm_f32_batch_kernel(
     const I* __restrict__ brp, const I* __restrict__ bci, const float* __restrict__ vals,
     const float* __restrict__ B, float* __restrict__ C, int64_t M, int64_t K, int64_t N,
-    int64_t Kb, const int32_t* __restrict__ order, const I* __restrict__ row_map)
+    int64_t Kb, const int32_t* __restrict__ order, const I* __restrict__ row_map, int64_t nc,
+    const uint32_t* __restrict__ nonfinite)
 {
     static_assert(NQ == 1 || NQ == 2, "64 or 128 columns per workgroup");
     static_assert(D >= 2 && D <= 8, "2 .. 8 blocks per ring pass");
@@ -216,6 +221,8 @@ __global__ __launch_bounds__(64 * W, (W <= 4 ? 16 / W : 1)) void spmm_f32_batch_
         for (int q = 0; q < NQ; ++q) bq[f][q] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
     uint32_t inflight = 0;  // batches held in ap / bq (wave-uniform)
+    bool whole = false;     // multiply every column (wave-uniform)
+    if constexpr (EX) whole = __builtin_amdgcn_ballot_w64(nonfinite[lane] != 0u) != 0;
 
     auto multiply = [&](const float a, const float4_t (&b)[NQ]) __attribute__((always_inline)) {
 #pragma unroll
@@ -293,6 +300,8 @@ __global__ __launch_bounds__(64 * W, (W <= 4 ? 16 / W : 1)) void spmm_f32_batch_
                                  __builtin_amdgcn_ballot_w64(P[1] != 0.f),
                                  __builtin_amdgcn_ballot_w64(P[2] != 0.f),
                                  __builtin_amdgcn_ballot_w64(P[3] != 0.f));
+        if constexpr (EX)
+            if (whole) m = kAllColumns;
         // a block column outside the grid (malformed input) contributes
         // nothing; so do the B rows >= K of a ragged last block column
         if (cb >= kb32) m = 0;
@@ -483,7 +492,13 @@ __global__ __launch_bounds__(64 * W, (W <= 4 ? 16 / W : 1)) void spmm_f32_batch_
 #pragma unroll
         for (int w = 1; w < W; ++w) v += *reinterpret_cast<const float4_t*>(red + w * 16 * kCols + row * kCols + c4);
         const int64_t crow = row_map ? (int64_t)row_map[grow] : grow;
-        *reinterpret_cast<float4_t*>(C + crow * N + col) = v;
+        if constexpr (EX) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (col + e < nc) C[crow * nc + col + e] = v[e];
+        } else {
+            *reinterpret_cast<float4_t*>(C + crow * N + col) = v;
+        }
     }
 }
 
@@ -494,21 +509,21 @@ __global__ __launch_bounds__(64 * W, (W <= 4 ? 16 / W : 1)) void spmm_f32_batch_
 // Grids of fewer than 512 workgroups: 16 waves per workgroup (one per CU),
 // 4 blocks per pass, so that short grids still spread each block-row's
 // blocks over many waves.
-template <typename I, int NQ>
+template <typename I, int NQ, bool EX>
 void launch_batch(dim3 grid, hipStream_t s, const I* brp, const I* bci, const float* v, const float* b,
                   float* C, int64_t M, int64_t K, int64_t N, int64_t Kb, const int32_t* order,
-                  const I* row_map)
+                  const I* row_map, int64_t nc, const uint32_t* nonfinite)
 {
     const bool short_grid = (int64_t)grid.x * grid.y < 512;
     if (short_grid)
-        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, NQ, 16, 4, 4>), grid, dim3(64 * 16), 0, s, brp,
-                           bci, v, b, C, M, K, N, Kb, order, row_map);
+        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, NQ, 16, 4, 4, EX>), grid, dim3(64 * 16), 0, s, brp,
+                           bci, v, b, C, M, K, N, Kb, order, row_map, nc, nonfinite);
     else if constexpr (NQ == 2)
-        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, 2, 4, 8, 4>), grid, dim3(64 * 4), 0, s, brp, bci,
-                           v, b, C, M, K, N, Kb, order, row_map);
+        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, 2, 4, 8, 4, EX>), grid, dim3(64 * 4), 0, s, brp, bci,
+                           v, b, C, M, K, N, Kb, order, row_map, nc, nonfinite);
     else
-        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, 1, 4, 8, 6>), grid, dim3(64 * 4), 0, s, brp, bci,
-                           v, b, C, M, K, N, Kb, order, row_map);
+        hipLaunchKernelGGL((spmm_f32_batch_kernel<I, 1, 4, 8, 6, EX>), grid, dim3(64 * 4), 0, s, brp, bci,
+                           v, b, C, M, K, N, Kb, order, row_map, nc, nonfinite);
 }
 
 // ---------------------------------------------------------------------------
@@ -663,23 +678,29 @@ bool spmm_f32_batch_covers(int64_t K, int64_t Kb, int64_t N, const void* B, cons
 template <typename I>
 void bcsr_spmm_f32_batch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                          const float* bvals, const float* B, float* C, int64_t N,
-                         const int32_t* order, const I* row_map, hipStream_t s)
+                         const int32_t* order, const I* row_map, hipStream_t s, int64_t nc,
+                         const uint32_t* nonfinite)
 {
-    if (N <= 64)
-        launch_batch<I, 1>(dim3((unsigned)Mb, 1), s, brp, bci, bvals, B, C, M, K, N, Kb, order,
-                           row_map);
+    const dim3 grid((unsigned)Mb, (unsigned)((N + 127) / 128));
+    if (N <= 64 && nc > 0)
+        launch_batch<I, 1, true>(grid, s, brp, bci, bvals, B, C, M, K, N, Kb, order, row_map, nc, nonfinite);
+    else if (N <= 64)
+        launch_batch<I, 1, false>(grid, s, brp, bci, bvals, B, C, M, K, N, Kb, order, row_map, N, nullptr);
+    else if (nc > 0)
+        launch_batch<I, 2, true>(grid, s, brp, bci, bvals, B, C, M, K, N, Kb, order, row_map, nc, nonfinite);
     else
-        launch_batch<I, 2>(dim3((unsigned)Mb, (unsigned)((N + 127) / 128)), s, brp, bci, bvals, B, C,
-                           M, K, N, Kb, order, row_map);
+        launch_batch<I, 2, false>(grid, s, brp, bci, bvals, B, C, M, K, N, Kb, order, row_map, N, nullptr);
     XSPMM_LAUNCH_CHECK();
 }
 
 template void bcsr_spmm_f32_batch<int32_t>(int64_t, int64_t, int64_t, int64_t, const int32_t*,
                                            const int32_t*, const float*, const float*, float*,
-                                           int64_t, const int32_t*, const int32_t*, hipStream_t);
+                                           int64_t, const int32_t*, const int32_t*, hipStream_t,
+                                           int64_t, const uint32_t*);
 template void bcsr_spmm_f32_batch<int64_t>(int64_t, int64_t, int64_t, int64_t, const int64_t*,
                                            const int64_t*, const float*, const float*, float*,
-                                           int64_t, const int32_t*, const int64_t*, hipStream_t);
+                                           int64_t, const int32_t*, const int64_t*, hipStream_t,
+                                           int64_t, const uint32_t*);
 
 template <typename I>
 bool spmm_f32_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, const void* a,
