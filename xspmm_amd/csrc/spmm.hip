@@ -37,6 +37,7 @@
 //
 // Work split: one workgroup per block-row (grid.x, or the dispatch order of
 // order_rows_kernel / xcd_rows_kernel), N split over grid.y.
+#include <cmath>
 #include <cstdlib>
 #include <mutex>
 #include <string>
@@ -68,11 +69,12 @@ __device__ __forceinline__ half8_t load_h8(const uint16_t* p)
 // kernels that read B rows 16 bytes at a time then cover every N.  Bound by
 // memory (one read and one write of B): 3.2 us at 4999 x 31.
 // marks[0 .. 64) (256 bytes, all written): byte i is set when workgroup i of
-// the (at most 256) met an Inf or NaN.
+// the (at most 256) met an Inf or NaN.  Without COPY only the marks are made
+// (B's rows start on 16 bytes already).
 // ---------------------------------------------------------------------------
 constexpr int kPadMarks = 256;
 constexpr int kPadThreads = 256;
-template <typename U>
+template <typename U, bool COPY>
 __global__ __launch_bounds__(kPadThreads) void pad_b_kernel(const U* __restrict__ B, U* __restrict__ Bp,
                                                             int64_t K, int64_t N, int64_t Np,
                                                             unsigned char* __restrict__ marks)
@@ -89,12 +91,15 @@ __global__ __launch_bounds__(kPadThreads) void pad_b_kernel(const U* __restrict_
         const U* src = B + k * N + c;
         typedef U vec_t __attribute__((ext_vector_type(V)));
         vec_t v;
+        if constexpr (COPY) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            v[e] = c + e < N ? src[e] : (U)0;
-            bad |= (v[e] & kExp) == kExp;
+            for (int e = 0; e < V; ++e) v[e] = c + e < N ? src[e] : (U)0;
+            *reinterpret_cast<vec_t*>(Bp + (size_t)t * V) = v;
+        } else {
+            v = *reinterpret_cast<const vec_t*>(src);
         }
-        *reinterpret_cast<vec_t*>(Bp + (size_t)t * V) = v;
+#pragma unroll
+        for (int e = 0; e < V; ++e) bad |= (v[e] & kExp) == kExp;
     }
     const int any = __syncthreads_or(bad ? 1 : 0);
     if (threadIdx.x == 0) marks[blockIdx.x] = any ? 1 : 0;
@@ -812,8 +817,8 @@ __device__ void batch_row_exact(const I* __restrict__ brp, const I* __restrict__
 // (HIP's second __launch_bounds__ argument is the minimum number of waves per
 // SIMD: kBW for four resident workgroups per CU, kBW / 2 for two.)
 //
-// EX (N % 8 != 0): B is pad_b_kernel's copy with rows of N columns, C has pk.nc
-// of them.  The reference multiplies every column of a block, so an Inf or NaN
+// EX (N % 8 != 0, or a full grid): B has rows of N columns (pad_b_kernel's copy
+// unless they start on 16 bytes anyway), C has pk.nc of them.  The reference multiplies every column of a block, so an Inf or NaN
 // in B reaches rows whose block only covers it, and an Inf in A keeps its
 // sign; skipping zero columns and compacting by one-hot products would lose
 // both.  A workgroup that meets a non-finite value (B: the pad kernel's marks;
@@ -1854,10 +1859,10 @@ template bool spmm_dispatch_order_cols<int64_t>(const int64_t*, const int64_t*, 
 
 namespace {
 
-// B with rows of Np columns (N rounded up to 16 bytes) and its marks, made on
-// the stream by pad_b_kernel, and room for order_rows int32, all one piece of
-// the arena (an allocation costs the host about 15 us); bt null when a fixed
-// arena has no room for it.
+// B with rows of Np columns (N rounded up to 16 bytes; B itself when its rows
+// start there already) and its marks, made on the stream by pad_b_kernel, and
+// room for order_rows int32, all one piece of the arena (an allocation costs
+// the host about 15 us); bt null when a fixed arena has no room for it.
 template <typename T>
 struct PaddedB {
     const T* bt = nullptr;
@@ -1873,22 +1878,48 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     constexpr int64_t V = 16 / (int64_t)sizeof(T);
     PaddedB<T> p;
     p.Np = (N + V - 1) / V * V;
+    const bool copy = p.Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
     Carve cv;
     const size_t o_marks = cv.take(kPadMarks);
-    const size_t o_bt = cv.take((size_t)(K > 0 ? K : 1) * (size_t)p.Np * sizeof(T));
+    const size_t o_bt = cv.take(copy ? (size_t)(K > 0 ? K : 1) * (size_t)p.Np * sizeof(T) : 0);
     const size_t o_order = cv.take((size_t)order_rows * sizeof(int32_t));
     if (!arena.fits(cv.end)) return p;
     char* const base = static_cast<char*>(arena.take(cv.end));
     const int64_t vecs = K * (p.Np / V);
-    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads));
-    hipLaunchKernelGGL((pad_b_kernel<U>), dim3((unsigned)wgs), dim3(kPadThreads), 0, s,
-                       reinterpret_cast<const U*>(B), reinterpret_cast<U*>(base + o_bt), K, N, p.Np,
-                       reinterpret_cast<unsigned char*>(base + o_marks));
+    const dim3 wgs((unsigned)std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads)));
+    const U* src = reinterpret_cast<const U*>(B);
+    U* bt = copy ? reinterpret_cast<U*>(base + o_bt) : nullptr;
+    unsigned char* marks = reinterpret_cast<unsigned char*>(base + o_marks);
+    if (copy)
+        hipLaunchKernelGGL((pad_b_kernel<U, true>), wgs, dim3(kPadThreads), 0, s, src, bt, K, N, p.Np, marks);
+    else
+        hipLaunchKernelGGL((pad_b_kernel<U, false>), wgs, dim3(kPadThreads), 0, s, src, bt, K, N, p.Np, marks);
     XSPMM_LAUNCH_CHECK();
-    p.bt = reinterpret_cast<const T*>(base + o_bt);
-    p.marks = reinterpret_cast<const uint32_t*>(base + o_marks);
+    p.bt = copy ? reinterpret_cast<const T*>(bt) : B;
+    p.marks = reinterpret_cast<const uint32_t*>(marks);
     p.order = reinterpret_cast<int32_t*>(base + o_order);
     return p;
+}
+
+// Whether a fully populated fp16 grid takes the GEMM-tiled kernel rather than
+// the column batches, by the times the two were measured to take (us, full
+// grids of 2048 x 1024 to 14336 x 4096, N = 8 .. 1024):
+//   tiled: 0.32 per block column and round of tiles (256 x 256 of C, one per
+//          CU); a tile costs the same however few columns it has;
+//   batch: per block column, 0.055 (N <= 16) to 0.108 (N > 64) while its
+//          workgroups (block-rows x 128 columns) fit one to a CU, about half
+//          of that for each further one; and 18 us for the pass over B and
+//          the host's allocation of its marks.
+// E.g. 4096 x 4096, N = 8: 84 us tiled, 17 in batches; N = 512: 95 and 67;
+// N = 1024: 96 and 118; 14336 x 4096, N = 128: 93 and 67; N = 256: 93 and 123.
+bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
+{
+    constexpr double kCus = 256.0;
+    const double tiles = (double)((Mb + 15) / 16) * (double)((N + 255) / 256);
+    const double tiled = 0.32 * (double)Kb * std::ceil(tiles / kCus);
+    const double per_block = N <= 16 ? 0.055 : N <= 32 ? 0.063 : N <= 64 ? 0.075 : 0.108;
+    const double wgs = (double)Mb * (double)((N + 127) / 128) / kCus;
+    return tiled <= per_block * (double)Kb * std::max(1.0, 0.35 + 0.49 * wgs) + 18.0;
 }
 
 // The Tier-1 launcher: kernel choice as described at the top of this file;
@@ -1915,7 +1946,9 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         // fit 32 bits; B row indices fit 24 bits
         const Fp16Kernel choice = fp16_kernel_choice();
         // every block present: GEMM-tiled kernel (matrix-core bound)
-        if (choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, N))
+        const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, (N + 7) / 8 * 8);
+        const bool tiled = full && dense_f16_pays(Mb, Kb, N);
+        if (tiled && N % 8 == 0)
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         const bool offsets32 = K * N * 2 <= (int64_t(1) << 31) && N < (int64_t(1) << 22) &&
                                Kb < (int64_t(1) << 20);
@@ -1923,7 +1956,7 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         if (chunks > 65535) throw std::invalid_argument("xSpMM: N too large.");
         const dim3 ggrid((unsigned)Mb, (unsigned)chunks);
         if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && N % 8 == 0 &&
-            offsets32) {
+            offsets32 && !full) {
             // more block-rows than resident workgroups (4 per CU on 256 CUs,
             // times two): dispatch the longest rows first
             const int32_t* order = order_in;
@@ -1961,15 +1994,16 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         // on every matrix and N tried (1 .. 127): 16384^2 templates, N = 17,
         // 342 -> 77 us; 50000^2 power-law graph, N = 1, 867 -> 104 us;
         // 5003 x 4999 at 2 %, N = 31, 96 -> 29 us; 8192^2 with 5 % of the
-        // blocks, N = 7, 24 -> 23 us.
+        // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
+        // range come here with any N: it multiplies every column of a block,
+        // and so must the batches where B holds an Inf or NaN.
         const int64_t Np = (N + 7) / 8 * 8;
-        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && N % 8 != 0 &&
+        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) &&
             K * Np * 2 <= (int64_t(1) << 31) && Np < (int64_t(1) << 22) && Kb < (int64_t(1) << 20)) {
-            const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, Np);
-            const bool own_order = !full && !order_in && spmm_order_wanted(Mb);
+            const bool own_order = !tiled && !order_in && spmm_order_wanted(Mb);
             const PaddedB<uint16_t> pb = pad_b<uint16_t>(b, K, N, own_order ? Mb : 0, arena, s);
             if (pb.bt) {
-                if (full)
+                if (tiled)
                     return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
                 const int32_t* order = order_in;
                 if (own_order) {
@@ -1996,6 +2030,8 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
                 return true;
             }
         }
+        if (full && N % 8 == 0)  // B beyond the batches' range, or no room for the marks
+            return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         if (row_map) return false;  // the other fp16 kernels store rows in place
         if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32) {
             if (N <= 64)
