@@ -184,6 +184,23 @@ int xspmm_bcsr_spmm_band(int vtype, int itype, int64_t M, int64_t K, int64_t Mb,
                          int64_t N, void* stream);
 
 /*
+ * xspmm_bcsr_spmm with what a program keeps beside a matrix: a dispatch order
+ * (xspmm_bcsr_dispatch_order_cols; NULL: none) and band != 0 when
+ * xspmm_bcsr_band_rows said so.  The kernel follows from the sizes; on a band
+ * that is the band kernel where it is the faster one (for fp32 not below
+ * about 32 columns, nor on small grids).  scratch (NULL, or 256-byte aligned
+ * device memory of scratch_bytes, kept until the call's work on `stream` is
+ * done) holds a product's temporaries if they fit: 512 + K * N' * value bytes
+ * + 4 * Mb do for every product, rounded up to 256 each, N' = N rounded up to
+ * a multiple of 16 bytes.  What does not fit is allocated on the stream.
+ * Asynchronous on `stream`.
+ * Replaces the same call as xspmm_bcsr_spmm.
+ */
+int xspmm_bcsr_spmm_auto(int vtype, int itype, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb,
+                         const void* brp, const void* bci, const void* bvals, const void* B, float* C, int64_t N,
+                         const int32_t* order, int band, void* scratch, int64_t scratch_bytes, void* stream);
+
+/*
  * CSR -> BCSR, phase 1: writes bcsr_row_ptr[Mb+1] (device) for r x c blocks,
  * Mb = ceil(M/r), and stores nnzb in *nnzb_out (host).  Synchronizes `stream`.
  * Fails with XSPMM_ERR_INVALID if a column index lies outside [0, K).

@@ -39,6 +39,8 @@ def integer_csr(kind, M, K, dtype, itype, seed):
                 np.minimum(np.arange(0, K + 15, 16) + i % 16, K - 1))
         elif kind == "band":
             c = np.arange(max(0, i - 70), min(K, i + 71))
+        elif kind == "wide":
+            c = np.arange(max(0, i - 300), min(K, i + 301))
         elif kind == "deep":
             c = np.unique(rng.integers(0, K, 48))
         else:
@@ -69,9 +71,11 @@ def product(A, B):
 
 
 # fp32 takes the padded copy from 2^18 products of a block with a 16-column tile
-# and N > 16 ("deep": 82000 blocks), the short-grid kernel below
+# and N > 16 ("deep": 73521 blocks), the tile kernel below; full grids of many
+# columns (2050 x 1601 from N = 250) the kernel of banded grids, and bands ("wide")
+# of few columns the tile kernel
 SHAPES = [("deep", 4099, 5003), ("sparse", 8197, 203), ("sparse", 333, 500), ("band", 1003, 997), ("full", 515, 97),
-          ("full", 131, 1601)]
+          ("full", 131, 1601), ("full", 2050, 1601), ("wide", 4003, 3997)]
 
 
 @pytest.mark.parametrize("itype", [np.int32, np.int64])
@@ -81,7 +85,7 @@ def test_odd_n_exact(torch, kind, M, K, dtype, itype):
     rp, ci, vals = integer_csr(kind, M, K, dtype, itype, seed=M)
     A = X.csr_to_bcsr(X.CSRMatrix.from_host(M, K, rp, ci, vals, device="cuda:0"))
     rng = np.random.default_rng(1)
-    for N in (1, 2, 7, 8, 15, 17, 33, 63, 65, 72, 127, 129, 257, 301):
+    for N in (1, 2, 7, 8, 15, 17, 33, 63, 65, 72, 127, 129, 256, 257, 301):
         print(kind, M, K, dtype.__name__, itype.__name__, N, flush=True)
         B = rng.integers(-8, 9, size=(K, N)).astype(dtype)
         guard = torch.full((M * N + 64,), -7.0, device="cuda:0")
@@ -105,13 +109,42 @@ def test_f32_off_16_bytes(torch, itype):
         assert np.array_equal(X.spmm(A, b, c).cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("itype", [np.int32, np.int64])
+def test_f32_full_grid_in_another_order(torch, itype):
+    """A caller's full grid whose rows hold their blocks in any order, and one
+    whose block columns lie outside the grid (they contribute nothing)."""
+    M, K, N = 2050, 1601, 260
+    rp, ci, vals = integer_csr("full", M, K, np.float32, itype, seed=4)
+    A = X.csr_to_bcsr(X.CSRMatrix.from_host(M, K, rp, ci, vals, device="cuda:0"))
+    assert A.num_blocks == A.num_block_rows * A.num_block_cols
+    B = np.random.default_rng(3).integers(-8, 9, size=(K, N)).astype(np.float32)
+    want = product(A, B)
+    b = torch.as_tensor(B).cuda()
+    assert np.array_equal(X.spmm(A, b).cpu().numpy(), want)
+    Kb = A.num_block_cols
+    at = torch.arange(A.num_blocks, device="cuda:0").view(-1, Kb)
+    at[5] = at[5].flip(0)          # one block-row reversed
+    at[-1] = at[-1].roll(3)
+    flat = at.reshape(-1)
+    S = X.BCSRMatrix(A.num_block_rows, Kb, 16, 16, M, K, A.row_ptr, A.col_ind[flat].contiguous(),
+                     A.values.view(-1, 256)[flat].reshape(-1).contiguous())
+    assert np.array_equal(X.spmm(S, b).cpu().numpy(), want)
+    ci2 = A.col_ind.clone()
+    ci2[40 * Kb + 7] = Kb + 3      # outside the grid
+    S = X.BCSRMatrix(A.num_block_rows, Kb, 16, 16, M, K, A.row_ptr, ci2, A.values)
+    v = A.values.clone()
+    v.view(-1, 256)[40 * Kb + 7] = 0
+    Z = X.BCSRMatrix(A.num_block_rows, Kb, 16, 16, M, K, A.row_ptr, A.col_ind, v)
+    assert np.array_equal(X.spmm(S, b).cpu().numpy(), product(Z, B))
+
+
 @pytest.mark.parametrize("where", ["A", "B"])
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("kind,M,K", SHAPES)
 def test_nonfinite_reaches_what_the_reference_reaches(torch, kind, M, K, dtype, where):
     rp, ci, vals = integer_csr(kind, M, K, dtype, np.int32, seed=M + 1)
     for N, special in ((5, np.inf), (67, -np.inf), (131, np.nan), (40, np.inf)):
-        if N % 8 == 0 and kind not in ("full", "band"):
+        if N % 8 == 0 and kind not in ("full", "band", "wide"):
             continue  # the column batches of aligned rows skip zero columns
         print(kind, M, K, dtype.__name__, where, N, flush=True)
         v = vals.copy()

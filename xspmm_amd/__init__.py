@@ -71,6 +71,8 @@ def load():
     L.xspmm_bcsr_band_rows.argtypes = [i32, i32, i64, i64, i64, i64, i64, i64, p, p, C.POINTER(C.c_int), p]
     L.xspmm_bcsr_spmm_band.restype = i32
     L.xspmm_bcsr_spmm_band.argtypes = [i32, i32, i64, i64, i64, i64, i64, p, p, p, p, p, i64, p]
+    L.xspmm_bcsr_spmm_auto.restype = i32
+    L.xspmm_bcsr_spmm_auto.argtypes = [i32, i32, i64, i64, i64, i64, i64, p, p, p, p, p, i64, p, i32, p, i64, p]
     L.xspmm_bcsr_dispatch_order_cols.restype = i32
     L.xspmm_bcsr_dispatch_order_cols.argtypes = [i32, i64, p, p, p, C.POINTER(C.c_int), p]
     L.xspmm_csr_to_bcsr_count.restype = i32
@@ -341,18 +343,12 @@ def spmm(A: BCSRMatrix, B, C_out=None, N: int | None = None):
         C_out = torch.empty((A.num_rows, N), dtype=torch.float32, device=dev)
     _check_dense(B, "B", A.num_cols, N, A.values.dtype, dev)
     _check_dense(C_out, "C_out", A.num_rows, N, torch.float32, dev)
-    if A.band_rows():
-        _check(L.xspmm_bcsr_spmm_band(vcode(B.dtype), icode(A.row_ptr.dtype), A.num_rows, A.num_cols,
-                                      A.num_block_rows, A.num_block_cols, A.num_blocks,
-                                      _ptr(A.row_ptr), _ptr(A.col_ind), _ptr(A.values), _ptr(B),
-                                      _ptr(C_out), N, _stream()))
-        return C_out
+    band = A.band_rows()
     order = A.dispatch_order()
-    _check(L.xspmm_bcsr_spmm_ordered(vcode(B.dtype), icode(A.row_ptr.dtype), A.num_rows,
-                                     A.num_cols, A.num_block_rows, A.num_block_cols, A.num_blocks,
-                                     _ptr(A.row_ptr), _ptr(A.col_ind), _ptr(A.values), _ptr(B),
-                                     _ptr(C_out), N, _ptr(order) if order is not None else None,
-                                     _stream()))
+    _check(L.xspmm_bcsr_spmm_auto(vcode(B.dtype), icode(A.row_ptr.dtype), A.num_rows, A.num_cols,
+                                  A.num_block_rows, A.num_block_cols, A.num_blocks, _ptr(A.row_ptr),
+                                  _ptr(A.col_ind), _ptr(A.values), _ptr(B), _ptr(C_out), N,
+                                  _ptr(order) if order is not None else None, int(band), None, 0, _stream()))
     return C_out
 
 

@@ -165,17 +165,10 @@ void spmm(const BCSRMatrix<InputType, IndexType>& A, const InputType* B, OutputT
         if (A.get_r_block() != 16 || A.get_c_block() != 16)
             throw std::invalid_argument("xSpMM: the MFMA tile kernel requires 16x16 blocks.");
         use_device(h);
-        if (A.get_band_rows()) {
-            detail::bcsr_spmm_band<dev_t<InputType>, IndexType>(
-                A.get_num_rows(), A.get_num_cols(), A.get_num_block_rows(), A.get_num_block_cols(),
-                A.get_num_blocks(), A.get_bcsr_row_ptr(), A.get_bcsr_col_ind(), dev(A.get_bcsr_values()),
-                dev(B), C, N, kStream);
-            return;
-        }
-        (void)detail::bcsr_spmm_ex<dev_t<InputType>, IndexType>(
+        detail::bcsr_spmm_auto<dev_t<InputType>, IndexType>(
             A.get_num_rows(), A.get_num_cols(), A.get_num_block_rows(), A.get_num_block_cols(),
             A.get_num_blocks(), A.get_bcsr_row_ptr(), A.get_bcsr_col_ind(), dev(A.get_bcsr_values()),
-            dev(B), C, N, A.get_dispatch_order(), nullptr, kStream);
+            dev(B), C, N, A.get_dispatch_order(), A.get_band_rows(), nullptr, 0, kStream);
         return;
     }
     throw std::runtime_error("xSpMM: CPU SpMM fallback is not yet implemented. Please use a GPU Executor.");

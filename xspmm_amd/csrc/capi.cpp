@@ -208,6 +208,23 @@ int xspmm_bcsr_spmm_band(int vtype, int itype, int64_t M, int64_t K, int64_t Mb,
     });
 }
 
+int xspmm_bcsr_spmm_auto(int vtype, int itype, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb,
+                         const void* brp, const void* bci, const void* bvals, const void* B, float* C, int64_t N,
+                         const int32_t* order, int band, void* scratch, int64_t scratch_bytes, void* stream)
+{
+    return guarded([&] {
+        if (scratch_bytes < 0 || (reinterpret_cast<uintptr_t>(scratch) & 255) != 0)
+            throw std::invalid_argument("xSpMM: scratch must be 256-byte aligned, its size not negative.");
+        with_types(vtype, itype, [&](auto tv, auto ti) {
+            using T = typename decltype(tv)::type;
+            using I = typename decltype(ti)::type;
+            bcsr_spmm_auto<T, I>(M, K, Mb, Kb, nnzb, static_cast<const I*>(brp), static_cast<const I*>(bci),
+                                 static_cast<const T*>(bvals), static_cast<const T*>(B), C, N, order, band != 0,
+                                 scratch, (size_t)scratch_bytes, as_stream(stream));
+        });
+    });
+}
+
 int xspmm_csr_to_bcsr_count(int itype, int64_t M, int64_t K, int64_t nnz, const void* rp,
                             const void* ci, int64_t r_block, int64_t c_block,
                             void* bcsr_row_ptr, int64_t* nnzb_out, void* stream)

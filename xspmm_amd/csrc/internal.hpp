@@ -114,8 +114,9 @@ private:
 class TempArena {
 public:
     explicit TempArena(hipStream_t s) : s_(s) {}
-    TempArena(void* base, size_t bytes, hipStream_t s)
-        : s_(s), base_(static_cast<char*>(base)), cap_(bytes) {}
+    // spill: what does not fit the given memory is allocated instead
+    TempArena(void* base, size_t bytes, hipStream_t s, bool spill = false)
+        : s_(s), base_(static_cast<char*>(base)), cap_(base ? bytes : 0), spill_(spill) {}
     TempArena(const TempArena&) = delete;
     TempArena& operator=(const TempArena&) = delete;
     bool fixed() const { return base_ != nullptr; }
@@ -123,16 +124,17 @@ public:
     // whether take(bytes) has room for them
     bool fits(size_t bytes) const {
         const size_t at = (used_ + 255) & ~size_t(255);
-        return !base_ || (at <= cap_ && bytes <= cap_ - at);
+        return !base_ || spill_ || (at <= cap_ && bytes <= cap_ - at);
     }
     void* take(size_t bytes) {
         if (bytes == 0) return nullptr;
-        if (!base_) {
+        const size_t at = (used_ + 255) & ~size_t(255);
+        const bool room = base_ && at <= cap_ && bytes <= cap_ - at;
+        if (!base_ || (spill_ && !room)) {
             owned_.emplace_back(bytes, s_);
             return owned_.back().get();
         }
-        const size_t at = (used_ + 255) & ~size_t(255);
-        if (at > cap_ || bytes > cap_ - at)
+        if (!room)
             throw std::invalid_argument(
                 "xSpMM: this product needs " + std::to_string(at + bytes) +
                 " bytes of scratch; the allocation-free entry point has " + std::to_string(cap_) +
@@ -147,6 +149,7 @@ private:
     hipStream_t s_;
     char* base_ = nullptr;
     size_t cap_ = 0, used_ = 0;
+    bool spill_ = false;
     std::vector<Scratch> owned_;
 };
 
@@ -234,6 +237,17 @@ bool bcsr_spmm_ex(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, co
 template <typename T, typename I>
 void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp, const I* bci,
                     const T* bvals, const T* B, float* C, int64_t N, hipStream_t s);
+// Tier-1 with everything kept on a matrix: its dispatch order (or null) and
+// whether its block-rows are contiguous runs (band; spmm_band_wanted).  The
+// kernel follows from the sizes: a contiguous grid takes a band kernel where
+// that is the faster one.  Temporaries come from scratch (bcsr_spmm_scratch
+// bytes always do; null or less: stream-ordered allocations), which the caller
+// keeps for the call's work on s.
+template <typename T, typename I>
+void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp, const I* bci,
+                    const T* bvals, const T* B, float* C, int64_t N, const int32_t* order, bool band, void* scratch,
+                    size_t scratch_bytes, hipStream_t s);
+size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N);
 // Tier-1 without any allocation: the temporaries come from a fixed device
 // array of kNoAllocScratchBytes (one copy per GPU, shared by every call on
 // it).  Throws std::invalid_argument when a product needs more.
@@ -289,8 +303,7 @@ bool spmm_f16_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, c
                      const int32_t* order, const I* row_map, hipStream_t s);
 
 // Tier-1 fp32 column-batch SpMM (spmm_f32.hip): covers N % 4 == 0 with B and
-// C 16-byte aligned, K * N * 4 <= 2^31 and Kb < 2^21 (XSPMM_F32_KERNEL=tile
-// declines it); order and row_map as for bcsr_spmm_ex.  With nc > 0, B is a
+// C 16-byte aligned, K * N * 4 <= 2^31 and Kb < 2^21; order and row_map as for bcsr_spmm_ex.  With nc > 0, B is a
 // copy padded to N columns, C has nc (any alignment) and nonfinite holds the
 // copy's 256 bytes of Inf / NaN marks: when one is set, every column of a block
 // is multiplied, so that B meets each row as in the reference.
@@ -336,12 +349,22 @@ bool spmm_band_f16_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N);
 // equal shares of the groups' blocks per workgroup, cut groups summed in part
 // order; stream-ordered scratch).  False (nothing
 // launched) when the shape is not covered (N % 4 != 0, B or C not 16-byte
-// aligned, K * N * 4 > 2^31).
+// aligned, K * N * 4 > 2^31).  nc > 0: C has nc <= N columns, at any address
+// (B padded to N).
 bool spmm_band_f32_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N, const void* B, const void* C);
+// Estimated times (us) of its two launches for N columns.
+void spmm_band_f32_times(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, double* one, double* balanced);
 template <typename I>
 bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const float* bvals, const float* B, float* C, int64_t N, const I* row_map,
-                        int64_t nnzb, hipStream_t s);
+                        int64_t nnzb, hipStream_t s, int64_t nc = 0);
+// The same kernel, one group per workgroup, for a grid with every block present
+// (nnzb == Mb * Kb) in any stored order: each workgroup checks its block-rows
+// and multiplies them block by block when they are not in column order.
+template <typename I>
+bool bcsr_spmm_full_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
+                        const float* bvals, const float* B, float* C, int64_t N, const I* row_map,
+                        hipStream_t s, int64_t nc = 0);
 // Whether Tier-1 should take a band kernel for this grid of fp16
 // (value_bytes 2) or fp32 (4) blocks: every block-row contiguous, the grid not
 // full, the groups' spans gathering fewer B rows than the column-batch kernel

@@ -25,10 +25,11 @@
 // fp32 kernels.  v_mfma_f32_16x16x4f32 takes one k per lane, so B is read
 // row-major directly:
 //   spmm_f32_batch_kernel   (spmm_f32.hip) default where the grid has at
-//                           least 512 workgroups of 128 columns: the non-zero
-//                           block columns of a block-row packed four to a
-//                           K = 4 batch;
-//   spmm_f32_short_kernel   short grids: lane l loads A[l&15][4g .. 4g+3]
+//                           least 512 workgroups of 128 columns and N > 8: the
+//                           non-zero block columns of a block-row packed four
+//                           to a K = 4 batch;
+//   spmm_f32_band_kernel    (spmm_band.hip) full and banded grids of many columns;
+//   spmm_f32_short_kernel   short grids and N <= 8: lane l loads A[l&15][4g .. 4g+3]
 //                           (g = l>>4) once per block and issues four MFMAs,
 //                           step s pairing A[i][4g+s] with B[16*col + 4g + s][n]
 //                           (B through a buffer resource);
@@ -39,6 +40,8 @@
 // order_rows_kernel / xcd_rows_kernel), N split over grid.y.
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
+#include <limits>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -1536,7 +1539,7 @@ __global__ __launch_bounds__(64 * kF32Waves) void spmm_f32_kernel(const I* __res
 }
 
 // ---------------------------------------------------------------------------
-// fp32 short-grid kernel where B's byte offsets fit 30 bits (16 * Kb * N * 4
+// fp32 tile kernel (short grids, few columns) where B's byte offsets fit 30 bits (16 * Kb * N * 4
 // <= 2^30): the tile kernel's product with B read through a buffer resource.
 // A lane's B offset within a block's 16 rows is fixed for the kernel, so each
 // B load is one add and one buffer load; an offset past the end of B (rows
@@ -1554,11 +1557,12 @@ constexpr int kF32ShortUnroll = 4;
 constexpr uint32_t kF32ShortPast = 1u << 30;
 constexpr int64_t kF32ShortMaxBytes = int64_t(1) << 30;
 
-template <typename I, int NTW>
+// STREAM: blocks are read past the last-level cache.
+template <typename I, int NTW, bool STREAM>
 __global__ __launch_bounds__(64 * kF32ShortWaves) void spmm_f32_short_kernel(
     const I* __restrict__ brp, const I* __restrict__ bci, const float* __restrict__ vals,
     const float* __restrict__ B, float* __restrict__ C, int64_t M, int64_t K, int64_t N, int64_t Kb,
-    int ntiles)
+    int ntiles, const int32_t* __restrict__ order, const I* __restrict__ row_map)
 {
     constexpr int W = kF32ShortWaves;
     constexpr int U = kF32ShortUnroll;
@@ -1568,7 +1572,10 @@ __global__ __launch_bounds__(64 * kF32ShortWaves) void spmm_f32_short_kernel(
     const int li = lane & 15;
     const int g = lane >> 4;
     const int tile0 = blockIdx.y * NTW;
-    const int64_t br = blockIdx.x;
+    const int64_t br = order ? (int64_t)order[blockIdx.x] : (int64_t)blockIdx.x;
+    // a caller-supplied order holds a permutation of the block-rows; an id
+    // outside the grid is skipped rather than read past row_ptr
+    if ((uint64_t)br >= (uint64_t)gridDim.x) return;
     const int64_t rs = brp[br];
     const int64_t re = brp[br + 1];
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(B, (uint32_t)(K * N * 4));
@@ -1597,7 +1604,11 @@ __global__ __launch_bounds__(64 * kF32ShortWaves) void spmm_f32_short_kernel(
         for (int u = 0; u < U; ++u) {
             const int64_t b0 = blk + u * W;
             const int64_t b = b0 < re ? b0 : re - 1;
-            a[u] = *reinterpret_cast<const float4_t*>(vals + b * 256 + li * 16 + g * 4);
+            const float4_t* const ap = reinterpret_cast<const float4_t*>(vals + b * 256 + li * 16 + g * 4);
+            if constexpr (STREAM)
+                a[u] = __builtin_nontemporal_load(ap);
+            else
+                a[u] = *ap;
             const int64_t col = (int64_t)bci[b];
             base[u] = (col >= 0 && col < Kb) ? (uint32_t)col * rowbytes : kF32ShortPast;
         }
@@ -1635,7 +1646,7 @@ __global__ __launch_bounds__(64 * kF32ShortWaves) void spmm_f32_short_kernel(
         for (int w = 1; w < W; ++w) sum += red[w][row][c];
         const int64_t grow = br * 16 + row;
         const int64_t col = (int64_t)tile0 * 16 + c;
-        if (grow < M && col < N && tile0 + c / 16 < ntiles) C[grow * N + col] = sum;
+        if (grow < M && col < N && tile0 + c / 16 < ntiles) C[(row_map ? (int64_t)row_map[grow] : grow) * N + col] = sum;
     }
 }
 
@@ -1645,7 +1656,7 @@ __global__ __launch_bounds__(64 * kF32ShortWaves) void spmm_f32_short_kernel(
 bool f32_short_wanted(int64_t Kb, int64_t N)
 {
     const char* e = std::getenv("XSPMM_F32_SHORT");
-    if (e && std::string(e) == "off") return false;
+    if (e && std::strcmp(e, "off") == 0) return false;
     return N > 0 && N <= kF32ShortMaxBytes / 64 && Kb <= kF32ShortMaxBytes / (64 * N);
 }
 
@@ -1711,16 +1722,87 @@ bool wide_batches(int64_t Mb, int64_t N)
     return Mb * ((N + 255) / 256) >= 1024;
 }
 
-// fp32: the column-batch kernel runs one workgroup per block-row and 128
-// columns; a grid shorter than this takes the tile kernel, which splits each
-// block-row over 8 waves and narrower column tiles.  XSPMM_F32_KERNEL=batch
-// forces the batch kernel (where it covers the shape), =tile the tile kernel.
+// Column tiles of 16 per workgroup of the fp32 tile kernel: 4 (fewer B loads
+// per block; also for three tiles, which two per workgroup would stream A twice
+// for) unless that leaves fewer than 512 workgroups, when narrower tiles spread
+// the block-rows over more CUs.
+int f32_tiles_per_group(int64_t Mb, int64_t ntiles)
+{
+    int ntw = ntiles >= 3 ? 4 : (ntiles >= 2 ? 2 : 1);
+    while (ntw > 1 && Mb * ((ntiles + ntw - 1) / ntw) < 512) ntw /= 2;
+    return ntw;
+}
+
+// fp32 kernels: whole blocks in 16-column tiles with 16 waves on each block-row
+// (kTile), column batches (kBatch, one workgroup per block-row and 128
+// columns), four block-rows sharing each B load (kShared; full grids, and grids
+// of contiguous block-rows).  XSPMM_F32_KERNEL=batch forces the batches (where
+// they cover the shape), =tile the tile kernel.
+enum class F32Kernel { kTile, kBatch, kShared };
 constexpr int64_t kF32BatchMinGroups = 512;
 
-bool f32_kernel_forced_batch()
+// The choice, from measured times (us).
+// Full grids and grids of contiguous block-rows, whose blocks are mostly full
+// (512 x 8192 to 14336 x 4096 full, bands of 5 to 90 % of 2984^2 to 16384^2; N =
+// 4 .. 1024), per block of an average block-row:
+//   kShared: full grid, 0.33 while its workgroups (four block-rows x 64
+//            columns) fit one to a CU, 0.52 per round of two; a band, the
+//            launcher's estimates of its two launches (one workgroup per CU
+//            runs 1.5 times as fast as two);
+//   kBatch:  0.13 (N <= 64) or 0.19 on a short grid, then with its workgroups;
+//   kTile:   with its workgroups and the columns of each;
+//   padding B costs 18 more.  kTile and kShared multiply whole blocks, as does
+//   kBatch on a padded copy; kBatch on B itself skips zero columns, which an
+//   Inf in B shows, so it stays with the full grids of 512 workgroups or more.
+//   4096 x 4096 full, tile / batch / shared: N = 8 16 / 33 / 84, N = 64 40 / 33 /
+//   86, N = 512 235 / 171 / 135; 14336 x 4096: N = 8 42 / 110 / 85, N = 1024
+//   1582 / 1159 / 924; bands, tile / shared: 16384^2 50 % N = 16 95 / 182, N = 64
+//   235 / 187; 11089^2 60 % N = 16 46 / 103; 4096^2 80 % N = 32 19 / 45, N = 64
+//   30 / 45; 2984^2 11 % N = 64 9 / 11; 8003^2 7.5 % N = 64 19 / 16.
+// Other grids: one 16-column tile of at most 8 columns takes whole blocks (a
+// block costs one B load whatever its fill: N = 4, blocks of 5 columns 138 ->
+// 68 us, power-law graph 274 -> 157, 8192^2 with 5 % full blocks 12.4 -> 6.0,
+// 1.7 columns 137 -> 141); wider ones the batches from 512 workgroups; on a
+// padded copy of B, the batches from 2^18 products of a block with a tile (N =
+// 17: 300980 blocks 123 -> 80, 97367 blocks 43 -> 58; N = 33: 97367 blocks 71 ->
+// 58, 14465 blocks 14 -> 24).
+// whole: the tile kernel covers B (f32_short_wanted).
+F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool aligned, bool whole,
+                            bool contiguous)
 {
-    const char* e = std::getenv("XSPMM_F32_KERNEL");
-    return e && std::string(e) == "batch";
+    const int64_t tiles = (N + 15) / 16;
+    const bool full = nnzb == Mb * Kb;
+    // a band of more columns keeps the kernel its rows were chosen for (tile is
+    // ahead only on small grids: 4096^2 80 %, N = 128, 44 / 57)
+    if ((full || (contiguous && N <= 64)) && nnzb > 0 && whole && N < (int64_t(1) << 22) && Kb < (int64_t(1) << 20)) {
+        const double pad = aligned ? 0.0 : 18.0;
+        const double blocks = (double)nnzb / (double)Mb;
+        const double groups = (double)((Mb + 3) / 4) * (double)((N + 63) / 64);
+        const double rows = (double)Mb * (double)((N + 127) / 128);
+        double shared;
+        if (full) {
+            shared = blocks * (groups <= 256.0 ? 0.33 : 0.52 * std::ceil(groups / 512.0));
+        } else {
+            double one, balanced;
+            spmm_band_f32_times(Mb, Kb, nnzb, (N + 63) / 64 * 64, &one, &balanced);
+            shared = std::min(groups <= 256.0 ? 0.65 * one : one, 1.05 * balanced);
+        }
+        shared += 1.5 + pad;
+        double batch = std::numeric_limits<double>::infinity();
+        if (!aligned || (full && rows >= (double)kF32BatchMinGroups))
+            batch = blocks * (N <= 64 ? std::max(0.13, 0.00048 * rows) : std::max(0.19, 0.00065 * rows)) + 2.5 + pad;
+        const int ntw = f32_tiles_per_group(Mb, tiles);
+        const double wgs = (double)Mb * (double)((tiles + ntw - 1) / ntw);
+        const double tile = blocks * std::max(0.045, wgs * (ntw == 1 ? 1.9e-4 : ntw == 2 ? 3.3e-4 : 5.4e-4)) +
+                            (ntw == 4 ? 6.0 : ntw == 2 ? 5.0 : 2.0);
+        if (shared < std::min(batch, tile)) return F32Kernel::kShared;
+        return batch < tile ? F32Kernel::kBatch : F32Kernel::kTile;
+    }
+    if (contiguous) return F32Kernel::kShared;
+    if (aligned)
+        return (N > 8 || !whole) && Mb * ((N + 127) / 128) >= kF32BatchMinGroups ? F32Kernel::kBatch
+                                                                                 : F32Kernel::kTile;
+    return N > 16 && nnzb * tiles >= (int64_t(1) << 18) ? F32Kernel::kBatch : F32Kernel::kTile;
 }
 
 void check_shape(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N)
@@ -1924,10 +2006,12 @@ bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
 
 // The Tier-1 launcher: kernel choice as described at the top of this file;
 // temporaries (the dispatch order, repacked B panels) come from `arena`.
+// contiguous (fp32): every block-row is one run of block columns.
 template <typename T, typename I>
 bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                       const I* bci, const T* bvals, const T* B, float* C, int64_t N,
-                      const int32_t* order_in, const I* row_map, TempArena& arena, hipStream_t s)
+                      const int32_t* order_in, const I* row_map, TempArena& arena, hipStream_t s,
+                      bool contiguous = false)
 {
     check_shape(M, K, Mb, Kb, nnzb, N);
     if (M == 0 || N == 0 || Mb == 0) return true;
@@ -2069,69 +2153,70 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
     } else {
         const float* v = reinterpret_cast<const float*>(bvals);
         const float* b = reinterpret_cast<const float*>(B);
-        // column batches (spmm_f32.hip) unless the grid is too short to keep
-        // the chip busy with one workgroup per block-row
-        if (spmm_f32_batch_covers(K, Kb, N, B, C) &&
-            (f32_kernel_forced_batch() || Mb * ((N + 127) / 128) >= kF32BatchMinGroups)) {
-            const int32_t* order = order_in;
-            if (!order && spmm_order_wanted(Mb)) {
-                int32_t* buf = arena.take_as<int32_t>((size_t)Mb);
-                spmm_dispatch_order<I>(brp, Mb, buf, s);
-                order = buf;
-            }
-            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, b, C, N, order, row_map, s);
+        const bool aligned = spmm_f32_batch_covers(K, Kb, N, B, C);
+        const int64_t Np = (N + 3) / 4 * 4;
+        const bool whole = f32_short_wanted(Kb, N);
+        const char* forced = std::getenv("XSPMM_F32_KERNEL");
+        F32Kernel kernel = F32Kernel::kTile;
+        if ((aligned || spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr)) &&
+            !(forced && std::strcmp(forced, "tile") == 0))
+            kernel = forced && std::strcmp(forced, "batch") == 0
+                         ? F32Kernel::kBatch
+                         : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, whole, contiguous);
+        const bool order_here = kernel != F32Kernel::kShared && !order_in && spmm_order_wanted(Mb);
+        auto shared = [&](const float* bb, int64_t n, int64_t nc) {
+            return contiguous
+                       ? bcsr_spmm_band_f32<I>(M, K, Mb, Kb, brp, bci, v, bb, C, n, row_map, nnzb, s, nc)
+                       : bcsr_spmm_full_f32<I>(M, K, Mb, Kb, brp, bci, v, bb, C, n, row_map, s, nc);
+        };
+        auto order_with = [&](int32_t* buf) -> const int32_t* {
+            if (!order_here) return order_in;
+            spmm_dispatch_order<I>(brp, Mb, buf, s);
+            return buf;
+        };
+        auto order_rows = [&]() { return order_with(order_here ? arena.take_as<int32_t>((size_t)Mb) : nullptr); };
+        if (kernel != F32Kernel::kTile && aligned) {
+            if (kernel == F32Kernel::kShared) return shared(b, N, 0);
+            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, b, C, N, order_rows(), row_map, s);
             return true;
         }
-        // N % 4 != 0, or B or C off 16 bytes: the column batches on a padded
-        // copy of B, from 2^18 products of a block with a 16-column tile, where
-        // they make up for the copy (N = 17: 300980 blocks 123 -> 80 us, 97367
-        // blocks 43 -> 58 us; N = 33: 97367 blocks 71 -> 58, 14465 blocks
-        // 14 -> 24).  One tile (N <= 16) stays below, where a block costs one
-        // B load whatever its fill (N = 1: 367862 blocks of 5 columns 105 us,
-        // 151 in batches).
-        const int64_t Np = (N + 3) / 4 * 4;
-        if (spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr) &&
-            (f32_kernel_forced_batch() || (N > 16 && nnzb * ntiles64 >= (int64_t(1) << 18)))) {
-            const bool own_order = !order_in && spmm_order_wanted(Mb);
-            const PaddedB<float> pb = pad_b<float>(b, K, N, own_order ? Mb : 0, arena, s);
+        if (kernel != F32Kernel::kTile) {
+            // N % 4 != 0, or B or C off 16 bytes: the same kernels on a padded
+            // copy of B
+            const PaddedB<float> pb = pad_b<float>(b, K, N, order_here ? Mb : 0, arena, s);
+            if (pb.bt && kernel == F32Kernel::kShared) return shared(pb.bt, Np, N);
             if (pb.bt) {
-                const int32_t* order = order_in;
-                if (own_order) {
-                    spmm_dispatch_order<I>(brp, Mb, pb.order, s);
-                    order = pb.order;
-                }
-                bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order, row_map, s, N, pb.marks);
+                bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order_with(pb.order), row_map, s, N,
+                                       pb.marks);
                 return true;
             }
         }
-        if (row_map) return false;  // the fp32 tile kernel stores rows in place
-        // 16-column tiles per wave: 4 (fewer B loads per block) unless that
-        // leaves fewer than 512 workgroups, when narrower tiles spread the
-        // block-rows over more CUs
-        int ntw = ntiles >= 4 ? 4 : (ntiles >= 2 ? 2 : 1);
-        while (ntw > 1 && Mb * ((ntiles + ntw - 1) / ntw) < 512) ntw /= 2;
+        const int ntw = f32_tiles_per_group(Mb, ntiles);
         const int64_t gy = (ntiles + ntw - 1) / ntw;
         if (gy > 65535) throw std::invalid_argument("xSpMM: N too large.");
         const dim3 fgrid((unsigned)Mb, (unsigned)gy);
-        if (f32_short_wanted(Kb, N)) {
-            const dim3 sblock(64 * kF32ShortWaves);
-            switch (ntw) {
-            case 4:
-                hipLaunchKernelGGL((spmm_f32_short_kernel<I, 4>), fgrid, sblock, 0, s, brp, bci, v,
-                                   b, C, M, K, N, Kb, ntiles);
-                break;
-            case 2:
-                hipLaunchKernelGGL((spmm_f32_short_kernel<I, 2>), fgrid, sblock, 0, s, brp, bci, v,
-                                   b, C, M, K, N, Kb, ntiles);
-                break;
-            default:
-                hipLaunchKernelGGL((spmm_f32_short_kernel<I, 1>), fgrid, sblock, 0, s, brp, bci, v,
-                                   b, C, M, K, N, Kb, ntiles);
-                break;
-            }
+        if (whole) {
+            // blocks beyond the 256 MB last-level cache are read past it
+            // (775 MB, N = 4: 150 -> 141 us; 100 MB, N = 16: 26 -> 30)
+            const bool stream = nnzb > (int64_t(1) << 18);
+            const int32_t* order =
+                !order_here || arena.fits((size_t)Mb * sizeof(int32_t)) ? order_rows() : nullptr;
+            auto launch = [&](auto k) {
+                hipLaunchKernelGGL(k, fgrid, dim3(64 * kF32ShortWaves), 0, s, brp, bci, v, b, C, M, K, N, Kb,
+                                   ntiles, order, row_map);
+            };
+            if (ntw == 4)
+                launch(spmm_f32_short_kernel<I, 4, false>);
+            else if (ntw == 2)
+                launch(spmm_f32_short_kernel<I, 2, false>);
+            else if (stream)
+                launch(spmm_f32_short_kernel<I, 1, true>);
+            else
+                launch(spmm_f32_short_kernel<I, 1, false>);
             XSPMM_LAUNCH_CHECK();
             return true;
         }
+        if (row_map) return false;  // the 64-bit tile kernel stores rows in place
         const dim3 fblock(64 * kF32Waves);
         switch (ntw) {
         case 4:
@@ -2213,21 +2298,52 @@ void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
     check_alignment(bvals, B, sizeof(T) == 2);
     if constexpr (sizeof(T) == 2) {
         if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, s)) return;
-        // N % 8 != 0: on a padded copy of B
-        const int64_t Np = (N + 7) / 8 * 8;
-        if (spmm_band_f16_covers(K, Kb, Mb, Np)) {
-            TempArena arena(s);
-            const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K, N, 0, arena, s);
-            if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, pb.bt, C, Np, nullptr, s, N)) return;
-        }
     } else {
         if (bcsr_spmm_band_f32<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, nnzb, s)) return;
     }
     (void)bcsr_spmm_ex<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, nullptr, nullptr, s);
 }
+
+template <typename T, typename I>
+void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp, const I* bci,
+                    const T* bvals, const T* B, float* C, int64_t N, const int32_t* order, bool band, void* scratch,
+                    size_t scratch_bytes, hipStream_t s)
+{
+    TempArena arena(scratch, scratch_bytes, s, true);
+    if constexpr (sizeof(T) == 2) {
+        if (band) {
+            check_shape(M, K, Mb, Kb, nnzb, N);
+            if (M == 0 || N == 0 || Mb == 0) return;
+            check_alignment(bvals, B, true);
+            if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, s)) return;
+            // N % 8 != 0: on a padded copy of B
+            const int64_t Np = (N + 7) / 8 * 8;
+            if (spmm_band_f16_covers(K, Kb, Mb, Np)) {
+                const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K, N, 0, arena, s);
+                if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, pb.bt, C, Np, nullptr, s, N)) return;
+            }
+        }
+    }
+    const bool contiguous = sizeof(T) == 4 && band && spmm_band_f32_covers(K, Kb, Mb, (N + 3) / 4 * 4, nullptr, nullptr);
+    (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order, nullptr, arena, s, contiguous);
+}
+
+size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N)
+{
+    const int64_t V = 16 / value_bytes;
+    Carve cv;  // as pad_b
+    cv.take(kPadMarks);
+    cv.take((size_t)(K > 0 ? K : 1) * (size_t)((N + V - 1) / V * V) * (size_t)value_bytes);
+    cv.take(spmm_order_wanted(Mb) ? (size_t)Mb * sizeof(int32_t) : 0);
+    return cv.end;
+}
+
 #define XSPMM_SPMM_BAND(T, I)                                                                          \
     template void bcsr_spmm_band<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*, const I*, \
-                                       const T*, const T*, float*, int64_t, hipStream_t);
+                                       const T*, const T*, float*, int64_t, hipStream_t);              \
+    template void bcsr_spmm_auto<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*, const I*, \
+                                       const T*, const T*, float*, int64_t, const int32_t*, bool,      \
+                                       void*, size_t, hipStream_t);
 XSPMM_SPMM_BAND(uint16_t, int32_t)
 XSPMM_SPMM_BAND(uint16_t, int64_t)
 XSPMM_SPMM_BAND(float, int32_t)

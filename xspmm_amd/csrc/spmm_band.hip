@@ -475,6 +475,67 @@ __global__ __launch_bounds__(1024) void band_plan_kernel(const I* __restrict__ b
     for (int64_t i = threadIdx.x; i < (int64_t)P * chunks; i += 1024) sp.arrivals[i] = 0;
 }
 
+// Whether block-rows br0 .. br0 + rows - 1 hold the columns 0 .. Kb - 1 in
+// order; every thread of the workgroup (256) gets the answer.
+template <typename I>
+__device__ bool band_group_is_full(const I* __restrict__ brp, const I* __restrict__ bci, int64_t br0,
+                                   int64_t rows, int64_t Kb)
+{
+    bool ok = true;
+    const int64_t rs = (int64_t)brp[br0];
+    if ((int64_t)threadIdx.x <= rows) ok = (int64_t)brp[br0 + threadIdx.x] - rs == (int64_t)threadIdx.x * Kb;
+    // the row pointers decide before any column is read through them
+    if (!__syncthreads_and(ok ? 1 : 0)) return false;
+    const uint32_t kb = (uint32_t)Kb, total = (uint32_t)(rows * Kb);
+    for (uint32_t i = threadIdx.x; i < total; i += 256) ok &= (int64_t)bci[rs + i] == (int64_t)(i % kb);
+    return __syncthreads_and(ok ? 1 : 0) != 0;
+}
+
+// The 64 x 64 tile of the group at br0, column n0 on, from blocks in any order
+// (reference src/common/spmm_math.hpp:68-114): wave w multiplies block-row
+// br0 + w block by block; columns outside [0, Kb) contribute nothing.
+template <typename I>
+__device__ void band_group_generic(const I* __restrict__ brp, const I* __restrict__ bci,
+                                   const float* __restrict__ vals, const float* __restrict__ B,
+                                   float* __restrict__ C, int64_t M, int64_t K, int64_t N, int64_t Mb,
+                                   int64_t Kb, int64_t br0, int64_t n0, const I* __restrict__ row_map,
+                                   int64_t nc)
+{
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15, g = lane >> 4;
+    const int64_t br = br0 + (threadIdx.x >> 6);
+    if (br >= Mb) return;
+    float4_t acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const int64_t be = (int64_t)brp[br + 1];
+    for (int64_t b = (int64_t)brp[br]; b < be; ++b) {
+        const int64_t col = (int64_t)bci[b];
+        if (col < 0 || col >= Kb) continue;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float a = vals[b * 256 + li * 16 + 4 * g + s];
+            const int64_t k = 16 * col + 4 * g + s;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t n = n0 + 16 * j + li;
+                const float x = (k < K && n < N) ? B[k * N + n] : 0.f;
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x, acc[j], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int64_t n = n0 + 16 * j + li;
+        if (n >= nc) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t row = 16 * br + 4 * g + q;
+            if (row < M) C[(row_map ? (int64_t)row_map[row] : row) * nc + n] = acc[j][q];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // fp32 banded grids: spmm_f32_band_kernel.  v_mfma_f32_16x16x4f32 takes one K
 // index per lane group (lane (i, k) holds A[i][k] and B[k][i]), so B rows go
@@ -499,14 +560,19 @@ __global__ __launch_bounds__(1024) void band_plan_kernel(const I* __restrict__ b
 // Output tile j of a wave holds columns n0 + 4n + j (lane (n, g): rows
 // 4g .. 4g + 3), as in the fp32 column-batch kernel.  Each block-row must be
 // one contiguous run of block columns (spmm_band_wanted); N % 4 == 0, B and C
-// 16-byte aligned.  SPLIT: the balanced launch (grid P x chunks, with the plan
-// of band_plan_kernel); otherwise one group per workgroup.
-template <typename I, int L, bool SPLIT>
+// 16-byte aligned (nc < N columns of C, or C off 16 bytes, store one by one: B
+// is a copy with padded rows then).  SPLIT: the balanced launch (grid P x chunks,
+// with the plan of band_plan_kernel); otherwise one group per workgroup.
+// FULL: a grid with every block present (nnzb == Mb * Kb), whose block-rows are
+// contiguous runs too unless the caller stored its blocks in another order:
+// each workgroup checks its own block-rows first (1/256 of their bytes).
+template <typename I, int L, bool SPLIT, bool FULL>
 __global__ __launch_bounds__(256, 2) void spmm_f32_band_kernel(
     const I* __restrict__ brp, const I* __restrict__ bci, const float* __restrict__ vals,
     const float* __restrict__ B, float* __restrict__ C, int64_t M, int64_t K, int64_t N, int64_t Mb,
-    const I* __restrict__ row_map, BandSplit sp)
+    int64_t Kb, const I* __restrict__ row_map, int64_t nc, BandSplit sp)
 {
+    static_assert(!(SPLIT && FULL), "full grids load every workgroup alike");
     typedef float float4v_t __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float red[4 * 4 * 16 * 64];  // [wave][row][16][64]
     __shared__ int32_t s_first[4];
@@ -653,15 +719,28 @@ __global__ __launch_bounds__(256, 2) void spmm_f32_band_kernel(
         const int64_t br = grp * 4 + (e >> 8);
         const int64_t grow = br * 16 + ((e >> 4) & 15);
         const int64_t col = n0 + 4 * (e & 15);
-        if (br >= Mb || grow >= M || col >= N) return;
+        if (br >= Mb || grow >= M || col >= nc) return;
         const int64_t crow = row_map ? (int64_t)row_map[grow] : grow;
-        *reinterpret_cast<float4v_t*>(C + crow * N + col) = v;
+        float* const dst = C + crow * nc + col;
+        if ((nc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
+            *reinterpret_cast<float4v_t*>(dst) = v;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (col + i < nc) dst[i] = v[i];
+        }
     };
 
     if constexpr (!SPLIT) {
         const uint32_t G = gridDim.x;
         const uint32_t x8 = blockIdx.x & 7u;
         const uint32_t grp = kBandXcd ? x8 * (G >> 3) + min(x8, G & 7u) + (blockIdx.x >> 3) : blockIdx.x;
+        if constexpr (FULL) {
+            if (!band_group_is_full<I>(brp, bci, (int64_t)grp * 4, min((int64_t)4, Mb - (int64_t)grp * 4), Kb)) {
+                band_group_generic<I>(brp, bci, vals, B, C, M, K, N, Mb, Kb, (int64_t)grp * 4, n0, row_map, nc);
+                return;
+            }
+        }
         group_blocks(grp, 0, 0x7fffffff);
         for (int e = threadIdx.x; e < 4 * 16 * 16; e += 256) store_quad(grp, e, tile_quad(e));
     } else {
@@ -856,37 +935,46 @@ int band_split_mode()
 
 }  // namespace
 
+// us:
+//   balanced:  W + 25 us (plan kernel, schedule loads, hand-off), with
+//              W = nnzb N / (850 per us and CU x CUs), the rate the
+//              balanced launch keeps on the 16384^2 90 % band;
+//   one group: W / (q s), q the share of the grid's workgroup rounds that
+//              its G x chunks workgroups fill (two per CU), s = 1 - f^2 / 2
+//              the average group's share of the widest span on a band of
+//              fill f = nnzb / (Mb Kb) (0.76 at the 90 % band, 0.90 at 50 %).
+void spmm_band_f32_times(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, double* one, double* balanced)
+{
+    const double cus = (double)band_device_cus();
+    const double W = (double)nnzb * (double)N / (850.0 * cus);
+    const double wgs = (double)((Mb + 3) / 4) * (double)((N + 63) / 64), cap = 2.0 * cus;
+    const double q = wgs / (std::ceil(wgs / cap) * cap);
+    const double f = (double)nnzb / ((double)Mb * (double)Kb);
+    *one = W / (q * (1.0 - f * f / 2.0));
+    *balanced = W + 25.0;
+}
+
 template <typename I>
 bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const float* bvals, const float* B, float* C, int64_t N, const I* row_map,
-                        int64_t nnzb, hipStream_t s)
+                        int64_t nnzb, hipStream_t s, int64_t nc)
 {
-    if (!spmm_band_f32_covers(K, Kb, Mb, N, B, C)) return false;
+    if (!spmm_band_f32_covers(K, Kb, Mb, N, B, nc > 0 ? nullptr : C)) return false;
+    if (nc <= 0) nc = N;
     const int64_t G = (Mb + 3) / 4;
     const int64_t chunks = (N + 63) / 64;
     const int64_t P = std::min<int64_t>(kPlanSlots, ((int64_t)band_device_cus() + 7) / 8 * 8);
     const size_t tile_bytes = (size_t)chunks * 2 * (size_t)P * kBandPart32 * sizeof(float);
     // The balanced launch (on grids of at most kPlanGroups groups) where the
-    // one-group-per-workgroup launch is predicted to take 10 % longer:
-    //   balanced:  W + 25 us (plan kernel, schedule loads, hand-off), with
-    //              W = nnzb N / (850 per us and CU x CUs), the rate the
-    //              balanced launch keeps on the 16384^2 90 % band;
-    //   one group: W / (q s), q the share of the grid's workgroup rounds that
-    //              its G x chunks workgroups fill (two per CU), s = 1 - f^2 / 2
-    //              the average group's share of the widest span on a band of
-    //              fill f = nnzb / (Mb Kb) (0.76 at the 90 % band, 0.90 at 50 %).
+    // one-group-per-workgroup launch is predicted to take 10 % longer.
     // Measured rule: it picks the faster launch on every band of 4096^2 to
     // 16384^2 and N of 64 to 256 timed both ways.
     const int mode = band_split_mode();
     bool pays = false;
     if (mode == 1) {
-        const double cus = (double)band_device_cus();
-        const double W = (double)nnzb * (double)N / (850.0 * cus);
-        const double wgs = (double)G * (double)chunks, cap = 2.0 * cus;
-        const double q = wgs / (std::ceil(wgs / cap) * cap);
-        const double f = (double)nnzb / ((double)Mb * (double)Kb);
-        const double sp_share = 1.0 - f * f / 2.0;
-        pays = W / (q * sp_share) > 1.1 * (W + 25.0);
+        double one, balanced;
+        spmm_band_f32_times(Mb, Kb, nnzb, N, &one, &balanced);
+        pays = one > 1.1 * balanced;
     }
     if (mode > 0 && nnzb > 0 && (mode == 2 || pays) && G <= kPlanGroups && tile_bytes <= (size_t(512) << 20)) {
         Carve cv;
@@ -912,23 +1000,44 @@ bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* b
         hipLaunchKernelGGL((band_plan_kernel<I>), dim3(1), dim3(1024), 0, s, brp, bci, Mb, nnzb, sp,
                            (int32_t)chunks);
         XSPMM_LAUNCH_CHECK();
-        hipLaunchKernelGGL((spmm_f32_band_kernel<I, XSPMM_BAND_F32_DEPTH, true>), dim3((unsigned)P, (unsigned)chunks),
-                           dim3(256), 0, s, brp, bci, bvals, B, C, M, K, N, Mb, row_map, sp);
+        hipLaunchKernelGGL((spmm_f32_band_kernel<I, XSPMM_BAND_F32_DEPTH, true, false>),
+                           dim3((unsigned)P, (unsigned)chunks), dim3(256), 0, s, brp, bci, bvals, B, C, M, K, N,
+                           Mb, Kb, row_map, nc, sp);
         XSPMM_LAUNCH_CHECK();
         return true;
     }
     const dim3 grid((unsigned)G, (unsigned)chunks);
-    hipLaunchKernelGGL((spmm_f32_band_kernel<I, XSPMM_BAND_F32_DEPTH, false>), grid, dim3(256), 0, s, brp, bci,
-                       bvals, B, C, M, K, N, Mb, row_map, BandSplit{});
+    hipLaunchKernelGGL((spmm_f32_band_kernel<I, XSPMM_BAND_F32_DEPTH, false, false>), grid, dim3(256), 0, s, brp,
+                       bci, bvals, B, C, M, K, N, Mb, Kb, row_map, nc, BandSplit{});
     XSPMM_LAUNCH_CHECK();
     return true;
 }
+
+template <typename I>
+bool bcsr_spmm_full_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
+                        const float* bvals, const float* B, float* C, int64_t N, const I* row_map,
+                        hipStream_t s, int64_t nc)
+{
+    if (!spmm_band_f32_covers(K, Kb, Mb, N, B, nc > 0 ? nullptr : C)) return false;
+    const dim3 grid((unsigned)((Mb + 3) / 4), (unsigned)((N + 63) / 64));
+    hipLaunchKernelGGL((spmm_f32_band_kernel<I, XSPMM_BAND_F32_DEPTH, false, true>), grid, dim3(256), 0, s, brp,
+                       bci, bvals, B, C, M, K, N, Mb, Kb, row_map, nc > 0 ? nc : N, BandSplit{});
+    XSPMM_LAUNCH_CHECK();
+    return true;
+}
+#define XSPMM_FULL_F32(I)                                                                             \
+    template bool bcsr_spmm_full_f32<I>(int64_t, int64_t, int64_t, int64_t, const I*, const I*,        \
+                                        const float*, const float*, float*, int64_t, const I*,         \
+                                        hipStream_t, int64_t);
+XSPMM_FULL_F32(int32_t)
+XSPMM_FULL_F32(int64_t)
+#undef XSPMM_FULL_F32
 template bool bcsr_spmm_band_f32<int32_t>(int64_t, int64_t, int64_t, int64_t, const int32_t*,
                                           const int32_t*, const float*, const float*, float*, int64_t,
-                                          const int32_t*, int64_t, hipStream_t);
+                                          const int32_t*, int64_t, hipStream_t, int64_t);
 template bool bcsr_spmm_band_f32<int64_t>(int64_t, int64_t, int64_t, int64_t, const int64_t*,
                                           const int64_t*, const float*, const float*, float*, int64_t,
-                                          const int64_t*, int64_t, hipStream_t);
+                                          const int64_t*, int64_t, hipStream_t, int64_t);
 
 template bool bcsr_spmm_band_f16<int32_t>(int64_t, int64_t, int64_t, int64_t, const int32_t*,
                                           const int32_t*, const uint16_t*, const uint16_t*, float*,

@@ -668,8 +668,6 @@ __global__ __launch_bounds__(256, 4) void spmm_f32_packed_kernel(
 
 bool spmm_f32_batch_covers(int64_t K, int64_t Kb, int64_t N, const void* B, const void* C)
 {
-    const char* e = std::getenv("XSPMM_F32_KERNEL");
-    if (e && std::string(e) == "tile") return false;
     return N % 4 == 0 && N > 0 && K * N * 4 <= (int64_t(1) << 31) && Kb < (int64_t(1) << 21) &&
            (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 &&
            (N + 127) / 128 <= 65535;
