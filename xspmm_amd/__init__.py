@@ -166,6 +166,28 @@ def _stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+_TYPE_CODES = None  # torch dtype -> vcode / icode
+_raw_stream = None  # device index -> its current stream's handle
+
+
+def _call_tables():
+    """What each call would look up in torch again, looked up once."""
+    global _TYPE_CODES, _raw_stream
+    torch = _torch()
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+        lambda dev: torch.cuda.current_stream(dev).cuda_stream)
+    _TYPE_CODES = {torch.float16: F16, torch.float32: F32, torch.int32: I32, torch.int64: I64}
+    return _TYPE_CODES
+
+
+def _dense_ok(t, rows, cols, dtype, device):
+    """Whether t is plainly what _check_dense accepts: a contiguous
+    rows x cols tensor of `dtype` on `device` (fp16: 16-byte aligned).
+    Anything else goes through _check_dense, which decides and words errors."""
+    return (type(t) is _torch().Tensor and t.dtype is dtype and t.device == device and t.dim() == 2
+            and t.shape[0] == rows and t.shape[1] == cols and t.is_contiguous())
+
+
 def _device(dev=None):
     torch = _torch()
     if dev is None:
@@ -261,12 +283,17 @@ class BCSRMatrix:
     def num_blocks(self) -> int:
         return int(self.col_ind.numel())
 
+    def _layout_key(self):
+        rp, ci = self.row_ptr, self.col_ind
+        return (id(rp), rp.data_ptr(), rp._version, id(ci), ci.data_ptr(), ci._version,
+                self.num_block_rows)
+
     def dispatch_order(self):
         """The cached dispatch order for the current row_ptr (computed on
         first use), or None when Tier-1 does not order this grid."""
-        key = (id(self.row_ptr), self.row_ptr.data_ptr(), self.row_ptr._version,
-               id(self.col_ind), self.col_ind.data_ptr(), self.col_ind._version,
-               int(self.num_block_rows))
+        return self._find_order(self._layout_key())
+
+    def _find_order(self, key):
         if self._order_key != key:
             torch = _torch()
             order = torch.empty(int(self.num_block_rows) + 1, dtype=torch.int32,
@@ -283,9 +310,9 @@ class BCSRMatrix:
     def band_rows(self) -> bool:
         """Whether Tier-1 multiplies this grid with a band kernel (decided on
         first use for the current row_ptr and col_ind)."""
-        key = (id(self.row_ptr), self.row_ptr.data_ptr(), self.row_ptr._version,
-               id(self.col_ind), self.col_ind.data_ptr(), self.col_ind._version,
-               int(self.num_block_rows))
+        return self._find_band(self._layout_key())
+
+    def _find_band(self, key):
         if self._band_key != key:
             band = C.c_int(0)
             if self.r_block == 16 and self.c_block == 16:
@@ -336,19 +363,42 @@ def spmm(A: BCSRMatrix, B, C_out=None, N: int | None = None):
     K x N row-major on the device; returns C (M x N fp32)."""
     torch = _torch()
     L = load()
+    codes = _TYPE_CODES or _call_tables()
     if N is None:
         N = int(B.shape[1]) if B.dim() == 2 else int(B.numel() // max(A.num_cols, 1))
-    dev = A.row_ptr.device
+    rp, ci, vals = A.row_ptr, A.col_ind, A.values
+    dev = rp.device
     if C_out is None:
         C_out = torch.empty((A.num_rows, N), dtype=torch.float32, device=dev)
-    _check_dense(B, "B", A.num_cols, N, A.values.dtype, dev)
-    _check_dense(C_out, "C_out", A.num_rows, N, torch.float32, dev)
-    band = A.band_rows()
-    order = A.dispatch_order()
-    _check(L.xspmm_bcsr_spmm_auto(vcode(B.dtype), icode(A.row_ptr.dtype), A.num_rows, A.num_cols,
-                                  A.num_block_rows, A.num_block_cols, A.num_blocks, _ptr(A.row_ptr),
-                                  _ptr(A.col_ind), _ptr(A.values), _ptr(B), _ptr(C_out), N,
-                                  _ptr(order) if order is not None else None, int(band), None, 0, _stream()))
+    vt = vals.dtype
+    if not (_dense_ok(B, A.num_cols, N, vt, dev) and (vt is torch.float32 or B.data_ptr() % 16 == 0)):
+        _check_dense(B, "B", A.num_cols, N, vt, dev)
+    if not _dense_ok(C_out, A.num_rows, N, torch.float32, dev):
+        _check_dense(C_out, "C_out", A.num_rows, N, torch.float32, dev)
+    key = A._layout_key()
+    band = A._band if A._band_key == key else A._find_band(key)
+    order = A._order if A._order_key == key else A._find_order(key)
+    # rows of B off 16 bytes: a product may take a padded copy of B (and, on a
+    # long grid, an order), from torch's allocator, which costs a tenth of the
+    # library's own stream-ordered allocation.  Freed on this stream when the
+    # call returns, so only later work of the same stream reuses it.
+    vec = 8 if vt is torch.float16 else 4
+    ws, ws_bytes = None, 0
+    cur = torch.cuda.current_device()
+    if N % vec and dev.index == cur:
+        ws_bytes = 1024 + A.num_cols * (N + vec) * (16 // vec) + 4 * A.num_block_rows
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    # (an empty tensor's address is not passed on)
+    rc = L.xspmm_bcsr_spmm_auto(codes[vt] if vt in codes else vcode(vt),
+                                codes[rp.dtype] if rp.dtype in codes else icode(rp.dtype), A.num_rows, A.num_cols,
+                                A.num_block_rows, A.num_block_cols, ci.numel(), rp.data_ptr(),
+                                ci.data_ptr() or None, vals.data_ptr() or None, B.data_ptr() or None,
+                                C_out.data_ptr() or None, N,
+                                order.data_ptr() if order is not None else None, 1 if band else 0,
+                                ws.data_ptr() if ws is not None else None, ws_bytes,
+                                _raw_stream(cur))
+    if rc != OK:
+        _check(rc)
     return C_out
 
 
@@ -522,13 +572,20 @@ class SpMMPlan:
         torch = _torch()
         if self._h is None:
             raise RuntimeError("SpMMPlan is closed")
+        _TYPE_CODES or _call_tables()
         if N is None:
             N = int(B.shape[1])
+        dev, vt = self.device, self.value_dtype
         if C_out is None:
-            C_out = torch.empty((self.num_rows, N), dtype=torch.float32, device=self.device)
-        _check_dense(B, "B", self.num_cols, N, self.value_dtype, self.device)
-        _check_dense(C_out, "C_out", self.num_rows, N, torch.float32, self.device)
-        _check(self._L.xspmm_plan_execute(self._h, _ptr(B), _ptr(C_out), N, _stream()))
+            C_out = torch.empty((self.num_rows, N), dtype=torch.float32, device=dev)
+        if not (_dense_ok(B, self.num_cols, N, vt, dev) and (vt is torch.float32 or B.data_ptr() % 16 == 0)):
+            _check_dense(B, "B", self.num_cols, N, vt, dev)
+        if not _dense_ok(C_out, self.num_rows, N, torch.float32, dev):
+            _check_dense(C_out, "C_out", self.num_rows, N, torch.float32, dev)
+        rc = self._L.xspmm_plan_execute(self._h, B.data_ptr() or None, C_out.data_ptr() or None, N,
+                                        _raw_stream(torch.cuda.current_device()))
+        if rc != OK:
+            _check(rc)
         return C_out
 
     def close(self):
