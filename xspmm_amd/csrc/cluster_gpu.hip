@@ -36,7 +36,7 @@
 // 64 words per row), their popcounts, each row's block list, the per-block
 // row lists (counts, exclusive scan, scatter) and each row's partners --
 // the rows close enough to join it while the pattern is still its own, by
-// all pairs on the int8 matrix cores or through the row lists.  A seed whose partners are
+// all pairs on the fp4 matrix cores or through the row lists.  A seed whose partners are
 // all clustered forms a cluster of one without a scan, and any other seed
 // starts its scan at its highest-positioned partner.
 #include <cstdlib>
@@ -453,85 +453,82 @@ __global__ __launch_bounds__(256) void partners_bitmap_kernel(const uint64_t* __
     }
 }
 
-// All pairs on the int8 matrix cores: |q_i & q_j| is entry (i, j) of the
-// Gram matrix Q Q^T of the 0/1 row bitmaps, an exact integer dot product.
+// All pairs on the fp4 matrix cores: |q_i & q_j| is entry (i, j) of the
+// Gram matrix Q Q^T of the 0/1 row bitmaps, an exact dot product.
 // A workgroup of four waves takes a 128 x 128 tile (rows i of tile ti, rows
-// j of tile tj >= ti: the upper triangle, numbered row by row), each wave a
-// 64 x 64 quarter as 4 x 4 products v_mfma_i32_16x16x64_i8.  The tile's
-// 256 bitmap rows and their counts are staged in LDS first (rows padded to
-// 4 NQ + 1 words for W <= 4 NQ, the words past W zero; the odd stride
-// spreads a read's 16 rows over the banks).  Lane group g of a wave reads word 4q + g
-// of its rows for word quad q and spreads 16 of its bits per product into
-// 16 bytes 0 / -1.  The A and B operands of a product come from the same
-// spreading of the same word, so whatever K order the instruction's lane
-// layout implies, it pairs equal bits of q_i and q_j, and (-1)(-1) = 1.
+// j of tile tj >= ti: the upper triangle), each wave a
+// 64 x 64 quarter as 4 x 4 products v_mfma_scale_f32_16x16x128_f8f6f4.  The
+// tile's 256 bitmap rows and their counts are staged in LDS first (rows of 8 NS
+// words for W <= 8 NS, the words past W zero).  Lane group g of a wave reads words
+// 8s + 2g and 8s + 2g + 1 of its rows for step s: 128 bits, one of every four
+// consecutive ones in each of four products.  A bit becomes an e2m1 value by
+// masking alone: the bits of mask 0x1.., 0x2.. and 0x4.. stand for 0.5, 1 and 2,
+// the fourth set (moved down by one) for 2 again, and the product's block scale
+// makes each of them 1.  The A and B operands of a product come from the same
+// masking of the same words, so whatever K order the instruction's lane layout
+// implies, it pairs equal bits of q_i and q_j.  Sums are whole numbers below
+// 2^12, exact in the fp32 accumulators.
 // Every pair j > i of the tile whose product passes a cheap bound (below)
 // gets the exact Jaccard test in the accumulator layout (lane (l, g) holds
 // rows 4g .. 4g+3 of column l of each 16 x 16 block), and a close pair is
 // listed for both rows, as in the popcount kernel.
+// Per 128 bits of a row, 5 vector operations per dword make the operands of 64
+// products of 16 cycles, so a tile is bound by its start (rows out of L2, three
+// workgroups to a CU to cover it) rather than by the matrix cores: 16384 rows of
+// 1024 bits 134 -> 90 us, 6758 rows 72 -> 56, against the int8 form (twice the
+// products, 16 operations per dword, half of them 64-bit shifts).  Two or four
+// tiles per workgroup in turn were slower (112 to 175 us).
 constexpr int kGramTile = 128;
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-
-// bits 15-s, 31-s, 47-s and 63-s of w (0 <= s < 16) as four bytes 0 or -1:
-// v_perm_b32 selectors 8..11 replicate the top bits of bytes 1, 3, 5 and 7.
-// One 64-bit shift per dword (the compiler would split it into two 32-bit
-// operations).
-template <int S>
-__device__ __forceinline__ int spread_bits(uint64_t w)
-{
-    static_assert(S >= 0 && S < 16, "shift of 0 .. 15");
-    uint64_t y = w;
-    if constexpr (S != 0) asm("v_lshlrev_b64 %0, %1, %2" : "=v"(y) : "i"(S), "v"(w));
-    return (int)__builtin_amdgcn_perm((uint32_t)(y >> 32), (uint32_t)y, 0x0b0a0908u);
-}
-// the 16 bytes of bits 16 C .. 16 C + 15 of the spreading order
-template <int C>
-__device__ __forceinline__ i32x4_t spread_chunk(uint64_t w)
-{
-    return i32x4_t{spread_bits<4 * C>(w), spread_bits<4 * C + 1>(w), spread_bits<4 * C + 2>(w),
-                   spread_bits<4 * C + 3>(w)};
-}
-
-// NQ: word quads per row (W <= 4 NQ)
-template <int NQ>
-__global__ __launch_bounds__(256, 3) void partners_gram_kernel(const uint64_t* __restrict__ bits,
+// NS: steps of eight words per row (W <= 8 NS)
+template <int NS>
+__global__ __launch_bounds__(256, NS <= 2 ? 3 : 2) void partners_gram_kernel(const uint64_t* __restrict__ bits,
                                                              const int32_t* __restrict__ count,
                                                              int M, int W, int T, float thr,
                                                              int32_t* pn, int32_t* partners)
 {
-    constexpr int wp = 4 * NQ + 1;
-    __shared__ uint64_t gram_lds[2 * kGramTile * wp + kGramTile];  // words, then 256 counts
-    // tile (ti, tj): row t of the triangle holds T - t tiles, so the rows
-    // above t hold start(t) = t T - t (t - 1) / 2; ti is the largest t with
-    // start(t) <= id (the smaller root of start(t) = id, then corrected)
-    const int64_t id = blockIdx.x;
-    auto start = [&](int64_t t) { return t * T - t * (t - 1) / 2; };
-    const double b2 = 2.0 * T + 1.0;
-    int64_t ti = (int64_t)((b2 - sqrt(fmax(b2 * b2 - 8.0 * (double)id, 0.0))) * 0.5);
-    ti = min(max(ti, (int64_t)0), (int64_t)T - 1);
-    while (ti > 0 && start(ti) > id) --ti;
-    while (ti + 1 < T && start(ti + 1) <= id) ++ti;
-    const int64_t tj = ti + (id - start(ti));
+    // a row's 16-byte chunk c is kept at chunk c ^ swz(row): the 16 rows that one
+    // read touches then lie on 64 different banks
+    constexpr int kChunks = 4 * NS;
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) u32x4_t gram_lds[2 * kGramTile * kChunks];
+    __shared__ __align__(16) int32_t lcount[2 * kGramTile];
+    auto swz = [](int row) { return (row / (4 / NS)) & (kChunks - 1); };
+    // tile (ti, tj) of the triangle tj >= ti (T x T grid: the rest leaves)
+    const int ti = (int)blockIdx.x;
+    const int tj = ti + (int)blockIdx.y;
+    if (tj >= T) return;
 
-    // stage rows i (local 0..127) and rows j (local 128..255): four threads
-    // per row, each taking every fourth word; rows past M read as zeros
-    int32_t* const lcount = reinterpret_cast<int32_t*>(gram_lds + 2 * kGramTile * wp);
-    {
-        const int t = threadIdx.x;
-        for (int rr = t >> 2; rr < 2 * kGramTile; rr += 64) {
-            const int64_t row = rr < kGramTile ? ti * kGramTile + rr : tj * kGramTile + rr - kGramTile;
-            const bool valid = row < M;
-            const uint64_t* src = bits + (valid ? row : 0) * W;
+    // rows of a tile: two threads per row, thread h of a row takes chunks h, h +
+    // 2, ...; rows past M and words past W are zeros
+    const int srow = threadIdx.x >> 1, sh = threadIdx.x & 1;
+    auto load_rows = [&](int tile, u32x4_t (&v)[2 * NS], int& c) __attribute__((always_inline)) {
+        const int64_t row = (int64_t)tile * kGramTile + srow;
+        const bool valid = row < M;
+        const uint64_t* src = bits + (valid ? row : 0) * W;
 #pragma unroll
-            for (int u = 0; u < NQ; ++u) {
-                const int w = 4 * u + (t & 3);
-                gram_lds[rr * wp + w] = valid && w < W ? src[w] : 0ULL;
-            }
+        for (int u = 0; u < 2 * NS; ++u) {
+            const int w = 2 * (2 * u + sh);
+            const uint64_t x = valid && w < W ? src[w] : 0ULL;
+            const uint64_t y = valid && w + 1 < W ? src[w + 1] : 0ULL;
+            v[u] = u32x4_t{(uint32_t)x, (uint32_t)(x >> 32), (uint32_t)y, (uint32_t)(y >> 32)};
         }
-        const int64_t row = t < kGramTile ? ti * kGramTile + t : tj * kGramTile + t - kGramTile;
-        lcount[t] = row < M ? count[row] : 0;
-    }
+        c = valid ? count[row] : 0;
+    };
+    auto store_rows = [&](int at, const u32x4_t (&v)[2 * NS], int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2 * NS; ++u) gram_lds[(at + srow) * kChunks + ((2 * u + sh) ^ swz(srow))] = v[u];
+        if (sh == 0) lcount[at + srow] = c;
+    };
+    u32x4_t vi[2 * NS], vj[2 * NS];
+    int ci, cj;
+    load_rows(ti, vi, ci);
+    load_rows(tj, vj, cj);
+    store_rows(0, vi, ci);
+    store_rows(kGramTile, vj, cj);
     __syncthreads();
 
     const int lane = threadIdx.x & 63;
@@ -539,104 +536,125 @@ __global__ __launch_bounds__(256, 3) void partners_gram_kernel(const uint64_t* _
     const int li = lane & 15, g = lane >> 4;
     const int il0 = (wave >> 1) * 64;               // local row of the quarter's first i
     const int jl0 = kGramTile + (wave & 1) * 64;    // and of its first j
-    const int64_t i0 = ti * kGramTile + il0;
-    const int64_t j0 = tj * kGramTile + jl0 - kGramTile;
-    // a quarter wholly on or below the diagonal, or past the last row, holds
-    // no pair j > i (no barrier follows: the wave may leave)
-    if (j0 + 63 <= i0 || i0 >= M || j0 >= M) return;
+    const int64_t i0 = (int64_t)ti * kGramTile + il0;
 
     // Candidates.  close() holds only if inter >= RN(a_lo uni) >= a' uni
     // with a' = a_lo (1 - 2^-24) and uni = c_i + c_j - inter, that is only if
     // inter >= a' / (1 + a') (c_i + c_j).  beta rounds that factor down by
     // 2^-16 (more than its float roundings), so f = floor(beta c) gives
-    // f_i + f_j <= a' / (1 + a') (c_i + c_j): each accumulator starts at
-    // -(f_i + f_j), and a pair whose product ends below zero is not close.
+    // f_i + f_j <= a' / (1 + a') (c_i + c_j): a pair whose product is below
+    // f_i + f_j is not close.
     const JaccardTest jt(thr);
     const float beta = jt.a_lo > 0.0f ? jt.a_lo / (1.0f + jt.a_lo) * (1.0f - 0x1p-16f) : 0.0f;
-    int fi[4][4], fj[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        // rows il0 + 16 m + 4 g + r (r = 0..3) and row jl0 + 16 m + li
-        const int4 c4 = *reinterpret_cast<const int4*>(lcount + il0 + 16 * m + 4 * g);
-        fi[m][0] = (int)(beta * (float)c4.x);
-        fi[m][1] = (int)(beta * (float)c4.y);
-        fi[m][2] = (int)(beta * (float)c4.z);
-        fi[m][3] = (int)(beta * (float)c4.w);
-        fj[m] = (int)(beta * (float)lcount[jl0 + 16 * m + li]);
-    }
-    i32x4_t acc[4][4];
+    // (swz depends on a row's place in its 16 rows only: 16 / (4 / NS) >= kChunks
+    // rows repeat it)
+    const u32x4_t* const wi = gram_lds + (il0 + li) * kChunks;
+    const u32x4_t* const wj = gram_lds + (jl0 + li) * kChunks;
+
+    const int64_t j0 = (int64_t)tj * kGramTile + jl0 - kGramTile;
+    // a quarter wholly on or below the diagonal, or past the last row, holds
+    // no pair j > i
+    if (j0 + 63 <= i0 || i0 >= M || j0 >= M) return;
+    f32x4_t acc[4][4];
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
         for (int n = 0; n < 4; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[m][n][r] = -(fi[m][r] + fj[n]);
+            for (int r = 0; r < 4; ++r) acc[m][n][r] = 0.f;
 
-    const uint64_t* const wi = gram_lds + (il0 + li) * wp + g;
-    const uint64_t* const wj = gram_lds + (jl0 + li) * wp + g;
-    // (eight quads unrolled would need more than 256 registers)
-#pragma unroll(NQ > 4 ? 4 : NQ)
-    for (int q = 0; q < NQ; ++q) {
-        uint64_t a[4], b[4];
+#pragma unroll 1
+    for (int st = 0; st < NS; ++st) {
+        u32x4_t a[4], b[4];
+        const int c = (4 * st + g) ^ swz(li);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            a[m] = wi[16 * m * wp + 4 * q];
-            b[m] = wj[16 * m * wp + 4 * q];
+            a[m] = wi[16 * m * kChunks + c];
+            b[m] = wj[16 * m * kChunks + c];
         }
-        auto chunk = [&]<int C>() __attribute__((always_inline)) {
-            i32x4_t A[4], B[4];
+        // the bits of `mask`, each worth 1 after the block scale 2^(scale - 127)
+        // on both operands
+        auto product = [&](uint32_t mask, int scale) __attribute__((always_inline)) {
+            constexpr int kFp4 = 4;  // e2m1
+            i32x8_t B[4];
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int d = 0; d < 8; ++d) B[n][d] = d < 4 ? (int)(b[n][d & 3] & mask) : 0;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
-                A[m] = spread_chunk<C>(a[m]);
-                B[m] = spread_chunk<C>(b[m]);
-            }
+                // (in this order: hoisted operands would spill)
+                __builtin_amdgcn_sched_barrier(0);
+                i32x8_t A;
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
+                for (int d = 0; d < 8; ++d) A[d] = d < 4 ? (int)(a[m][d & 3] & mask) : 0;
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[m], B[n], acc[m][n], 0, 0, 0);
+                    acc[m][n] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B[n], acc[m][n], kFp4, kFp4,
+                                                                                 0, scale, 0, scale);
+            }
         };
-        chunk.template operator()<0>();
-        chunk.template operator()<1>();
-        chunk.template operator()<2>();
-        chunk.template operator()<3>();
+        product(0x11111111u, 128);  // 0.5
+        product(0x22222222u, 127);  // 1
+        product(0x44444444u, 126);  // 2
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                a[m][d] >>= 1;
+                b[m][d] >>= 1;
+            }
+        product(0x44444444u, 126);
     }
 
     // no candidate in the whole quarter (the usual case): done
+    // the bounds of rows il0 + 16 m + 4 g + r (r = 0..3) and of row jl0 + 16 n + li
+    auto bounds_i = [&](int m) __attribute__((always_inline)) -> i32x4_t {
+        const i32x4_t c4 = *reinterpret_cast<const i32x4_t*>(lcount + il0 + 16 * m + 4 * g);
+        return i32x4_t{(int)(beta * (float)c4[0]), (int)(beta * (float)c4[1]), (int)(beta * (float)c4[2]),
+                       (int)(beta * (float)c4[3])};
+    };
+    int fj[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) fj[n] = (int)(beta * (float)lcount[jl0 + 16 * n + li]);
     bool any = false;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < 4; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        const i32x4_t fi = bounds_i(m);
 #pragma unroll
         for (int n = 0; n < 4; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) any |= acc[m][n][r] >= 0;
-    if (!__any(any)) return;
-    // the partner counts of the quarter's rows as the epilogue starts (they
-    // only grow): pairs whose two lists had overflowed by then are skipped
-    // without a read; the others read the count again before an add
-    int pn_i[4][4], pn_j[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) pn_i[m][r] = partner_count(pn, min((int)i0 + 16 * m + 4 * g + r, M - 1));
-        pn_j[m] = partner_count(pn, min((int)j0 + 16 * m + li, M - 1));
+            for (int r = 0; r < 4; ++r) any |= (int)acc[m][n][r] >= fi[r] + fj[n];
     }
+    if (!__any(any)) return;
+    // the partner counts as a pass starts (they only grow): pairs whose two
+    // lists had overflowed by then are skipped without a read; the others
+    // read the count again before an add
+    int pn_j[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) pn_j[n] = partner_count(pn, min((int)j0 + 16 * n + li, M - 1));
     // every pair of the quarter has i < j < M (uniform)
     const bool interior = j0 >= i0 + 64 && j0 + 64 <= M;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < 4; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        const i32x4_t fi = bounds_i(m);
+        int pn_i[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pn_i[r] = partner_count(pn, min((int)i0 + 16 * m + 4 * g + r, M - 1));
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int n = 0; n < 4; ++n) {
-                if (acc[m][n][r] < 0) continue;
-                const int inter = acc[m][n][r] + fi[m][r] + fj[n];
+                const int inter = (int)acc[m][n][r];
+                if (inter < fi[r] + fj[n]) continue;
                 // row numbers fit 31 bits (M < 2^31)
                 const int i = (int)i0 + 16 * m + 4 * g + r;
                 const int j = (int)j0 + 16 * n + li;
                 if (!interior && (i >= M || j >= M || j <= i)) continue;
                 // both lists already overflowed: nothing to add
-                const int ni = pn_i[m][r], nj = pn_j[n];
+                const int ni = pn_i[r], nj = pn_j[n];
                 if (ni > kPartnerCap && nj > kPartnerCap) continue;
                 const int ci = lcount[il0 + 16 * m + 4 * g + r], cj = lcount[jl0 + 16 * n + li];
                 if (jt.close(inter, ci + cj - inter)) {  // partnership is symmetric
@@ -644,6 +662,7 @@ __global__ __launch_bounds__(256, 3) void partners_gram_kernel(const uint64_t* _
                     if (nj <= kPartnerCap && partner_count(pn, j) <= kPartnerCap) add_partner(pn, partners, j, i);
                 }
             }
+    }
 }
 
 // Pairs through the per-block row lists: one workgroup per row i counts
@@ -1289,9 +1308,9 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
         const int Mi = (int)M, Wi = (int)W;
         if (bitmap_partners && !popcount_partners) {
             const int64_t T = (M + kGramTile - 1) / kGramTile;
-            const dim3 g((unsigned)(T * (T + 1) / 2));
-            auto kern = W <= 4 ? partners_gram_kernel<1> : W <= 8 ? partners_gram_kernel<2>
-                      : W <= 16 ? partners_gram_kernel<4> : partners_gram_kernel<8>;
+            const dim3 g((unsigned)T, (unsigned)T);
+            auto kern = W <= 8 ? partners_gram_kernel<1> : W <= 16 ? partners_gram_kernel<2>
+                      : partners_gram_kernel<4>;
             hipLaunchKernelGGL(kern, g, dim3(256), 0, s, bits, count, Mi, Wi, (int)T, dist_thresh, pn,
                                partners);
         } else {
