@@ -351,8 +351,7 @@ __global__ void reversed_perm_kernel(I* perm, int64_t M)
         perm[i] = (I)(M - 1 - i);
 }
 
-// The row list total and the bad-column flag side by side, for one copy to
-// the host.
+// The row list total and the bad-column flag, for the host to read.
 __global__ void status_kernel(const int64_t* __restrict__ total, const int* __restrict__ bad,
                               int64_t* __restrict__ status)
 {
@@ -360,6 +359,17 @@ __global__ void status_kernel(const int64_t* __restrict__ total, const int* __re
         status[0] = *total;
         status[1] = *bad;
     }
+}
+
+// The sum of the squares of n counts, for the host to read (one workgroup).
+__global__ __launch_bounds__(kClThreads) void square_sum_kernel(const int32_t* __restrict__ c, int64_t n,
+                                                                int64_t* __restrict__ words)
+{
+    __shared__ int64_t red[kClWaves];
+    int64_t sq = 0;
+    for (int64_t i = threadIdx.x; i < n; i += kClThreads) sq += (int64_t)c[i] * c[i];
+    const int64_t total = block_sum64(sq, red);
+    if (threadIdx.x == 0) words[0] = total;
 }
 
 // --- partner lists -------------------------------------------------------------
@@ -1217,7 +1227,6 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
     const size_t o_cb = cv.take((size_t)M * sizeof(int32_t));
     const size_t o_plist = cv.take((size_t)nb * sizeof(int32_t));
     const size_t o_partners = cv.take((size_t)M * kPartnerCap * sizeof(int32_t));
-    const size_t o_status = cv.take(2 * sizeof(int64_t));
     Scratch tmp(cv.end, s);
     char* const base = tmp.as<char>();
     XSPMM_HIP_CHECK(hipMemsetAsync(base, 0, zeroed, s));
@@ -1287,22 +1296,16 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
     // row list offsets: their total, sum_b v_b = sum_i |q_i|, bounds the
     // engine estimate: (sum v_b)^2 / Kb <= sum v_b^2 <= sum v_b * min(M, sum v_b)
     device_exclusive_scan(ArrayValue<int32_t>{count}, M, rb_start, s);
-    int64_t* const status = reinterpret_cast<int64_t*>(base + o_status);
-    hipLaunchKernelGGL(status_kernel, dim3(1), dim3(64), 0, s, rb_start + M, bad, status);
+    HostWords words;
+    hipLaunchKernelGGL(status_kernel, dim3(1), dim3(64), 0, s, rb_start + M, bad, words.get());
     XSPMM_LAUNCH_CHECK();
-    // pinned, so that the copy does not hold the host: 16 bytes allocated
-    // once per host thread and never freed (a call reads them before it
-    // returns, so calls on one thread never share them)
-    thread_local int64_t* h_status = nullptr;
-    if (!h_status) XSPMM_HIP_CHECK(hipHostMalloc((void**)&h_status, 2 * sizeof(int64_t), hipHostMallocDefault));
-    XSPMM_HIP_CHECK(hipMemcpyAsync(h_status, status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     EventHandle copied;
     XSPMM_HIP_CHECK(hipEventRecord(copied.get(), s));
 
     // Partner lists (XSPMM_CLUSTER_PARTNERS=off leaves every seed on the
     // full path); pn starts at zero.  The all-pairs passes need only the
     // bitmaps and counts: they are enqueued before the host waits for the
-    // copy of the row list total, so the host decides and enqueues the rest
+    // row list total, so the host decides and enqueues the rest
     // while they run.  The row-list pass runs after the lists are built.
     if (use_partners && bitmap_partners) {
         const int Mi = (int)M, Wi = (int)W;
@@ -1326,8 +1329,9 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
     }
 
     XSPMM_HIP_CHECK(hipEventSynchronize(copied.get()));
-    const int64_t nrb = h_status[0];
-    h_bad = (int)h_status[1];
+    const int64_t nrb = words[0];
+    h_bad = (int)words[1];
+    words.release();
     check_bad();
     const double scan_work = 0.5 * (double)M * (double)M * (double)W;
     if (engine == kEngineAuto && Kb > 0) {
@@ -1341,12 +1345,12 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
         hipLaunchKernelGGL(block_counts_kernel, dim3((unsigned)((nb + kPrepThreads - 1) / kPrepThreads), (unsigned)gy),
                            dim3(kPrepThreads), 0, s, bits, M, W, Kb, bl_count);
         XSPMM_LAUNCH_CHECK();
-        std::vector<int32_t> h_bl((size_t)nb);
-        XSPMM_HIP_CHECK(hipMemcpyAsync(h_bl.data(), bl_count, (size_t)nb * sizeof(int32_t),
-                                       hipMemcpyDeviceToHost, s));
+        HostWords sums;
+        hipLaunchKernelGGL(square_sum_kernel, dim3(1), dim3(kClThreads), 0, s, bl_count, Kb, sums.get());
+        XSPMM_LAUNCH_CHECK();
         XSPMM_HIP_CHECK(hipStreamSynchronize(s));
-        int64_t sq = 0;
-        for (int64_t b = 0; b < Kb; ++b) sq += (int64_t)h_bl[(size_t)b] * h_bl[(size_t)b];
+        const int64_t sq = sums[0];
+        sums.release();
         // the same estimate as the host engines: index ~ 3 * sum v_b^2
         // counter updates, scan ~ M^2 * W / 2 word tests
         engine = 3.0 * (double)sq < scan_work ? kEngineIndex : kEngineScan;
@@ -1394,8 +1398,12 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
     hipLaunchKernelGGL(cluster_kernel<I>, dim3(1), dim3(kClThreads), 0, s, args, perm);
     XSPMM_LAUNCH_CHECK();
     if (engine_used) {
-        XSPMM_HIP_CHECK(hipMemcpyAsync(engine_used, bad + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+        HostWords used;
+        hipLaunchKernelGGL(status_kernel, dim3(1), dim3(64), 0, s, rb_start, bad + 1, used.get());
+        XSPMM_LAUNCH_CHECK();
         XSPMM_HIP_CHECK(hipStreamSynchronize(s));
+        *engine_used = (int)used[1];
+        used.release();
     }
 }
 

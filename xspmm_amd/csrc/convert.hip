@@ -853,14 +853,52 @@ __global__ __launch_bounds__(kThreads) void pack32_emit_kernel(
 
 }  // namespace
 
+namespace {
+
+// The block count and the error flag, for the host to read.
+template <typename I>
+__global__ void count_words_kernel(const I* __restrict__ total, const int* __restrict__ err, int64_t* __restrict__ words)
+{
+    if (threadIdx.x == 0) {
+        words[0] = (int64_t)*total;
+        words[1] = (int64_t)*err;
+    }
+}
+
+__global__ void copy_words_kernel(const int64_t* __restrict__ from, int n, int64_t* __restrict__ words)
+{
+    if ((int)threadIdx.x < n) words[threadIdx.x] = from[threadIdx.x];
+}
+
+// counts holds Mb entries.
+template <typename I>
+void count_blocks(const ConvGeometry& g, int64_t M, int64_t K, int64_t nnz, const I* rp, const I* ci, int64_t rb,
+                  int64_t cb, I* counts, I* brp, int* err, hipStream_t s)
+{
+    hipLaunchKernelGGL(set_value_kernel<int>, dim3(1), dim3(64), 0, s, err, 0);
+    XSPMM_LAUNCH_CHECK();
+    if (g.Mb > 0) {
+        hipLaunchKernelGGL(conv_count_kernel<I>, dim3((unsigned)g.Mb), dim3(kThreads), g.count_lds,
+                           s, M, K, nnz, rp, ci, rb, cb, g.nwords, counts, err);
+        XSPMM_LAUNCH_CHECK();
+    }
+    device_exclusive_scan(ArrayValue<I>{counts}, g.Mb, brp, s);
+}
+
+}  // namespace
+
 template <typename I>
 int64_t csr_to_bcsr_count(int64_t M, int64_t K, int64_t nnz, const I* rp, const I* ci,
                           int64_t rb, int64_t cb, I* brp, hipStream_t s)
 {
     const ConvGeometry g = conv_geometry(M, K, nnz, rb, cb);  // argument checks first
-    Scratch err(sizeof(int), s);
-    csr_to_bcsr_count_async<I>(M, K, nnz, rp, ci, rb, cb, brp, err.as<int>(), s);
-    return csr_to_bcsr_result<I>(brp, g.Mb, err.as<int>(), s);
+    Carve cv;
+    const size_t o_err = cv.take(sizeof(int));
+    const size_t o_counts = cv.take((size_t)(g.Mb > 0 ? g.Mb : 1) * sizeof(I));
+    Scratch tmp(cv.end, s);
+    int* const err = reinterpret_cast<int*>(tmp.as<char>() + o_err);
+    count_blocks<I>(g, M, K, nnz, rp, ci, rb, cb, reinterpret_cast<I*>(tmp.as<char>() + o_counts), brp, err, s);
+    return csr_to_bcsr_result<I>(brp, g.Mb, err, s);
 }
 
 template <typename I>
@@ -869,28 +907,23 @@ void csr_to_bcsr_count_async(int64_t M, int64_t K, int64_t nnz, const I* rp, con
 {
     const ConvGeometry g = conv_geometry(M, K, nnz, rb, cb);
     Scratch counts((size_t)(g.Mb > 0 ? g.Mb : 1) * sizeof(I), s);
-    hipLaunchKernelGGL(set_value_kernel<int>, dim3(1), dim3(64), 0, s, err, 0);
-    XSPMM_LAUNCH_CHECK();
-    if (g.Mb > 0) {
-        hipLaunchKernelGGL(conv_count_kernel<I>, dim3((unsigned)g.Mb), dim3(kThreads), g.count_lds,
-                           s, M, K, nnz, rp, ci, rb, cb, g.nwords, counts.as<I>(), err);
-        XSPMM_LAUNCH_CHECK();
-    }
-    device_exclusive_scan(ArrayValue<I>{counts.as<I>()}, g.Mb, brp, s);
+    count_blocks<I>(g, M, K, nnz, rp, ci, rb, cb, counts.as<I>(), brp, err, s);
 }
 
 template <typename I>
 int64_t csr_to_bcsr_result(const I* brp, int64_t Mb, const int* err, hipStream_t s)
 {
-    I nnzb = 0;
-    int bad = 0;
-    XSPMM_HIP_CHECK(hipMemcpyAsync(&nnzb, brp + Mb, sizeof(I), hipMemcpyDeviceToHost, s));
-    XSPMM_HIP_CHECK(hipMemcpyAsync(&bad, err, sizeof(int), hipMemcpyDeviceToHost, s));
+    HostWords words;
+    hipLaunchKernelGGL(count_words_kernel<I>, dim3(1), dim3(64), 0, s, brp + Mb, err, words.get());
+    XSPMM_LAUNCH_CHECK();
     XSPMM_HIP_CHECK(hipStreamSynchronize(s));
+    const int64_t nnzb = words[0];
+    const bool bad = words[1] != 0;
+    words.release();
     if (bad)
         throw std::invalid_argument(
             "csr_to_bcsr: invalid CSR (column index outside [0, K) or bad row_ptr).");
-    return (int64_t)nnzb;
+    return nnzb;
 }
 
 template <typename T, typename I>
@@ -979,10 +1012,13 @@ void csr_pack_analyse(int64_t M, int64_t K, int64_t nnz, const I* rp, const I* c
 
 PackStatus csr_pack_status(const int64_t* status, hipStream_t s)
 {
-    int64_t h[5] = {0, 0, 0, 0, 0};
-    XSPMM_HIP_CHECK(hipMemcpyAsync(h, status, sizeof(h), hipMemcpyDeviceToHost, s));
+    HostWords words;
+    hipLaunchKernelGGL(copy_words_kernel, dim3(1), dim3(64), 0, s, status, 5, words.get());
+    XSPMM_LAUNCH_CHECK();
     XSPMM_HIP_CHECK(hipStreamSynchronize(s));
-    return PackStatus{h[0], h[1], (int)h[2], (unsigned)h[3], h[4] != 0};
+    const PackStatus st{words[0], words[1], (int)words[2], (unsigned)words[3], words[4] != 0};
+    words.release();
+    return st;
 }
 
 template <typename I, typename V>

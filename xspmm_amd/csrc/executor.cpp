@@ -4,6 +4,7 @@
 #include <mutex>
 #include <new>
 #include <set>
+#include <vector>
 
 #include "internal.hpp"
 
@@ -97,4 +98,38 @@ void init_device_pool(int device)
 }
 
 }  // namespace detail
+// ---------------------------------------------------------------------------
+// Pinned words (internal.hpp): 64 slots to a 4 KB page, kept for the process.
+// ---------------------------------------------------------------------------
+namespace detail {
+namespace {
+std::mutex g_words_mu;
+std::vector<int64_t*>& free_words()
+{
+    static auto* v = new std::vector<int64_t*>;  // outlives every static destructor
+    return *v;
+}
+}  // namespace
+
+HostWords::HostWords()
+{
+    std::lock_guard<std::mutex> lock(g_words_mu);
+    auto& free = free_words();
+    if (free.empty()) {
+        void* page = nullptr;
+        XSPMM_HIP_CHECK(hipHostMalloc(&page, 4096, hipHostMallocPortable | hipHostMallocMapped));
+        for (int i = 63; i >= 0; --i) free.push_back(static_cast<int64_t*>(page) + 8 * i);
+    }
+    p_ = free.back();
+    free.pop_back();
+}
+
+void HostWords::release()
+{
+    std::lock_guard<std::mutex> lock(g_words_mu);
+    free_words().push_back(p_);
+    p_ = nullptr;
+}
+}  // namespace detail
+
 }  // namespace xspmm

@@ -153,6 +153,26 @@ private:
     std::vector<Scratch> owned_;
 };
 
+// Eight words of pinned host memory that a kernel writes and the host reads
+// after waiting for the stream: a result read back without a copy (a copy into
+// pageable memory costs about 25 us of host time, a launch 3).  Slots come from
+// pinned pages shared by all threads and devices, as many as calls were ever
+// waiting at once; release() hands the slot back once the stream has been
+// waited for (a slot that an error leaves behind is not used again, since the
+// kernel might still write it).
+class HostWords {
+public:
+    HostWords();
+    HostWords(const HostWords&) = delete;
+    HostWords& operator=(const HostWords&) = delete;
+    int64_t* get() const { return p_; }
+    int64_t operator[](int i) const { return const_cast<const volatile int64_t*>(p_)[i]; }
+    void release();
+
+private:
+    int64_t* p_;
+};
+
 // Elapsed times of stages bracketed by HIP events on stream s.  start() and
 // stop() only record the events, so the host goes on to the next stage
 // while the GPU runs this one; finish() waits for the last stop and writes

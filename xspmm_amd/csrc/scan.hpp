@@ -1,6 +1,7 @@
 // scan.hpp -- device-wide exclusive prefix sum of n values produced by a
-// functor, written as out[0..n] (out[n] = total).  Reduce-then-scan over
-// 2048-element tiles: tile sums -> one-workgroup scan of the sums -> tile scan.
+// functor, written as out[0..n] (out[n] = total).  Up to kScanOneMax values one
+// workgroup scans them all; above, reduce-then-scan over 2048-element tiles:
+// tile sums -> one-workgroup scan of the sums -> tile scan.
 // Used for bcsr_row_ptr (block counts per strip) and for the permuted
 // row_ptr (row lengths gathered through perm).
 #pragma once
@@ -111,6 +112,68 @@ __global__ __launch_bounds__(kScanThreads) void scan_final_kernel(F f, int64_t n
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = (I)partials[gridDim.x];
 }
 
+// Up to kScanOneMax values by one workgroup: every value is read up front (one
+// round of memory latency however the functor chains its loads), four
+// consecutive ones per thread and tile of 4096; the tiles' wave sums are scanned
+// together, so the kernel has two barriers.  Bound by latency: 16384 row lengths
+// through a permutation 8 us, where the three kernels above took 14 and the host
+// 25 more for their launches and the allocation of the tile sums.
+constexpr int kScanOneThreads = 1024;
+constexpr int kScanOneTile = 4 * kScanOneThreads;
+constexpr int kScanOneTiles = 8;
+constexpr int64_t kScanOneMax = (int64_t)kScanOneTile * kScanOneTiles;
+template <typename F, typename I>
+__global__ __launch_bounds__(kScanOneThreads) void scan_one_kernel(F f, int64_t n, I* out)
+{
+    constexpr int kWaves = kScanOneThreads / 64;
+    __shared__ int64_t sums[kScanOneTiles * kWaves + 1];  // [tile][wave], then exclusive
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    int64_t v[kScanOneTiles][4];
+#pragma unroll
+    for (int t = 0; t < kScanOneTiles; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t i = (int64_t)t * kScanOneTile + 4 * threadIdx.x + e;
+            v[t][e] = i < n ? f(i) : 0;
+        }
+    int64_t incl[kScanOneTiles];
+#pragma unroll
+    for (int t = 0; t < kScanOneTiles; ++t) incl[t] = v[t][0] + v[t][1] + v[t][2] + v[t][3];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+        for (int t = 0; t < kScanOneTiles; ++t) {
+            const int64_t x = __shfl_up(incl[t], d, 64);
+            if (lane >= d) incl[t] += x;
+        }
+    if (lane == 63)
+#pragma unroll
+        for (int t = 0; t < kScanOneTiles; ++t) sums[t * kWaves + wave] = incl[t];
+    __syncthreads();
+    if (wave == 0) {
+        // 128 sums, two per lane
+        static_assert(kScanOneTiles * kWaves == 128, "two sums per lane");
+        const int64_t a = sums[2 * lane], b = sums[2 * lane + 1];
+        const int64_t ex = wave_inclusive_scan(a + b) - (a + b);
+        sums[2 * lane] = ex;
+        sums[2 * lane + 1] = ex + a;
+        if (lane == 63) sums[128] = ex + a + b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kScanOneTiles; ++t) {
+        int64_t run = sums[t * kWaves + wave] + incl[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t i = (int64_t)t * kScanOneTile + 4 * threadIdx.x + e;
+            if (i < n) out[i] = (I)run;
+            run += v[t][e];
+        }
+    }
+    if (threadIdx.x == 0) out[n] = (I)sums[128];
+}
+
 template <typename I>
 __global__ void set_value_kernel(I* p, I v)
 {
@@ -129,6 +192,11 @@ void device_exclusive_scan(F f, int64_t n, I* out, hipStream_t s)
 {
     if (n <= 0) {
         hipLaunchKernelGGL(set_value_kernel<I>, dim3(1), dim3(64), 0, s, out, (I)0);
+        XSPMM_LAUNCH_CHECK();
+        return;
+    }
+    if (n <= kScanOneMax) {
+        hipLaunchKernelGGL((scan_one_kernel<F, I>), dim3(1), dim3(kScanOneThreads), 0, s, f, n, out);
         XSPMM_LAUNCH_CHECK();
         return;
     }

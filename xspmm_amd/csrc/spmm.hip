@@ -1408,7 +1408,8 @@ __global__ __launch_bounds__(kOrderThreads) void order_rows_kernel(const I* __re
 // and order[Mb] = 1 for the XCD ranges, 0 for the identity
 template <typename I>
 __global__ __launch_bounds__(256) void order_local_kernel(const I* __restrict__ brp, const I* __restrict__ bci,
-                                                          int64_t Mb, int32_t* __restrict__ order)
+                                                          int64_t Mb, int32_t* __restrict__ order,
+                                                          int64_t* __restrict__ words)
 {
     __shared__ int s_alike;
     const int t = threadIdx.x;
@@ -1438,7 +1439,10 @@ __global__ __launch_bounds__(256) void order_local_kernel(const I* __restrict__ 
         }
         order[i] = (int32_t)br;
     }
-    if (t == 0) order[Mb] = xcd ? 1 : 0;
+    if (t == 0) {
+        order[Mb] = xcd ? 1 : 0;
+        words[0] = xcd ? 1 : 0;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1929,12 +1933,13 @@ bool spmm_dispatch_order_cols(const I* brp, const I* bci, int64_t Mb, int32_t* o
         XSPMM_LAUNCH_CHECK();
         return true;
     }
-    hipLaunchKernelGGL((order_local_kernel<I>), dim3(1), dim3(256), 0, s, brp, bci, Mb, order);
+    HostWords words;
+    hipLaunchKernelGGL((order_local_kernel<I>), dim3(1), dim3(256), 0, s, brp, bci, Mb, order, words.get());
     XSPMM_LAUNCH_CHECK();
-    int32_t used = 0;
-    XSPMM_HIP_CHECK(hipMemcpyAsync(&used, order + Mb, sizeof(used), hipMemcpyDeviceToHost, s));
     XSPMM_HIP_CHECK(hipStreamSynchronize(s));
-    return used != 0;
+    const bool used = words[0] != 0;
+    words.release();
+    return used;
 }
 template bool spmm_dispatch_order_cols<int32_t>(const int32_t*, const int32_t*, int64_t, int32_t*, hipStream_t);
 template bool spmm_dispatch_order_cols<int64_t>(const int64_t*, const int64_t*, int64_t, int32_t*, hipStream_t);
