@@ -39,9 +39,11 @@
 // all pairs on the fp4 matrix cores or through the row lists.  A seed whose partners are
 // all clustered forms a cluster of one without a scan, and any other seed
 // starts its scan at its highest-positioned partner.
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "internal.hpp"
@@ -111,11 +113,28 @@ __device__ __forceinline__ void phase_sync()
     __syncthreads();
 }
 
+// Wave-wide maximum by DPP (six vector operations; the shuffle form is six LDS
+// round trips), the same value in every lane.
 __device__ __forceinline__ int wave_max(int v)
 {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    return v;
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return __builtin_amdgcn_readlane(v, 63);
+}
+// Wave-wide sum the same way (lanes a step does not reach add 0).
+__device__ __forceinline__ int wave_sum(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 __device__ __forceinline__ int64_t wave_sum64(int64_t v)
@@ -125,17 +144,18 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v)
     return v;
 }
 
-// Block-wide reductions over the 1024 threads (two barriers each).
-__device__ __forceinline__ int block_max(int v, int* red)
+// Block-wide reductions over the 1024 threads.  The maximum has one barrier:
+// consecutive calls use the two halves of red in turn (`turn`, the same in
+// every thread), and a half is written again only after the other half's
+// barrier, which every reader of it has reached.  The sums have two barriers.
+__device__ __forceinline__ int block_max(int v, int (*red)[kClWaves], int& turn)
 {
     v = wave_max(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    if ((threadIdx.x & 63) == 0) red[turn][threadIdx.x >> 6] = v;
     __syncthreads();
-    int m = red[0];
-#pragma unroll
-    for (int w = 1; w < kClWaves; ++w) m = max(m, red[w]);
-    __syncthreads();
-    return m;
+    int m = red[turn][threadIdx.x & (kClWaves - 1)];
+    turn ^= 1;
+    return wave_max(m);
 }
 
 __device__ __forceinline__ int64_t block_sum64(int64_t v, int64_t* red)
@@ -148,31 +168,6 @@ __device__ __forceinline__ int64_t block_sum64(int64_t v, int64_t* red)
     for (int w = 0; w < kClWaves; ++w) s += red[w];
     __syncthreads();
     return s;
-}
-
-// Exclusive scan over the 1024 threads; *total gets the sum (two barriers).
-__device__ __forceinline__ int64_t block_exscan64(int64_t v, int64_t* total, int64_t* red)
-{
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    int64_t incl = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int64_t t = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += t;
-    }
-    if (lane == 63) red[wave] = incl;
-    __syncthreads();
-    int64_t before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < kClWaves; ++w) {
-        const int64_t x = red[w];
-        if (w < wave) before += x;
-        all += x;
-    }
-    __syncthreads();
-    *total = all;
-    return before + incl - v;
 }
 
 // --- preparation kernels (one wave per row) ---------------------------------
@@ -792,15 +787,36 @@ struct ClusterArgs {
 
 // --- the clustering kernel ----------------------------------------------------
 
-template <typename I>
+// SMALL: every array of the loop state in LDS, as 16-bit values (the caller
+// gives small_lds(M, Kb) bytes; M and Kb at most 32767), so that a step of the
+// greedy waits for LDS instead of for L2: the loop is one chain of such waits.
+// The kernel with its state in device memory and a scan of the block's rows at
+// every step of a list took (us) 1278 for 1165 templates rows, 2592 for 6758
+// triangular rows and 3620 for a 4207-node graph; this one takes 783, 2020 and 1619.
+constexpr size_t small_lds(int64_t M, int64_t Kb)
+{
+    // un, pos, count, cnt, two candidate lists; plist; the pattern's words (read
+    // four at a time)
+    return 12 * (((size_t)M + 7) & ~size_t(7)) + 2 * (((size_t)Kb + 7) & ~size_t(7)) + 8 * (((size_t)Kb + 63) / 64 + 4);
+}
+
+// Bitmap words of a row that a thread of the scan keeps in registers.
+constexpr int kKeepWords = 16;
+
+template <typename I, bool SMALL>
 __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* __restrict__ perm)
 {
-    __shared__ uint32_t p32[kPatternWords32];  // pattern bitmap
-    __shared__ int red[kClWaves];
+    using T = std::conditional_t<SMALL, int16_t, int32_t>;
+    extern __shared__ __align__(16) unsigned char dyn[];
+    __shared__ __align__(16) uint32_t p32s[SMALL ? 1 : kPatternWords32];  // pattern bitmap
+    __shared__ int red[2][kClWaves];
+    int turn = 0;
     __shared__ int64_t red64[kClWaves];
-    __shared__ int s_cnt[4];                   // append counters: log, candidates, pattern
-    __shared__ int32_t s_blk[kClThreads];      // touch: blocks of the current chunk
-    __shared__ int64_t s_pre[kClThreads + 1];  // touch: their list offsets
+    __shared__ int s_cnt[4];                   // append counters: log, candidate lists a and b, pattern
+    __shared__ int s_pc;                       // the pattern's size after a commit
+    __shared__ int s_fp;                       // the next seed's first partner
+    __shared__ int red2[2][kClWaves];
+    __shared__ uint64_t s_q[kClWaves][kKeepWords];  // scan: the words of each wave's first grower
     __shared__ uint8_t s_flag[kClThreads];
     __shared__ int32_t s_rank[kClThreads];     // commit: visiting rank of each window position
     __shared__ int32_t s_nxt[kClThreads];      // commit: move chains over the positions past the new end
@@ -811,13 +827,60 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
     const int W = (int)a.W;  // 64-bit words per row bitmap
     const float thr = a.thresh;
     const JaccardTest jt(thr);
+    T *un, *pos, *cand_a, *cand_b, *plist;
+    const T* count;
+    uint32_t* p32;
+    const size_t mp = (((size_t)M + 7) & ~size_t(7));
+    uint32_t* const cnt2 = reinterpret_cast<uint32_t*>(dyn + 6 * mp);  // SMALL: |p & q_r|, two to a word
+    if constexpr (SMALL) {
+        un = reinterpret_cast<int16_t*>(dyn);
+        pos = un + mp;
+        T* const c = pos + mp;
+        cand_a = c + 2 * mp;
+        cand_b = cand_a + mp;
+        plist = cand_b + mp;
+        p32 = reinterpret_cast<uint32_t*>(plist + (((size_t)a.Kb + 7) & ~size_t(7)));
+        for (int i = t; i < M; i += kClThreads) c[i] = (T)a.count[i];
+        for (int i = t; i < (int)(mp / 2); i += kClThreads) cnt2[i] = 0u;
+        count = c;
+    } else {
+        un = a.un;
+        pos = a.pos;
+        cand_a = a.cand_a;
+        cand_b = a.cand_b;
+        plist = a.plist;
+        count = a.count;
+        p32 = p32s;
+    }
     uint64_t* p64 = reinterpret_cast<uint64_t*>(p32);
+    // a phase's end: in LDS a barrier, else phase_sync
+    auto sync = [&]() __attribute__((always_inline)) {
+        if constexpr (SMALL)
+            __syncthreads();
+        else
+            phase_sync();
+    };
+    // |p & q_r|: raised (returns the value before), read
+    auto cnt_add = [&](int r) __attribute__((always_inline)) -> int {
+        if constexpr (SMALL) {
+            const int sh = 16 * (r & 1);
+            return (int)((atomicAdd(&cnt2[r >> 1], 1u << sh) >> sh) & 0xffffu);
+        } else {
+            return atomicAdd(&a.cnt[r], 1);
+        }
+    };
+    auto cnt_get = [&](int r) __attribute__((always_inline)) -> int {
+        if constexpr (SMALL)
+            return (int)((cnt2[r >> 1] >> (16 * (r & 1))) & 0xffffu);
+        else
+            return __hip_atomic_load(&a.cnt[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
 
     for (int i = t; i < M; i += kClThreads) {
-        a.un[i] = i;
-        a.pos[i] = i;
+        un[i] = (T)i;
+        pos[i] = (T)i;
     }
-    for (int i = t; i < kPatternWords32; i += kClThreads) p32[i] = 0u;
+    for (int i = t; i < (SMALL ? 2 * W : kPatternWords32); i += kClThreads) p32[i] = 0u;
     if (t < 4) s_cnt[t] = 0;
 
     int engine = a.engine;
@@ -833,70 +896,73 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
         engine = 3.0 * s < 0.5 * (double)M * (double)M * (double)W ? kEngineIndex : kEngineScan;
     }
     if (t == 0) *a.engine_used = engine;
-    phase_sync();
+    sync();
 
     int n_un = M;  // every thread holds the same loop state
     int out = 0;
 
-    // Clusters of one, up to 4096 at a time.  The next seeds are un[n_un-1],
-    // un[n_un-2], ... for as long as each stays alone, and the partner lists
-    // decide that up front: the seed at position `at` is alone iff it has a
-    // list and none of its partners is unclustered below `at` (partners above
-    // `at` are the seeds before it, clustered by its turn).  The longest run
-    // of such seeds is committed at once.  Each thread takes kRunSeeds seeds
-    // per round (offsets t + 1024 u from the end) and reads their rows and
-    // partner counts before any partner list.
+    // Clusters of one.  The next seeds are un[n_un-1], un[n_un-2], ... for as
+    // long as each stays alone, and the partner lists decide that up front: the
+    // seed at position `at` is alone iff it has a list and none of its partners
+    // is unclustered below `at` (partners above `at` are the seeds before it,
+    // clustered by its turn).  The longest run of such seeds is committed at
+    // once.  A round looks at the next 64 seeds (one wave), and when all of
+    // them are alone at 4096 more at a time.  Returns the first seed not alone's
+    // highest unclustered partner position, above which nothing can join it, or
+    // -2 when its list is unknown.
     constexpr int kRunSeeds = 4;
-    constexpr int kRun = kRunSeeds * kClThreads;
-    auto singleton_runs = [&]() {
-        if (!a.pn) return;
+    auto singleton_runs = [&]() -> int {
+        if (!a.pn) return -2;
+        int look = 64;
         while (n_un > 0) {
-            int s[kRunSeeds], np[kRunSeeds];
-#pragma unroll
-            for (int u = 0; u < kRunSeeds; ++u) {
-                const int at = n_un - 1 - (t + kClThreads * u);
-                s[u] = at >= 0 ? a.un[at] : -1;
-            }
-#pragma unroll
-            for (int u = 0; u < kRunSeeds; ++u) np[u] = s[u] >= 0 ? a.pn[s[u]] : -1;
-            int first = kRun;  // this thread's first offset whose seed is not alone
+            int s[kRunSeeds], fp[kRunSeeds];
 #pragma unroll
             for (int u = 0; u < kRunSeeds; ++u) {
                 const int k = t + kClThreads * u, at = n_un - 1 - k;
-                bool alone = s[u] >= 0 && np[u] >= 0 && np[u] <= kPartnerCap;
-                for (int e = 0; alone && e < np[u]; ++e) {
-                    const int pr = a.pos[a.partners[(int64_t)s[u] * kPartnerCap + e]];
-                    if (pr >= 0 && pr < at) alone = false;
-                }
-                if (!alone && k < first) first = k;
+                s[u] = k < look && at >= 0 ? (int)un[at] : -1;
+                fp[u] = -2;
             }
-            const int run = -block_max(-first, red);  // the first seed not alone
+            int first = look;  // this thread's first offset whose seed is not alone
+#pragma unroll
+            for (int u = 0; u < kRunSeeds; ++u) {
+                const int k = t + kClThreads * u, at = n_un - 1 - k;
+                if (k >= look) continue;
+                const int np = s[u] >= 0 ? a.pn[s[u]] : -1;
+                if (np >= 0 && np <= kPartnerCap) {
+                    fp[u] = -1;
+                    // (lists are 128-byte rows: eight entries a read, past np ignored)
+                    const i32x4_t* list = reinterpret_cast<const i32x4_t*>(a.partners + (int64_t)s[u] * kPartnerCap);
+                    for (int e = 0; e < np; e += 8) {
+                        const i32x4_t l0 = list[e / 4], l1 = list[e / 4 + 1];
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const int r = j < 4 ? l0[j & 3] : l1[j & 3];
+                            if (e + j < np) {
+                                const int pr = pos[r];
+                                if (pr < at && pr > fp[u]) fp[u] = pr;
+                            }
+                        }
+                    }
+                }
+                if (fp[u] != -1 && k < first) first = k;
+            }
+            const int run = -block_max(-first, red, turn);  // the first seed not alone
 #pragma unroll
             for (int u = 0; u < kRunSeeds; ++u) {
                 const int k = t + kClThreads * u;
                 if (k < run) {
                     perm[out + k] = (I)s[u];
-                    a.pos[s[u]] = -1;
+                    pos[s[u]] = -1;
                 }
+                if (k == run && k < look) s_fp = fp[u];
             }
             out += run;
             n_un -= run;
-            phase_sync();
-            if (run < kRun) return;
+            sync();
+            if (run < look) return s_fp;
+            look = kRunSeeds * kClThreads;
         }
-    };
-
-    // Highest position of an unclustered partner of `seed` (-1: none), or
-    // -2 when the seed's partner list is unknown.  Two barriers.
-    auto first_partner = [&](int seed) -> int {
-        const int np = a.pn ? a.pn[seed] : -1;
-        if (np < 0 || np > kPartnerCap) return -2;
-        int key = -1;
-        if (t < np) {
-            const int pr = a.pos[a.partners[(int64_t)seed * kPartnerCap + t]];
-            if (pr >= 0) key = pr;
-        }
-        return block_max(key, red);
+        return -2;
     };
 
     // Commit the rows at the window positions hi - t with `flag` set, in
@@ -911,14 +977,41 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
     // so pointer jumping over k slots resolves them in log2(k) + 1 rounds.
     auto commit_flagged = [&](int hi, bool flag) {
         const int at = hi - t;
-        int64_t total;
-        const int rank = (int)block_exscan64(flag ? 1 : 0, &total, red64);  // t ascending = position descending
-        const int k = (int)total;
+        // rank: flagged threads below t (t ascending = position descending)
+        const uint64_t flagged = __builtin_amdgcn_ballot_w64(flag);
+        if ((t & 63) == 0) red[turn][t >> 6] = __popcll(flagged);
+        __syncthreads();
+        const int wn = red[turn][t & (kClWaves - 1)];
+        turn ^= 1;
+        int incl = wn;  // the wave counts up to lane % 16
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, false);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, false);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, false);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, false);
+        const int k = __builtin_amdgcn_readlane(incl, kClWaves - 1);
+        const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+        const int before = wave > 0 ? __builtin_amdgcn_readlane(incl, wave - 1) : 0;
+        const int rank = before + __popcll(flagged & ((1ull << (t & 63)) - 1ull));
+        if (k == 1) {
+            // one commit: the row at the end moves into its position
+            if (flag) {
+                const int row1 = un[at];
+                const int moved = un[n_un - 1];
+                perm[out] = (I)row1;
+                un[at] = (T)moved;
+                pos[moved] = (T)at;
+                pos[row1] = -1;
+            }
+            ++out;
+            --n_un;
+            sync();
+            return;
+        }
         if (k == 0) return;
         const int n0 = n_un, nf = n0 - k;
         int32_t row = -1;
         if (flag) {
-            row = a.un[at];
+            row = un[at];
             perm[out + rank] = (I)row;
             s_rank[t] = rank;
         }
@@ -932,7 +1025,7 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
                 const int src = n0 - 1 - s_rank[tw];  // the source of q's own commit
                 nx = src == q ? -1 : src - nf;         // src == q: q was the end itself, popped
             } else {
-                s_val[t] = a.un[q];
+                s_val[t] = un[q];
             }
             s_nxt[t] = nx;
         }
@@ -955,57 +1048,147 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
         }
         if (flag && at < nf) {
             const int32_t v = s_val[n0 - 1 - rank - nf];  // from the source of this commit
-            a.un[at] = v;
-            a.pos[v] = at;
+            un[at] = (T)v;
+            pos[v] = (T)at;
         }
-        if (flag) a.pos[row] = -1;
+        if (flag) pos[row] = -1;
         out += k;
         n_un = nf;
-        phase_sync();
+        sync();
     };
 
     if (engine == kEngineScan) {
         while (n_un > 0) {
-            singleton_runs();
+            const int fp = singleton_runs();
             if (n_un == 0) break;
-            const int seed = a.un[n_un - 1];
+            const int seed = un[n_un - 1];
             --n_un;
             if (t == 0) {
                 perm[out] = (I)seed;
-                a.pos[seed] = -1;
+                pos[seed] = -1;
             }
             ++out;
-            // positions above the first partner cannot join: start there
-            const int fp = first_partner(seed);
-            if (fp == -1) {
-                phase_sync();
-                continue;  // no unclustered partner: a cluster of one
-            }
             for (int w = t; w < W; w += kClThreads) p64[w] = a.bits[(int64_t)seed * W + w];
-            int pc = a.count[seed];
-            int hi = fp >= 0 ? fp : n_un - 1;  // highest position not yet visited
-            phase_sync();
+            int pc = count[seed];
+            // highest position not yet visited: positions above the first
+            // partner cannot join
+            int hi = fp >= 0 ? fp : n_un - 1;
+            if (W > kKeepWords) sync();
+            if (W <= kKeepWords) {
+                bool begun = false;  // the pattern is in place
+                // A window of 1024 positions keeps its rows' words and counts in
+                // registers: a commit changes no position below the committed one
+                // (the row moved into it comes from the end), so the rest of the
+                // window is tested again without a load.
+                for (; hi >= 0; hi -= kClThreads) {
+                    const int at = hi - t;
+                    int qc = 0;
+                    uint64_t x[kKeepWords];
+#pragma unroll
+                    for (int u = 0; u < kKeepWords; ++u) x[u] = 0ULL;
+                    if (at >= 0) {
+                        const int c = un[at];
+                        qc = count[c];
+                        const uint64_t* q = a.bits + (int64_t)c * W;
+#pragma unroll
+                        for (int u = 0; u < kKeepWords; ++u)
+                            if (u < W) x[u] = q[u];
+                    }
+                    if (!begun) sync();
+                    begun = true;
+                    int lim = hi + 1;  // positions below are not yet visited
+                    for (;;) {
+                        int grow = -1, inside = -1;  // this thread's position, as which kind of joiner
+                        if (at >= 0 && at < lim) {
+                            const int mn = qc < pc ? qc : pc, mx = qc < pc ? pc : qc;
+                            if (jt.may_close(mn, mx)) {  // |p&q| <= mn, |p|q| >= mx
+                                int inter = 0;
+#pragma unroll
+                                for (int u0 = 0; u0 < kKeepWords; u0 += 4)
+                                    if (u0 < W) {
+#pragma unroll
+                                        for (int u = u0; u < u0 + 4; ++u) inter += __popcll(x[u] & p64[u]);
+                                    }
+                                if (jt.close(inter, pc + qc - inter)) {
+                                    if (inter == qc)
+                                        inside = at;  // joining leaves the pattern as it is
+                                    else
+                                        grow = at;
+                                }
+                            }
+                        }
+                        const int wg = wave_max(grow), wi = wave_max(inside);
+                        if (grow >= 0 && grow == wg) {
+#pragma unroll
+                            for (int u = 0; u < kKeepWords; ++u)
+                                if (u < W) s_q[t >> 6][u] = x[u];
+                        }
+                        if ((t & 63) == 0) {
+                            red[turn][t >> 6] = wg;
+                            red2[turn][t >> 6] = wi;
+                        }
+                        __syncthreads();
+                        const int mg = red[turn][t & (kClWaves - 1)], mi = red2[turn][t & (kClWaves - 1)];
+                        turn ^= 1;
+                        const int best = wave_max(mg);  // the first joiner that grows the pattern
+                        // joiners inside the pattern, down to best, met it as it is
+                        if (wave_max(mi) > best) commit_flagged(hi, inside > best);
+                        if (best < 0) break;
+                        if (t < 64) {
+                            const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mg == best));
+                            int add = 0;
+                            if (t < W) {
+                                const uint64_t q = s_q[from][t], o = p64[t];
+                                add = __popcll(q & ~o);
+                                p64[t] = o | q;
+                            }
+                            add = wave_sum(add);
+                            if (t == 0) {
+                                s_pc = pc + add;
+                                const int c = un[best];
+                                perm[out] = (I)c;
+                                const int moved = un[n_un - 1];
+                                un[best] = (T)moved;
+                                pos[moved] = (T)best;
+                                pos[c] = -1;
+                            }
+                        }
+                        ++out;
+                        --n_un;
+                        lim = best;
+                        sync();
+                        pc = s_pc;
+                    }
+                }
+                __syncthreads();
+                continue;
+            }
             while (hi >= 0) {
                 const int at = hi - t;
                 // joiners: 2 at + 1 when q lies inside the pattern (joining
                 // leaves it unchanged), 2 at when q grows it
                 int key = -1;
                 if (at >= 0) {
-                    const int c = a.un[at];
-                    const int qc = a.count[c];
+                    const int c = un[at];
+                    const int qc = count[c];
                     const int mn = qc < pc ? qc : pc, mx = qc < pc ? pc : qc;
                     if (jt.may_close(mn, mx)) {  // |p&q| <= mn, |p|q| >= mx
                         const uint64_t* q = a.bits + (int64_t)c * W;
-                        int inter = 0, uni = 0;
-                        for (int w = 0; w < W; ++w) {
-                            const uint64_t x = q[w], y = p64[w];
-                            inter += __popcll(x & y);
-                            uni += __popcll(x | y);
+                        // |p | q| = |p| + |q| - |p & q|; eight words' loads at a time
+                        int inter = 0;
+                        for (int w0 = 0; w0 < W; w0 += 8) {
+                            uint64_t x[8];
+#pragma unroll
+                            for (int u = 0; u < 8; ++u) x[u] = w0 + u < W ? q[w0 + u] : 0ULL;
+#pragma unroll
+                            for (int u = 0; u < 8; ++u)
+                                if (w0 + u < W) inter += __popcll(x[u] & p64[w0 + u]);
                         }
+                        const int uni = pc + qc - inter;
                         if (jt.close(inter, uni)) key = 2 * at + (inter == qc ? 1 : 0);
                     }
                 }
-                const int top = block_max(key, red);
+                const int top = block_max(key, red, turn);
                 int best = top < 0 ? -1 : top >> 1;  // the first joiner in visiting order
                 if (top >= 0 && (top & 1)) {
                     // Joiners inside the pattern leave it as it is, so every joiner
@@ -1014,32 +1197,56 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
                     // commits those inside it in visiting order, with the
                     // reference's swap-removes (a row from above moves into each
                     // freed position), and best, if any, is committed below.
-                    best = block_max((key >= 0 && !(key & 1)) ? key >> 1 : -1, red);
+                    best = block_max((key >= 0 && !(key & 1)) ? key >> 1 : -1, red, turn);
                     commit_flagged(hi, key >= 0 && (key & 1) && (key >> 1) > best);
                 }
                 if (best < 0) {
                     hi -= kClThreads;
                     continue;
                 }
-                const int c = a.un[best];
-                int64_t add = 0;
-                for (int w = t; w < W; w += kClThreads) {
-                    const uint64_t q = a.bits[(int64_t)c * W + w], o = p64[w];
-                    add += __popcll(q & ~o);
-                    p64[w] = o | q;
-                }
-                pc += (int)block_sum64(add, red64);
-                if (t == 0) {
-                    perm[out] = (I)c;
-                    const int moved = a.un[n_un - 1];
-                    a.un[best] = moved;
-                    a.pos[moved] = best;
-                    a.pos[c] = -1;
+                if (W <= 64) {
+                    // the pattern's words, and so the commit, belong to one wave
+                    if (t < 64) {
+                        const int c = un[best];
+                        int add = 0;
+                        if (t < W) {
+                            const uint64_t q = a.bits[(int64_t)c * W + t], o = p64[t];
+                            add = __popcll(q & ~o);
+                            p64[t] = o | q;
+                        }
+                        add = wave_sum(add);
+                        if (t == 0) {
+                            s_pc = pc + add;
+                            perm[out] = (I)c;
+                            const int moved = un[n_un - 1];
+                            un[best] = (T)moved;
+                            pos[moved] = (T)best;
+                            pos[c] = -1;
+                        }
+                    }
+                } else {
+                    const int c = un[best];
+                    int64_t add = 0;
+                    for (int w = t; w < W; w += kClThreads) {
+                        const uint64_t q = a.bits[(int64_t)c * W + w], o = p64[w];
+                        add += __popcll(q & ~o);
+                        p64[w] = o | q;
+                    }
+                    add = block_sum64(add, red64);
+                    if (t == 0) {
+                        s_pc = pc + (int)add;
+                        perm[out] = (I)c;
+                        const int moved = un[n_un - 1];
+                        un[best] = (T)moved;
+                        pos[moved] = (T)best;
+                        pos[c] = -1;
+                    }
                 }
                 ++out;
                 --n_un;
                 hi = best - 1;
-                phase_sync();
+                sync();
+                pc = s_pc;
             }
             __syncthreads();
         }
@@ -1048,65 +1255,50 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
 
     // ---- index engine (0 <= dist_thresh < 1) ----
     // Raise cnt of the not-yet-visited rows of the lists of plist[b0, b1);
-    // rows whose cnt leaves zero are logged and appended to `cand`.
-    auto touch = [&](int b0, int b1, int limit, int32_t* cand) {
-        for (int c0 = b0; c0 < b1; c0 += kClThreads) {
-            const int nb = b1 - c0 < kClThreads ? b1 - c0 : kClThreads;
-            int64_t len = 0;
-            if (t < nb) {
-                const int32_t b = a.plist[c0 + t];
-                s_blk[t] = b;
-                len = a.bl_start[b + 1] - a.bl_start[b];
-            }
-            int64_t total;
-            const int64_t ex = block_exscan64(len, &total, red64);
-            if (t < nb) s_pre[t] = ex;
-            if (t == 0) s_pre[nb] = total;
-            __syncthreads();
-            for (int64_t e = t; e < total; e += kClThreads) {
-                int lo = 0, hi = nb - 1;  // last j with s_pre[j] <= e
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (s_pre[mid] <= e) lo = mid;
-                    else hi = mid - 1;
-                }
-                const int32_t r = a.bl_rows[a.bl_start[s_blk[lo]] + (e - s_pre[lo])];
-                const int pr = a.pos[r];
+    // rows whose cnt leaves zero are appended to `cand` (and logged).  One wave
+    // walks a list; below sixteen lists, several waves share each.
+    auto touch = [&](int b0, int b1, int limit, T* cand, int* ncand) {
+        const int nb = b1 - b0;
+        int share = 1;
+        while (share * nb < kClWaves && share < kClWaves) share *= 2;
+        const int lane = t & 63, wave = t >> 6;
+        for (int c = wave / share; c < nb; c += kClWaves / share) {
+            const int b = plist[b0 + c];
+            const int64_t e1 = a.bl_start[b + 1];
+            for (int64_t e = a.bl_start[b] + 64 * (wave % share) + lane; e < e1; e += 64 * share) {
+                const int r = a.bl_rows[e];
+                const int pr = pos[r];
                 if (pr < 0 || pr >= limit) continue;  // clustered or already visited
-                if (atomicAdd(&a.cnt[r], 1) == 0) {
-                    a.log[atomicAdd(&s_cnt[0], 1)] = r;
-                    cand[atomicAdd(&s_cnt[1], 1)] = r;
+                if (cnt_add(r) == 0) {
+                    if constexpr (!SMALL) a.log[atomicAdd(&s_cnt[0], 1)] = r;
+                    cand[atomicAdd(ncand, 1)] = (T)r;
                 }
             }
-            __syncthreads();
         }
     };
 
     while (n_un > 0) {
-        singleton_runs();
+        const int fp = singleton_runs();
         if (n_un == 0) break;
-        const int seed = a.un[n_un - 1];
+        const int seed = un[n_un - 1];
         --n_un;
         if (t == 0) {
             perm[out] = (I)seed;
-            a.pos[seed] = -1;
+            pos[seed] = -1;
         }
         ++out;
-        phase_sync();
+        sync();
 
-        if (a.count[seed] == 0) {
+        if (count[seed] == 0) {
             // Empty pattern: the remaining empty rows join, in descending
             // position order, and the pattern stays empty.  A swap-remove at
             // position i moves in a row from above i, already visited.
             for (int hi = n_un - 1; hi >= 0; hi -= kClThreads) {
                 const int at = hi - t;
-                commit_flagged(hi, at >= 0 && a.count[a.un[at]] == 0);
+                commit_flagged(hi, at >= 0 && count[un[at]] == 0);
             }
             continue;
         }
-
-        const int fp = first_partner(seed);
-        if (fp == -1) continue;  // no unclustered partner: a cluster of one
 
         // pattern := blocks of the seed
         {
@@ -1114,81 +1306,107 @@ __global__ __launch_bounds__(kClThreads) void cluster_kernel(ClusterArgs a, I* _
             const int n = (int)(a.rb_start[seed + 1] - rs);
             for (int k = t; k < n; k += kClThreads) {
                 const int32_t b = a.rb[rs + k];
-                a.plist[k] = b;
+                plist[k] = (T)b;
                 atomicOr(&p32[b >> 5], 1u << (b & 31));
             }
         }
-        int pc = a.count[seed];
+        int pc = count[seed];
         // positions below limit are not yet visited; those above the first
         // partner cannot join and are skipped
         int limit = fp >= 0 ? fp + 1 : n_un;
-        int32_t* cur = a.cand_a;
-        int32_t* nxt = a.cand_b;
-        phase_sync();
-        touch(0, pc, limit, cur);
-        phase_sync();
+        T* cur = cand_a;
+        T* nxt = cand_b;
+        int x = 1;  // s_cnt[x] counts cur, s_cnt[3 - x] counts nxt
+        sync();
+        touch(0, pc, limit, cur, &s_cnt[x]);
+        sync();
 
         for (;;) {
-            const int ncand = s_cnt[1];
-            __syncthreads();
-            if (t == 0) s_cnt[1] = 0;
-            __syncthreads();
+            const int ncand = s_cnt[x];
             // test the candidates, keeping those still below the limit
             int key = -1;
             for (int k = t; k < ncand; k += kClThreads) {
-                const int32_t r = cur[k];
-                const int pr = a.pos[r];
+                const int r = cur[k];
+                const int pr = pos[r];
                 if (pr < 0 || pr >= limit) continue;
-                nxt[atomicAdd(&s_cnt[1], 1)] = r;
-                const int inter = __hip_atomic_load(&a.cnt[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const int uni = pc + a.count[r] - inter;
+                nxt[atomicAdd(&s_cnt[3 - x], 1)] = (T)r;
+                const int inter = cnt_get(r);
+                const int uni = pc + count[r] - inter;
                 if (pr > key && jt.close(inter, uni)) key = pr;
             }
-            const int best = block_max(key, red);
-            int32_t* sw = cur;
+            const int best = block_max(key, red, turn);
+            T* sw = cur;
             cur = nxt;
             nxt = sw;
+            // the tested list is empty again (every thread has read its length)
+            if (t == 0) s_cnt[x] = 0;
+            x = 3 - x;
             if (best < 0) break;
-            const int r = a.un[best];
+            const int r = un[best];
+            if (t == 0) s_cnt[3] = pc;
+            sync();  // every thread has the row before the commit moves another there
             if (t == 0) {
                 perm[out] = (I)r;
-                const int moved = a.un[n_un - 1];
-                a.un[best] = moved;
-                a.pos[moved] = best;
-                a.pos[r] = -1;
+                const int moved = un[n_un - 1];
+                un[best] = (T)moved;
+                pos[moved] = (T)best;
+                pos[r] = -1;
             }
             ++out;
             --n_un;
             limit = best;
-            if (t == 0) s_cnt[2] = pc;
-            phase_sync();
             // blocks of r not yet in the pattern
             const int64_t rs = a.rb_start[r];
             const int n = (int)(a.rb_start[r + 1] - rs);
             for (int k = t; k < n; k += kClThreads) {
                 const int32_t b = a.rb[rs + k];
                 const uint32_t bit = 1u << (b & 31);
-                if ((atomicOr(&p32[b >> 5], bit) & bit) == 0u) a.plist[atomicAdd(&s_cnt[2], 1)] = b;
+                if ((atomicOr(&p32[b >> 5], bit) & bit) == 0u) plist[atomicAdd(&s_cnt[3], 1)] = (T)b;
             }
-            phase_sync();
-            const int pc_new = s_cnt[2];
-            touch(pc, pc_new, limit, cur);  // new candidates join the compacted list
+            sync();
+            const int pc_new = s_cnt[3];
+            touch(pc, pc_new, limit, cur, &s_cnt[x]);  // new candidates join the compacted list
             pc = pc_new;
-            phase_sync();
+            sync();
         }
 
         // reset the counters and the pattern
-        const int nlog = s_cnt[0];
-        for (int k = t; k < nlog; k += kClThreads)
-            __hip_atomic_store(&a.cnt[a.log[k]], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (SMALL) {
+            for (int i = t; i < (int)(mp / 2); i += kClThreads) cnt2[i] = 0u;
+        } else {
+            const int nlog = s_cnt[0];
+            for (int k = t; k < nlog; k += kClThreads)
+                __hip_atomic_store(&a.cnt[a.log[k]], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         for (int k = t; k < pc; k += kClThreads) {
-            const int32_t b = a.plist[k];
+            const int32_t b = plist[k];
             p32[b >> 5] = 0u;
         }
-        phase_sync();
+        sync();
         if (t < 4) s_cnt[t] = 0;
         __syncthreads();
     }
+}
+
+}  // namespace
+
+namespace {
+
+// LDS left to the loop state of a SMALL workgroup: 160 KB less its fixed arrays
+// (16 KB) and a margin.
+constexpr size_t kSmallLds = 142 * 1024;
+
+// Dynamic LDS above 64 KB has to be asked for, once per device and kernel.
+template <typename I>
+void allow_small_lds()
+{
+    static std::atomic<bool> done[64];
+    int dev = 0;
+    XSPMM_HIP_CHECK(hipGetDevice(&dev));
+    if (dev >= 0 && dev < 64 && done[dev].load(std::memory_order_relaxed)) return;
+    XSPMM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&cluster_kernel<I, true>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+    if (dev >= 0 && dev < 64) done[dev].store(true, std::memory_order_relaxed);
 }
 
 }  // namespace
@@ -1395,7 +1613,12 @@ void jaccard_clustering_device(int64_t M, int64_t K, int64_t nnz, const I* rp, c
     ClusterArgs args{M, W, Kb, dist_thresh, engine, bits, count, rb_start, rb, bl_start, bl_rows,
                      at(o_un), at(o_pos), at(o_cnt), at(o_logb), at(o_ca), at(o_cb), at(o_plist),
                      use_partners ? pn : nullptr, partners, bad + 1};
-    hipLaunchKernelGGL(cluster_kernel<I>, dim3(1), dim3(kClThreads), 0, s, args, perm);
+    if (M <= 32767 && Kb <= 32767 && small_lds(M, Kb) <= kSmallLds) {
+        allow_small_lds<I>();
+        hipLaunchKernelGGL((cluster_kernel<I, true>), dim3(1), dim3(kClThreads), small_lds(M, Kb), s, args, perm);
+    } else {
+        hipLaunchKernelGGL((cluster_kernel<I, false>), dim3(1), dim3(kClThreads), 0, s, args, perm);
+    }
     XSPMM_LAUNCH_CHECK();
     if (engine_used) {
         HostWords used;
