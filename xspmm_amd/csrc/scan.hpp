@@ -116,8 +116,9 @@ __global__ __launch_bounds__(kScanThreads) void scan_final_kernel(F f, int64_t n
 // round of memory latency however the functor chains its loads), four
 // consecutive ones per thread and tile of 4096; the tiles' wave sums are scanned
 // together, so the kernel has two barriers.  Bound by latency: 16384 row lengths
-// through a permutation 8 us, where the three kernels above took 14 and the host
-// 25 more for their launches and the allocation of the tile sums.
+// through a permutation 19 us in one workgroup, where the three kernels above
+// took 14 but another two launches (7 us each between kernels) and an allocation
+// for the tile sums (15 us on the host).
 constexpr int kScanOneThreads = 1024;
 constexpr int kScanOneTile = 4 * kScanOneThreads;
 constexpr int kScanOneTiles = 8;
