@@ -171,3 +171,33 @@ def test_plan_and_pipeline_odd_n(torch, dtype, cluster):
         b = torch.as_tensor(B).cuda()
         assert np.array_equal(plan.execute(b).cpu().numpy(), want)
         assert np.array_equal(X.spmm_pipeline(A, b, optimize_pattern=cluster)[0].cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("where", [None, "A", "B"])
+@pytest.mark.parametrize("cluster", [False, True])
+@pytest.mark.parametrize("itype", [np.int32, np.int64])
+def test_packed_plan_on_padded_b(torch, itype, cluster, where):
+    """fp16 plans of sparse blocks ("deep": 73521 of them) multiply their packed
+    batches on the padded copy from N = 257; an Inf or NaN takes whole blocks."""
+    M, K = 4099, 5003
+    rp, ci, vals = integer_csr("deep", M, K, np.float16, itype, seed=11)
+    if where == "A":
+        vals[len(vals) // 2] = np.inf
+    A = X.CSRMatrix.from_host(M, K, rp, ci, vals, device="cuda:0")
+    plan = X.SpMMPlan(A, optimize_pattern=cluster)
+    assert plan.packed_batches > 0
+    # the rows' order decides which blocks cover which rows
+    perm = X.jaccard_clustering(A) if cluster else torch.arange(M, dtype=A.row_ptr.dtype, device="cuda:0")
+    blocks = X.csr_to_bcsr(X.apply_permutation(A, perm))
+    rows = perm.cpu().numpy()
+    for N in (129, 257, 260, 391):
+        print(itype.__name__, cluster, where, N, flush=True)
+        B = np.random.default_rng(N).integers(1, 9, size=(K, N)).astype(np.float16)
+        if where == "B":
+            B[K // 2, N // 2] = np.nan if N == 260 else -np.inf
+        want = np.empty((M, N))
+        want[rows] = product(blocks, B)
+        guard = torch.full((M * N + 64,), -7.0, device="cuda:0")
+        C = plan.execute(torch.as_tensor(B).cuda(), guard[:M * N].view(M, N))
+        assert np.array_equal(C.cpu().numpy(), want, equal_nan=True)
+        assert bool((guard[M * N:] == -7.0).all())

@@ -268,6 +268,29 @@ void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
                     const T* bvals, const T* B, float* C, int64_t N, const int32_t* order, bool band, void* scratch,
                     size_t scratch_bytes, hipStream_t s);
 size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N);
+// B with rows of Np columns (N rounded up to 16 bytes; B itself when its rows
+// start there already) and its marks (256 bytes, one set where a part of B holds
+// an Inf or NaN), made on the stream by pad_b_kernel, and room for order_rows
+// int32, all one piece of the arena (an allocation costs the host about 15 us);
+// bt null when a fixed arena has no room for it.  T: uint16_t (fp16) or float.
+template <typename T>
+struct PaddedB {
+    const T* bt = nullptr;
+    const uint32_t* marks = nullptr;
+    int32_t* order = nullptr;
+    int64_t Np = 0;
+};
+template <typename T>
+PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena& arena, hipStream_t s);
+// A product's blocks whole, on padded B, where one of its marks is set; else
+// nothing (rows_exact_kernel): follows a packed product given the same marks.
+template <typename I>
+void bcsr_rows_exact(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci, const uint16_t* bvals,
+                     const uint16_t* B, float* C, int64_t N, int64_t nc, const I* row_map, const uint32_t* nonfinite,
+                     hipStream_t s);
+// Whether none of n fp16 values is an Inf or NaN (false as well when n is not a
+// multiple of 8, or beyond 2^30; synchronizes s).
+bool all_finite_f16(const void* values, int64_t n, hipStream_t s);
 // Tier-1 without any allocation: the temporaries come from a fixed device
 // array of kNoAllocScratchBytes (one copy per GPU, shared by every call on
 // it).  Throws std::invalid_argument when a product needs more.
@@ -320,7 +343,8 @@ void spmm_f16_pack_fill(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* b
 template <typename I>
 bool spmm_f16_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, const void* a,
                      const uint32_t* rows, const uint16_t* B, float* C, int64_t N,
-                     const int32_t* order, const I* row_map, hipStream_t s);
+                     const int32_t* order, const I* row_map, hipStream_t s,
+                     int64_t nc = 0, const uint32_t* nonfinite = nullptr);
 
 // Tier-1 fp32 column-batch SpMM (spmm_f32.hip): covers N % 4 == 0 with B and
 // C 16-byte aligned, K * N * 4 <= 2^31 and Kb < 2^21; order and row_map as for bcsr_spmm_ex.  With nc > 0, B is a

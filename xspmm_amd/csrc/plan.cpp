@@ -13,14 +13,16 @@
 //     bytes: fp16, the batch kernel's batches (spmm_f16_packed); fp32, the
 //     pipeline's packed fp32 batches formed from the permuted CSR
 //     (csr_pack_analyse / csr_pack_emit, spmm_f32_packed); both with the
-//     fused store;
+//     fused store; fp16, N % 8 != 0: on a padded copy of B where
+//     packed_pad_wanted says so;
 //   * a fully populated block grid takes the GEMM-tiled kernel, as in the
 //     pipeline, with the same fused store;
 //   * otherwise (fp32, other N) the product goes to a workspace kept by the
 //     plan (it only grows) and is un-permuted into C.
 // C equals the pipeline's C bit for bit: the same kernels accumulate in the
 // same order, only the row a result is stored to differs.  execute() does not
-// allocate once the workspace is large enough (never, on the fused path).
+// allocate once the workspace is large enough (never, on the fused path), but
+// for the padded copies of B, which are stream-ordered allocations.
 // Calls on one plan must not overlap (they share the workspace).
 #include <cstdlib>
 #include <cstring>
@@ -33,6 +35,18 @@ namespace xspmm {
 namespace detail {
 
 namespace {
+
+// Whether an fp16 product with N % 8 != 0 takes the packed batches, on a padded
+// copy of B: three launches and an allocation (25 us of host time: B's copy, the
+// batches, rows_exact_kernel for an Inf or NaN in B) against the BCSR kernels on
+// the same copy (from 23 us).  From 3 * 2^16 products of a block with 128 columns
+// (us, BCSR / packed: 47343 blocks, N = 257 27 / 28; 100926 blocks, N = 127 27 /
+// 27, N = 257 55 / 32; 553925 blocks, N = 3 100 / 29, N = 127 146 / 64; 756731
+// blocks, N = 127 91 / 39, N = 257 263 / 101).  C is the same bit for bit.
+bool packed_pad_wanted(int64_t nnzb, int64_t N)
+{
+    return nnzb * ((N + 127) / 128) >= 3 * (int64_t(1) << 16);
+}
 
 // Device memory owned for the plan's lifetime (not stream-ordered: a plan
 // outlives the streams it is used on).
@@ -156,6 +170,10 @@ public:
         poff_ = std::move(offsets);
         nbatches_ = nb;
         packed_ = true;
+        // an Inf or NaN of A' stands for a whole row's slots: padded products
+        // of such a matrix keep the BCSR kernels, which give the reference's.
+        // (Matrices that no N up to 1024 brings to the line skip the check.)
+        pads_ = packed_pad_wanted(nnzb_, 1024) && all_finite_f16(pa_.as<void>(), nb * 512, s);
     }
 
     // Packed fp32 column batches from the (permuted) CSR, as the pipeline
@@ -207,6 +225,9 @@ public:
                                               reinterpret_cast<const uint16_t*>(B), C, N, order,
                                               clustered_ ? perm_.as<I>() : nullptr, s))
                 return;
+            if (pads_ && packed_pad_wanted(nnzb_, N) &&
+                execute_padded(reinterpret_cast<const uint16_t*>(B), C, N, order, s))
+                return;
         } else {
             if (packed_ && spmm_f32_packed<I>(M_, K_, Mb_, poff_.as<int64_t>(), pa_.as<void>(),
                                               prow_.as<uint32_t>(), reinterpret_cast<const float*>(B), C,
@@ -231,6 +252,26 @@ public:
         unpermute_dense<I>(ws_.as<float>(), C, perm_.as<I>(), M_, N, s);
     }
 
+    // fp16, N % 8 != 0: the packed product on a padded copy of B.  Where B holds an
+    // Inf or NaN, which only the whole blocks carry to every row it reaches, the
+    // second kernel makes the product.  The copy is a stream-ordered allocation,
+    // as in the BCSR form.
+    bool execute_padded(const uint16_t* B, float* C, int64_t N, const int32_t* order, hipStream_t s)
+    {
+        const int64_t Np = (N + 7) / 8 * 8;
+        if (Np >= (int64_t(1) << 22) || K_ * Np * 2 > (int64_t(1) << 31)) return false;
+        if ((reinterpret_cast<uintptr_t>(B) & 15) != 0) return false;  // refused by the BCSR form
+        const I* rmap = clustered_ ? perm_.as<I>() : nullptr;
+        TempArena arena(s);
+        const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K_, N, 0, arena, s);
+        if (!spmm_f16_packed<I>(M_, K_, Mb_, poff_.as<int64_t>(), pa_.as<void>(), prow_.as<uint32_t>(), pb.bt, C,
+                                pb.Np, order, rmap, s, N, pb.marks))
+            return false;
+        bcsr_rows_exact<I>(M_, K_, Mb_, Kb_, brp_.as<I>(), bci_.as<I>(), bvals_.as<uint16_t>(), pb.bt, C, pb.Np, N,
+                           rmap, pb.marks, s);
+        return true;
+    }
+
     int64_t num_blocks() const override { return nnzb_; }
     int64_t num_packed_batches() const override { return packed_ ? nbatches_ : -1; }
     int64_t num_block_rows() const override { return Mb_; }
@@ -240,6 +281,7 @@ public:
 private:
     int64_t M_ = 0, K_ = 0, Mb_ = 0, Kb_ = 0, nnzb_ = 0, nbatches_ = 0;
     bool clustered_ = false, packed_ = false;
+    bool pads_ = false;  // packed, and taken for padded copies of B too
     DeviceBuffer perm_, brp_, bci_, bvals_, order_, ws_;
     DeviceBuffer poff_, pa_, prow_;  // packed column batches
 };

@@ -1243,18 +1243,23 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
 // same order, so C equals the batch kernel's C.  While a batch multiplies,
 // the next batch's B rows are in flight and the indices of the one after
 // are loading.  LDS holds only the B tile of each wave (8 KB).  grid = (block-rows, ceil(N / 128)); N % 8 == 0, K * N * 2 <= 2^31.
+// C has nc <= N columns (B padded to N).  Where nonfinite is given and a mark is
+// set, nothing is stored: rows_exact_kernel makes that product.
 // ---------------------------------------------------------------------------
 template <typename I, int NT>
 __global__ __launch_bounds__(64 * kBW, XSPMM_BATCH_MIN_WAVES) void spmm_f16_packed_kernel(
     const int64_t* __restrict__ offsets, const u32x4_t* __restrict__ pa,
     const uint32_t* __restrict__ prow, const uint16_t* __restrict__ B, float* __restrict__ C,
-    int64_t M, int64_t K, int64_t N, const int32_t* __restrict__ order, const I* __restrict__ row_map)
+    int64_t M, int64_t K, int64_t N, const int32_t* __restrict__ order, const I* __restrict__ row_map, int64_t nc,
+    const uint32_t* __restrict__ nonfinite)
 {
     static_assert(NT == 1 || NT == 2 || NT == 4 || NT == 8, "NT must be a power of two <= 8");
     constexpr int CPR = 2 * NT;    // 16-byte chunks per B row
     constexpr int RPL = 64 / CPR;  // B rows per load instruction
     __shared__ __align__(16) unsigned char smem[kBW * kBtBytes];
     const int lane = threadIdx.x & (kWave - 1);
+    // every wave sees the same marks: the whole workgroup leaves
+    if (nonfinite && __builtin_amdgcn_ballot_w64(nonfinite[lane] != 0u) != 0) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     unsigned char* const W = smem + wave * kBtBytes;
     const int64_t br = order ? (int64_t)order[blockIdx.x] : (int64_t)blockIdx.x;
@@ -1339,7 +1344,28 @@ __global__ __launch_bounds__(64 * kBW, XSPMM_BATCH_MIN_WAVES) void spmm_f16_pack
             a_cur = pa_w[(more ? bi + 1 : bi) * 64];
         }
     }
-    batch_tile_store<I, NT>(acc, smem, wave, g, li, br, n0, M, N, C, row_map);
+    batch_tile_store<I, NT>(acc, smem, wave, g, li, br, n0, M, nc, C, row_map);
+}
+
+// A packed product's other half: where a mark is set (pad_b_kernel's), every
+// block of the BCSR form whole, so that a non-finite value reaches what it
+// reaches in the reference; else nothing.  A packed product has no blocks to
+// multiply and its caller does not wait for the marks, so both kernels are
+// launched.  Workgroups walk the (block-row, 128 columns) pairs: an unmarked
+// call pays for 256 of them (2 us).
+constexpr int kExactGroups = 256;
+template <typename I>
+__global__ __launch_bounds__(64 * kBW) void rows_exact_kernel(
+    const I* __restrict__ brp, const I* __restrict__ bci, const uint16_t* __restrict__ vals,
+    const uint16_t* __restrict__ B,
+    float* __restrict__ C, int64_t M, int64_t K, int64_t N, int64_t nc, int64_t Mb, int64_t Kb,
+    const I* __restrict__ row_map, const uint32_t* __restrict__ nonfinite)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    if (__builtin_amdgcn_ballot_w64(nonfinite[lane] != 0u) == 0) return;
+    const int64_t pairs = Mb * ((nc + 127) / 128);
+    for (int64_t p = blockIdx.x; p < pairs; p += gridDim.x)
+        batch_row_exact<I, 8>(brp, bci, vals, B, C, M, K, N, nc, Kb, p % Mb, p / Mb * 128, row_map);
 }
 
 // ---------------------------------------------------------------------------
@@ -1869,9 +1895,10 @@ void spmm_f16_pack_fill(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* b
 template <typename I>
 bool spmm_f16_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, const void* a,
                      const uint32_t* rows, const uint16_t* B, float* C, int64_t N,
-                     const int32_t* order, const I* row_map, hipStream_t s)
+                     const int32_t* order, const I* row_map, hipStream_t s, int64_t nc, const uint32_t* nonfinite)
 {
     if (M == 0 || N == 0 || Mb == 0) return true;
+    if (nc <= 0) nc = N;
     check_alignment(a, B, true);
     if (N % 8 != 0 || K * N * 2 > (int64_t(1) << 31) || N >= (int64_t(1) << 22)) return false;
     const int64_t chunks = (N + 127) / 128;
@@ -1880,17 +1907,52 @@ bool spmm_f16_packed(int64_t M, int64_t K, int64_t Mb, const int64_t* offsets, c
     const u32x4_t* pa = static_cast<const u32x4_t*>(a);
     if (N <= 16)
         hipLaunchKernelGGL((spmm_f16_packed_kernel<I, 1>), grid, dim3(64 * kBW), 0, s, offsets, pa, rows,
-                           B, C, M, K, N, order, row_map);
+                           B, C, M, K, N, order, row_map, nc, nonfinite);
     else if (N <= 32)
         hipLaunchKernelGGL((spmm_f16_packed_kernel<I, 2>), grid, dim3(64 * kBW), 0, s, offsets, pa, rows,
-                           B, C, M, K, N, order, row_map);
+                           B, C, M, K, N, order, row_map, nc, nonfinite);
     else if (N <= 64)
         hipLaunchKernelGGL((spmm_f16_packed_kernel<I, 4>), grid, dim3(64 * kBW), 0, s, offsets, pa, rows,
-                           B, C, M, K, N, order, row_map);
+                           B, C, M, K, N, order, row_map, nc, nonfinite);
     else
         hipLaunchKernelGGL((spmm_f16_packed_kernel<I, 8>), grid, dim3(64 * kBW), 0, s, offsets, pa, rows,
-                           B, C, M, K, N, order, row_map);
+                           B, C, M, K, N, order, row_map, nc, nonfinite);
     XSPMM_LAUNCH_CHECK();
+    return true;
+}
+
+template <typename I>
+void bcsr_rows_exact(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci, const uint16_t* bvals,
+                     const uint16_t* B, float* C, int64_t N, int64_t nc, const I* row_map, const uint32_t* nonfinite,
+                     hipStream_t s)
+{
+    hipLaunchKernelGGL((rows_exact_kernel<I>), dim3(kExactGroups), dim3(64 * kBW), 0, s, brp, bci, bvals, B, C, M, K,
+                       N, nc, Mb, Kb, row_map, nonfinite);
+    XSPMM_LAUNCH_CHECK();
+}
+#define XSPMM_ROWS_EXACT(I)                                                                             \
+    template void bcsr_rows_exact<I>(int64_t, int64_t, int64_t, int64_t, const I*, const I*,             \
+                                     const uint16_t*, const uint16_t*, float*, int64_t, int64_t, const I*, \
+                                     const uint32_t*, hipStream_t);
+XSPMM_ROWS_EXACT(int32_t)
+XSPMM_ROWS_EXACT(int64_t)
+#undef XSPMM_ROWS_EXACT
+
+bool all_finite_f16(const void* values, int64_t n, hipStream_t s)
+{
+    // pad_b_kernel's pass without the copy: rows of 8 halves
+    const int64_t vecs = n / 8;
+    if (n % 8 != 0 || vecs > (int64_t(1) << 27)) return false;
+    Scratch marks(kPadMarks, s);
+    hipLaunchKernelGGL((pad_b_kernel<uint16_t, false>), dim3(kPadMarks), dim3(kPadThreads), 0, s,
+                       static_cast<const uint16_t*>(values), static_cast<uint16_t*>(nullptr), vecs, (int64_t)8,
+                       (int64_t)8, marks.as<unsigned char>());
+    XSPMM_LAUNCH_CHECK();
+    uint32_t host[kPadMarks / 4];
+    XSPMM_HIP_CHECK(hipMemcpyAsync(host, marks.get(), kPadMarks, hipMemcpyDeviceToHost, s));
+    XSPMM_HIP_CHECK(hipStreamSynchronize(s));
+    for (uint32_t m : host)
+        if (m != 0u) return false;
     return true;
 }
 
@@ -1911,7 +1973,7 @@ int64_t spmm_f16_pack_offsets(const int32_t* counts, int64_t n, int64_t* offsets
                                         hipStream_t);                                              \
     template bool spmm_f16_packed<I>(int64_t, int64_t, int64_t, const int64_t*, const void*,       \
                                      const uint32_t*, const uint16_t*, float*, int64_t,            \
-                                     const int32_t*, const I*, hipStream_t);
+                                     const int32_t*, const I*, hipStream_t, int64_t, const uint32_t*);
 XSPMM_PACK(int32_t)
 XSPMM_PACK(int64_t)
 #undef XSPMM_PACK
@@ -1944,20 +2006,6 @@ bool spmm_dispatch_order_cols(const I* brp, const I* bci, int64_t Mb, int32_t* o
 template bool spmm_dispatch_order_cols<int32_t>(const int32_t*, const int32_t*, int64_t, int32_t*, hipStream_t);
 template bool spmm_dispatch_order_cols<int64_t>(const int64_t*, const int64_t*, int64_t, int32_t*, hipStream_t);
 
-namespace {
-
-// B with rows of Np columns (N rounded up to 16 bytes; B itself when its rows
-// start there already) and its marks, made on the stream by pad_b_kernel, and
-// room for order_rows int32, all one piece of the arena (an allocation costs
-// the host about 15 us); bt null when a fixed arena has no room for it.
-template <typename T>
-struct PaddedB {
-    const T* bt = nullptr;
-    const uint32_t* marks = nullptr;
-    int32_t* order = nullptr;
-    int64_t Np = 0;
-};
-
 template <typename T>
 PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena& arena, hipStream_t s)
 {
@@ -1987,6 +2035,10 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     p.order = reinterpret_cast<int32_t*>(base + o_order);
     return p;
 }
+template PaddedB<uint16_t> pad_b<uint16_t>(const uint16_t*, int64_t, int64_t, int64_t, TempArena&, hipStream_t);
+template PaddedB<float> pad_b<float>(const float*, int64_t, int64_t, int64_t, TempArena&, hipStream_t);
+
+namespace {
 
 // Whether a fully populated fp16 grid takes the GEMM-tiled kernel rather than
 // the column batches, by the times the two were measured to take (us, full
