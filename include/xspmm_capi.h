@@ -332,7 +332,8 @@ int xspmm_plan_create(int vtype, int itype, int64_t M, int64_t K, int64_t nnz, c
  * the plan's A, in the original row order: identical to xspmm_spmm_pipeline's
  * C.  Asynchronous on `stream`.  On the fp16 path with N % 8 == 0 it is one
  * kernel launch with the un-permutation fused into the store, which streams
- * the plan's packed column batches when it has them; otherwise it uses a
+ * the plan's packed column batches when it has them (larger fp16 products with
+ * other N: on a padded copy of B, allocated on `stream`); otherwise it uses a
  * device workspace kept by the plan (grown, with a synchronization, when N
  * exceeds every earlier N).  Calls on one plan must not overlap.
  */
