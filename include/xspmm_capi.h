@@ -64,8 +64,8 @@ int xspmm_bcsr_spmm(int vtype, int itype, int64_t M, int64_t K, int64_t Mb, int6
 /*
  * Tier-1 BCSR SpMM that allocates nothing: the same arguments, kernels and
  * result (bit for bit) as xspmm_bcsr_spmm, but every temporary the launch
- * needs (the dispatch order of a long block-row grid, the repacked B panels
- * of the N % 8 != 0 path) comes from a fixed device array of
+ * needs (the dispatch order of a long block-row grid, the padded copy or
+ * repacked panels of a B whose rows start off 16 bytes) comes from a fixed device array of
  * xspmm_noalloc_scratch_bytes() bytes (8 MiB) that each GPU holds for the
  * life of the process.  No hipMalloc, hipFree or allocating library call is
  * made (the array's device address is looked up once per device, on the
