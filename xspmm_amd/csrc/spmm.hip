@@ -1796,9 +1796,11 @@ constexpr int64_t kF32BatchMinGroups = 512;
 // padded copy of B, the batches from 2^18 products of a block with a tile (N =
 // 17: 300980 blocks 123 -> 80, 97367 blocks 43 -> 58; N = 33: 97367 blocks 71 ->
 // 58, 14465 blocks 14 -> 24).
-// whole: the tile kernel covers B (f32_short_wanted).
+// whole: the tile kernel covers B (f32_short_wanted); share: kShared covers the
+// shape, whose 64-column chunks are one grid dimension (so are the tile kernel's
+// groups of tiles: neither reaches the last columns below 2^22).
 F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool aligned, bool whole,
-                            bool contiguous)
+                            bool share, bool contiguous)
 {
     const int64_t tiles = (N + 15) / 16;
     const bool full = nnzb == Mb * Kb;
@@ -1817,14 +1819,17 @@ F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, boo
             spmm_band_f32_times(Mb, Kb, nnzb, (N + 63) / 64 * 64, &one, &balanced);
             shared = std::min(groups <= 256.0 ? 0.65 * one : one, 1.05 * balanced);
         }
-        shared += 1.5 + pad;
-        double batch = std::numeric_limits<double>::infinity();
+        constexpr double kNever = std::numeric_limits<double>::infinity();
+        shared = share ? shared + 1.5 + pad : kNever;
+        double batch = kNever;
         if (!aligned || (full && rows >= (double)kF32BatchMinGroups))
             batch = blocks * (N <= 64 ? std::max(0.13, 0.00048 * rows) : std::max(0.19, 0.00065 * rows)) + 2.5 + pad;
         const int ntw = f32_tiles_per_group(Mb, tiles);
-        const double wgs = (double)Mb * (double)((tiles + ntw - 1) / ntw);
-        const double tile = blocks * std::max(0.045, wgs * (ntw == 1 ? 1.9e-4 : ntw == 2 ? 3.3e-4 : 5.4e-4)) +
-                            (ntw == 4 ? 6.0 : ntw == 2 ? 5.0 : 2.0);
+        const int64_t gy = (tiles + ntw - 1) / ntw;
+        const double wgs = (double)Mb * (double)gy;
+        const double tile = gy > 65535 ? kNever
+                                       : blocks * std::max(0.045, wgs * (ntw == 1 ? 1.9e-4 : ntw == 2 ? 3.3e-4 : 5.4e-4)) +
+                                             (ntw == 4 ? 6.0 : ntw == 2 ? 5.0 : 2.0);
         if (shared < std::min(batch, tile)) return F32Kernel::kShared;
         return batch < tile ? F32Kernel::kBatch : F32Kernel::kTile;
     }
@@ -2213,13 +2218,14 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         const bool aligned = spmm_f32_batch_covers(K, Kb, N, B, C);
         const int64_t Np = (N + 3) / 4 * 4;
         const bool whole = f32_short_wanted(Kb, N);
+        const bool share = spmm_band_f32_covers(K, Kb, Mb, Np, nullptr, nullptr);
         const char* forced = std::getenv("XSPMM_F32_KERNEL");
         F32Kernel kernel = F32Kernel::kTile;
         if ((aligned || spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr)) &&
             !(forced && std::strcmp(forced, "tile") == 0))
             kernel = forced && std::strcmp(forced, "batch") == 0
                          ? F32Kernel::kBatch
-                         : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, whole, contiguous);
+                         : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, whole, share, contiguous);
         const bool order_here = kernel != F32Kernel::kShared && !order_in && spmm_order_wanted(Mb);
         auto shared = [&](const float* bb, int64_t n, int64_t nc) {
             return contiguous
