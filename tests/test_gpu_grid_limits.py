@@ -1,6 +1,7 @@
 """Full grids at the N where one kernel's launch grid ends and another one still
 covers the product: the fp32 shared and tile kernels count 64-column groups in a
-grid dimension of 65535.  Integer values keep every sum exact, so C equals the dense product bit for bit.
+grid dimension of 65535, the fp16 column batches 128-column ones.  Integer values
+keep every sum exact, so C equals the dense product bit for bit.
 """
 from __future__ import annotations
 
@@ -45,3 +46,10 @@ def check(torch, M, K, N, dtype):
 def test_f32_columns_near_the_grid_limit(torch, M, N):
     print(M, N, flush=True)
     check(torch, M, 16, N, torch.float32)
+
+
+# 65535 * 128 = 8388480
+@pytest.mark.parametrize("N", [8388480, 8388488])
+def test_f16_columns_near_the_grid_limit(torch, N):
+    print(N, flush=True)
+    check(torch, 16, 16, N, torch.float16)

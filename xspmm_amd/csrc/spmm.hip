@@ -2093,7 +2093,10 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         const Fp16Kernel choice = fp16_kernel_choice();
         // every block present: GEMM-tiled kernel (matrix-core bound)
         const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, (N + 7) / 8 * 8);
-        const bool tiled = full && dense_f16_pays(Mb, Kb, N);
+        // (its tiles are one grid dimension and take N that the batches do not)
+        const int64_t Np = (N + 7) / 8 * 8;
+        const bool batchable = K * Np * 2 <= (int64_t(1) << 31) && Np < (int64_t(1) << 22) && Kb < (int64_t(1) << 20);
+        const bool tiled = full && (!batchable || dense_f16_pays(Mb, Kb, N));
         if (tiled && N % 8 == 0)
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         const bool offsets32 = K * N * 2 <= (int64_t(1) << 31) && N < (int64_t(1) << 22) &&
@@ -2143,9 +2146,7 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
         // range come here with any N: it multiplies every column of a block,
         // and so must the batches where B holds an Inf or NaN.
-        const int64_t Np = (N + 7) / 8 * 8;
-        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) &&
-            K * Np * 2 <= (int64_t(1) << 31) && Np < (int64_t(1) << 22) && Kb < (int64_t(1) << 20)) {
+        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) && batchable) {
             const bool own_order = !tiled && !order_in && spmm_order_wanted(Mb);
             const PaddedB<uint16_t> pb = pad_b<uint16_t>(b, K, N, own_order ? Mb : 0, arena, s);
             if (pb.bt) {
@@ -2176,7 +2177,7 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
                 return true;
             }
         }
-        if (full && N % 8 == 0)  // B beyond the batches' range, or no room for the marks
+        if (full && N % 8 == 0)  // no room for the marks
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         if (row_map) return false;  // the other fp16 kernels store rows in place
         if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32) {
