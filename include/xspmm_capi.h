@@ -52,8 +52,11 @@ int xspmm_abi_version(void);
  * overwritten.  bvals (and B when it is fp16) must start on a 16-byte
  * boundary: the kernels read them 16 bytes at a time, and a pointer off that
  * boundary fails with XSPMM_ERR_INVALID before anything is launched (the
- * same holds for the entry points below that take them).  Asynchronous on
- * `stream`.
+ * same holds for the entry points below that take them).  Temporaries are
+ * stream-ordered allocations; where B's rows start off 16 bytes, a padded copy
+ * of B of up to 8 MiB (fp16: or instead of panels that are larger too), so that
+ * the kernel is the one that xspmm_bcsr_spmm_noalloc runs
+ * (xspmm_bcsr_spmm_auto has no such limit).  Asynchronous on `stream`.
  * Replaces xspmm::spmm(const BCSRMatrix<In, Idx>&, const In* B, Out* C, Idx N)
  * (reference include/xspmm/xspmm.hpp:14-18, src/hip/unstructured_mtx_mul.hip:108-146).
  */

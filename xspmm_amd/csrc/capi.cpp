@@ -98,7 +98,7 @@ int xspmm_bcsr_spmm(int vtype, int itype, int64_t M, int64_t K, int64_t Mb, int6
             using I = typename decltype(ti)::type;
             bcsr_spmm<T, I>(M, K, Mb, Kb, nnzb, static_cast<const I*>(brp), static_cast<const I*>(bci),
                             static_cast<const T*>(bvals), static_cast<const T*>(B), C, N,
-                            as_stream(stream));
+                            as_stream(stream), kNoAllocScratchBytes);
         });
     });
 }
@@ -168,7 +168,7 @@ int xspmm_bcsr_spmm_ordered(int vtype, int itype, int64_t M, int64_t K, int64_t 
             (void)bcsr_spmm_ex<T, I>(M, K, Mb, Kb, nnzb, static_cast<const I*>(brp),
                                      static_cast<const I*>(bci), static_cast<const T*>(bvals),
                                      static_cast<const T*>(B), C, N, order, nullptr,
-                                     as_stream(stream));
+                                     as_stream(stream), kNoAllocScratchBytes);
         });
     });
 }

@@ -236,10 +236,14 @@ private:
 // float = fp32.
 // ---------------------------------------------------------------------------
 
-// Tier-1 BCSR SpMM with 16x16 blocks.  C[M x N] = A * B[K x N].
+// Tier-1 BCSR SpMM with 16x16 blocks.  C[M x N] = A * B[K x N].  pad_limit: bytes
+// that a padded copy of B may take (kNoAllocScratchBytes: bcsr_spmm_noalloc's
+// kernels, so the same C bit for bit).
+constexpr size_t kNoAllocScratchBytes = size_t(8) << 20;
 template <typename T, typename I>
 void bcsr_spmm(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
-               const I* bci, const T* bvals, const T* B, float* C, int64_t N, hipStream_t s);
+               const I* bci, const T* bvals, const T* B, float* C, int64_t N, hipStream_t s,
+               size_t pad_limit = SIZE_MAX);
 
 // Tier-1 with a precomputed dispatch order (null: built here when useful, see
 // spmm_order_wanted) and an optional output row map: product row r is stored
@@ -249,9 +253,9 @@ void bcsr_spmm(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const
 template <typename T, typename I>
 bool bcsr_spmm_ex(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                   const I* bci, const T* bvals, const T* B, float* C, int64_t N,
-                  const int32_t* order, const I* row_map, hipStream_t s);
+                  const int32_t* order, const I* row_map, hipStream_t s, size_t pad_limit = SIZE_MAX);
 // Tier-1 with the band kernel of T (uint16_t: fp16, float: fp32) where its
-// shape conditions hold, else as bcsr_spmm_ex with no order.  The band
+// shape conditions hold, else as the C entry of bcsr_spmm.  The band
 // kernels are only correct when every block-row is one contiguous run of
 // block columns (spmm_band_wanted checks).
 template <typename T, typename I>
@@ -271,8 +275,8 @@ size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N);
 // B with rows of Np columns (N rounded up to 16 bytes; B itself when its rows
 // start there already) and its marks (256 bytes, one set where a part of B holds
 // an Inf or NaN), made on the stream by pad_b_kernel, and room for order_rows
-// int32, all one piece of the arena (an allocation costs the host about 15 us);
-// bt null when a fixed arena has no room for it.  T: uint16_t (fp16) or float.
+// int32, all one piece of the arena (an allocation costs the host about 15 us).
+// T: uint16_t (fp16) or float.
 template <typename T>
 struct PaddedB {
     const T* bt = nullptr;
@@ -294,7 +298,6 @@ bool all_finite_f16(const void* values, int64_t n, hipStream_t s);
 // Tier-1 without any allocation: the temporaries come from a fixed device
 // array of kNoAllocScratchBytes (one copy per GPU, shared by every call on
 // it).  Throws std::invalid_argument when a product needs more.
-constexpr size_t kNoAllocScratchBytes = size_t(8) << 20;
 template <typename T, typename I>
 void bcsr_spmm_noalloc(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                        const I* bci, const T* bvals, const T* B, float* C, int64_t N,

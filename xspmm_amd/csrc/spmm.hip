@@ -2011,6 +2011,25 @@ bool spmm_dispatch_order_cols(const I* brp, const I* bci, int64_t Mb, int32_t* o
 template bool spmm_dispatch_order_cols<int32_t>(const int32_t*, const int32_t*, int64_t, int32_t*, hipStream_t);
 template bool spmm_dispatch_order_cols<int64_t>(const int64_t*, const int64_t*, int64_t, int32_t*, hipStream_t);
 
+namespace {
+
+// pad_b's piece of the arena (value_bytes a value; copy: B's rows start off 16 bytes)
+struct PadPieces {
+    size_t marks, bt, order, end;
+};
+PadPieces pad_pieces(int value_bytes, int64_t K, int64_t Np, bool copy, int64_t order_rows)
+{
+    Carve cv;
+    PadPieces p;
+    p.marks = cv.take(kPadMarks);
+    p.bt = cv.take(copy ? (size_t)(K > 0 ? K : 1) * (size_t)Np * (size_t)value_bytes : 0);
+    p.order = cv.take((size_t)order_rows * sizeof(int32_t));
+    p.end = cv.end;
+    return p;
+}
+
+}  // namespace
+
 template <typename T>
 PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena& arena, hipStream_t s)
 {
@@ -2019,17 +2038,13 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     PaddedB<T> p;
     p.Np = (N + V - 1) / V * V;
     const bool copy = p.Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
-    Carve cv;
-    const size_t o_marks = cv.take(kPadMarks);
-    const size_t o_bt = cv.take(copy ? (size_t)(K > 0 ? K : 1) * (size_t)p.Np * sizeof(T) : 0);
-    const size_t o_order = cv.take((size_t)order_rows * sizeof(int32_t));
-    if (!arena.fits(cv.end)) return p;
-    char* const base = static_cast<char*>(arena.take(cv.end));
+    const PadPieces at = pad_pieces(sizeof(T), K, p.Np, copy, order_rows);
+    char* const base = static_cast<char*>(arena.take(at.end));
     const int64_t vecs = K * (p.Np / V);
     const dim3 wgs((unsigned)std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads)));
     const U* src = reinterpret_cast<const U*>(B);
-    U* bt = copy ? reinterpret_cast<U*>(base + o_bt) : nullptr;
-    unsigned char* marks = reinterpret_cast<unsigned char*>(base + o_marks);
+    U* bt = copy ? reinterpret_cast<U*>(base + at.bt) : nullptr;
+    unsigned char* marks = reinterpret_cast<unsigned char*>(base + at.marks);
     if (copy)
         hipLaunchKernelGGL((pad_b_kernel<U, true>), wgs, dim3(kPadThreads), 0, s, src, bt, K, N, p.Np, marks);
     else
@@ -2037,7 +2052,7 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     XSPMM_LAUNCH_CHECK();
     p.bt = copy ? reinterpret_cast<const T*>(bt) : B;
     p.marks = reinterpret_cast<const uint32_t*>(marks);
-    p.order = reinterpret_cast<int32_t*>(base + o_order);
+    p.order = reinterpret_cast<int32_t*>(base + at.order);
     return p;
 }
 template PaddedB<uint16_t> pad_b<uint16_t>(const uint16_t*, int64_t, int64_t, int64_t, TempArena&, hipStream_t);
@@ -2069,11 +2084,14 @@ bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
 // The Tier-1 launcher: kernel choice as described at the top of this file;
 // temporaries (the dispatch order, repacked B panels) come from `arena`.
 // contiguous (fp32): every block-row is one run of block columns.
+// pad_limit: the temporaries a padded copy of B may take.  The choice depends on
+// sizes, types and alignment alone, never on the room an arena has left, so calls
+// given the same limit run the same kernels.
 template <typename T, typename I>
 bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                       const I* bci, const T* bvals, const T* B, float* C, int64_t N,
                       const int32_t* order_in, const I* row_map, TempArena& arena, hipStream_t s,
-                      bool contiguous = false)
+                      size_t pad_limit = SIZE_MAX, bool contiguous = false)
 {
     check_shape(M, K, Mb, Kb, nnzb, N);
     if (M == 0 || N == 0 || Mb == 0) return true;
@@ -2146,38 +2164,40 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
         // range come here with any N: it multiplies every column of a block,
         // and so must the batches where B holds an Inf or NaN.
-        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) && batchable) {
-            const bool own_order = !tiled && !order_in && spmm_order_wanted(Mb);
+        // (Beyond the limit N % 8 != 0 repacks panels, unless those exceed it too.)
+        const size_t panel_bytes = (size_t)(Kb > 0 ? Kb : 1) * (size_t)(ntiles64 * 16) * 16 * sizeof(uint16_t);
+        // An order counts whether or not the caller has one: it decides no kernel.
+        const bool own_order = !tiled && !order_in && spmm_order_wanted(Mb);
+        const size_t pad_bytes = pad_pieces(2, K, Np, N % 8 != 0, !tiled && spmm_order_wanted(Mb) ? Mb : 0).end;
+        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) && batchable &&
+            (pad_bytes <= pad_limit || (N % 8 != 0 && panel_bytes > pad_limit))) {
             const PaddedB<uint16_t> pb = pad_b<uint16_t>(b, K, N, own_order ? Mb : 0, arena, s);
-            if (pb.bt) {
-                if (tiled)
-                    return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
-                const int32_t* order = order_in;
-                if (own_order) {
-                    spmm_dispatch_order<I>(brp, Mb, pb.order, s);
-                    order = pb.order;
-                }
-                BatchPack pk{};
-                pk.nc = N;
-                pk.nonfinite = pb.marks;
-                auto launch = [&](auto nt) {
-                    hipLaunchKernelGGL((spmm_f16_batch_kernel<I, decltype(nt)::value, BatchMode::kMultiply, 1, false, true>),
-                                       ggrid, dim3(64 * kBW), 0, s, brp, bci, v, pb.bt, C, M, K, Np, Kb, order,
-                                       row_map, pk);
-                };
-                if (N <= 16)
-                    launch(std::integral_constant<int, 1>{});
-                else if (N <= 32)
-                    launch(std::integral_constant<int, 2>{});
-                else if (N <= 64)
-                    launch(std::integral_constant<int, 4>{});
-                else
-                    launch(std::integral_constant<int, 8>{});
-                XSPMM_LAUNCH_CHECK();
-                return true;
+            if (tiled) return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
+            const int32_t* order = order_in;
+            if (own_order) {
+                spmm_dispatch_order<I>(brp, Mb, pb.order, s);
+                order = pb.order;
             }
+            BatchPack pk{};
+            pk.nc = N;
+            pk.nonfinite = pb.marks;
+            auto launch = [&](auto nt) {
+                hipLaunchKernelGGL((spmm_f16_batch_kernel<I, decltype(nt)::value, BatchMode::kMultiply, 1, false, true>),
+                                   ggrid, dim3(64 * kBW), 0, s, brp, bci, v, pb.bt, C, M, K, Np, Kb, order,
+                                   row_map, pk);
+            };
+            if (N <= 16)
+                launch(std::integral_constant<int, 1>{});
+            else if (N <= 32)
+                launch(std::integral_constant<int, 2>{});
+            else if (N <= 64)
+                launch(std::integral_constant<int, 4>{});
+            else
+                launch(std::integral_constant<int, 8>{});
+            XSPMM_LAUNCH_CHECK();
+            return true;
         }
-        if (full && N % 8 == 0)  // no room for the marks
+        if (full && N % 8 == 0)  // the marks and an order exceed the limit
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         if (row_map) return false;  // the other fp16 kernels store rows in place
         if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32) {
@@ -2191,7 +2211,7 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             return true;
         }
         const int64_t Nw = ntiles64 * 16;
-        uint16_t* bt = arena.take_as<uint16_t>((size_t)(Kb > 0 ? Kb : 1) * (size_t)Nw * 16);
+        uint16_t* bt = static_cast<uint16_t*>(arena.take(panel_bytes));
         if (Kb > 0) {
             const int64_t per_kb = Nw * 2;
             const dim3 pg((unsigned)((per_kb + 255) / 256), (unsigned)(Kb < 65535 ? Kb : 65535));
@@ -2227,6 +2247,11 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             kernel = forced && std::strcmp(forced, "batch") == 0
                          ? F32Kernel::kBatch
                          : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, whole, share, contiguous);
+        if (kernel != F32Kernel::kTile && !aligned) {
+            const bool copy = Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
+            const int64_t order_rows = kernel == F32Kernel::kBatch && spmm_order_wanted(Mb) ? Mb : 0;
+            if (pad_pieces(4, K, Np, copy, order_rows).end > pad_limit) kernel = F32Kernel::kTile;
+        }
         const bool order_here = kernel != F32Kernel::kShared && !order_in && spmm_order_wanted(Mb);
         auto shared = [&](const float* bb, int64_t n, int64_t nc) {
             return contiguous
@@ -2248,12 +2273,10 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             // N % 4 != 0, or B or C off 16 bytes: the same kernels on a padded
             // copy of B
             const PaddedB<float> pb = pad_b<float>(b, K, N, order_here ? Mb : 0, arena, s);
-            if (pb.bt && kernel == F32Kernel::kShared) return shared(pb.bt, Np, N);
-            if (pb.bt) {
-                bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order_with(pb.order), row_map, s, N,
-                                       pb.marks);
-                return true;
-            }
+            if (kernel == F32Kernel::kShared) return shared(pb.bt, Np, N);
+            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order_with(pb.order), row_map, s, N,
+                                   pb.marks);
+            return true;
         }
         const int ntw = f32_tiles_per_group(Mb, ntiles);
         const int64_t gy = (ntiles + ntw - 1) / ntw;
@@ -2336,21 +2359,21 @@ void* noalloc_scratch(int dev)
 
 template <typename T, typename I>
 void bcsr_spmm(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
-               const I* bci, const T* bvals, const T* B, float* C, int64_t N, hipStream_t s)
+               const I* bci, const T* bvals, const T* B, float* C, int64_t N, hipStream_t s, size_t pad_limit)
 {
     TempArena arena(s);
     (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, nullptr, nullptr,
-                                 arena, s);
+                                 arena, s, pad_limit);
 }
 
 template <typename T, typename I>
 bool bcsr_spmm_ex(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                   const I* bci, const T* bvals, const T* B, float* C, int64_t N,
-                  const int32_t* order_in, const I* row_map, hipStream_t s)
+                  const int32_t* order_in, const I* row_map, hipStream_t s, size_t pad_limit)
 {
     TempArena arena(s);
     return bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order_in, row_map,
-                                  arena, s);
+                                  arena, s, pad_limit);
 }
 
 template <typename T, typename I>
@@ -2365,7 +2388,7 @@ void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
     } else {
         if (bcsr_spmm_band_f32<I>(M, K, Mb, Kb, brp, bci, bvals, B, C, N, nullptr, nnzb, s)) return;
     }
-    (void)bcsr_spmm_ex<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, nullptr, nullptr, s);
+    bcsr_spmm<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, s, kNoAllocScratchBytes);
 }
 
 template <typename T, typename I>
@@ -2389,7 +2412,8 @@ void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
         }
     }
     const bool contiguous = sizeof(T) == 4 && band && spmm_band_f32_covers(K, Kb, Mb, (N + 3) / 4 * 4, nullptr, nullptr);
-    (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order, nullptr, arena, s, contiguous);
+    (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order, nullptr, arena, s, SIZE_MAX,
+                                 contiguous);
 }
 
 size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N)
@@ -2425,15 +2449,16 @@ void bcsr_spmm_noalloc(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnz
     XSPMM_HIP_CHECK(hipGetDevice(&dev));
     TempArena arena(noalloc_scratch(dev), kNoAllocScratchBytes, s);
     (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, nullptr, nullptr,
-                                 arena, s);
+                                 arena, s, kNoAllocScratchBytes);
 }
 
 #define XSPMM_SPMM_EX(T, I)                                                                      \
     template bool bcsr_spmm_ex<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*,      \
                                      const I*, const T*, const T*, float*, int64_t,              \
-                                     const int32_t*, const I*, hipStream_t);                     \
+                                     const int32_t*, const I*, hipStream_t, size_t);             \
     template void bcsr_spmm<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*,         \
-                                  const I*, const T*, const T*, float*, int64_t, hipStream_t);   \
+                                  const I*, const T*, const T*, float*, int64_t, hipStream_t,    \
+                                   size_t);                                                      \
     template void bcsr_spmm_noalloc<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*, \
                                           const I*, const T*, const T*, float*, int64_t,         \
                                           hipStream_t);
