@@ -958,7 +958,12 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
     uint32_t pending = 0;
     float inexact = 0.f;  // EX: 0 while every A' value is finite, else NaN
 
-    auto finish = [&]() __attribute__((always_inline)) {
+    // later: vector memory operations issued since the tile's loads, at least
+    // (kDma: loads complete in order, so waiting down to that many leaves the
+    // tile whole; the wait is written out because the compiler's own rests on
+    // its alias analysis, which a second LDS object in the kernel misleads)
+    auto finish = [&](auto later) __attribute__((always_inline)) {
+        if constexpr (kDma) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(later)::value) : "memory");
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             unsigned char* const T = tile(c);
@@ -990,9 +995,9 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
     int64_t pbase = 0;
     if constexpr (MODE == BatchMode::kPack) pbase = pk.offsets[br * kBW + wave];
     // Close the open batch of `cnt` slots: A' from the D registers (exact
-    // fp16 values), then multiply the previous batch and issue this one's
-    // B row loads in K order.
-    auto start = [&](uint32_t cnt) __attribute__((always_inline)) {
+    // fp16 values), then multiply the previous batch (later: see finish) and
+    // issue this one's B row loads in K order.
+    auto start = [&](uint32_t cnt, auto later) __attribute__((always_inline)) {
         if constexpr (MODE == BatchMode::kCount) {
             ++nbatch;
             return;
@@ -1016,7 +1021,7 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
 #pragma unroll
             for (int e = 0; e < 8; ++e) inexact = __builtin_fmaf((float)a[e], 0.f, inexact);
         }
-        if (started) finish();
+        if (started) finish(later);
         aop = a;
         uint32_t row[NT];
 #pragma unroll
@@ -1048,6 +1053,8 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
                         u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)off, 0, 0));
                 }
             }
+        // no load moves across: finish counts those that follow
+        if constexpr (kDma) asm volatile("" ::: "memory");
         started = true;
     };
 
@@ -1072,8 +1079,12 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
         *lds_ptr<uint16_t>(at) = (uint16_t)0u;
     };
 
-    // pair j of the ring pass whose index window is `win`
-    auto process = [&](const half8_t& pa, uint32_t win, int j) __attribute__((always_inline)) {
+    // pair j of the ring pass whose index window is `win`.  At least one load
+    // follows a batch's B rows before the next batch closes (stage_a after every
+    // pair), two at the start of a pass (its window).
+    auto process = [&](const half8_t& pa, uint32_t win, auto pair) __attribute__((always_inline)) {
+        constexpr int j = decltype(pair)::value;
+        constexpr std::integral_constant<int, j == 0 ? 2 : 1> later{};
         uint32_t c0, c1;
         // this lane's block column (lane l: block l >> 5 of the pair)
         uint32_t csel;
@@ -1114,7 +1125,7 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
         if (pm == 0u) return;
         const uint32_t cnt = (uint32_t)__builtin_popcount(pm);
         if (pending + cnt > 32u) {
-            start(pending);
+            start(pending, later);
             pending = 0;
         }
         if constexpr (MODE != BatchMode::kCount) {
@@ -1163,43 +1174,43 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
             }
             // next pass's window, issued a pass ahead like the A loads
             const uint32_t nwin = load_cols(q + A);
-            process(P0, win, 0);
+            process(P0, win, std::integral_constant<int, 0>{});
             stage_a(q + A, P0);
-            process(P1, win, 1);
+            process(P1, win, std::integral_constant<int, 1>{});
             stage_a(q + A + S, P1);
-            process(P2, win, 2);
+            process(P2, win, std::integral_constant<int, 2>{});
             stage_a(q + A + 2 * S, P2);
-            process(P3, win, 3);
+            process(P3, win, std::integral_constant<int, 3>{});
             stage_a(q + A + 3 * S, P3);
             if constexpr (D > 4) {
-                process(P4, win, 4);
+                process(P4, win, std::integral_constant<int, 4>{});
                 stage_a(q + A + 4 * S, P4);
             }
             if constexpr (D > 5) {
-                process(P5, win, 5);
+                process(P5, win, std::integral_constant<int, 5>{});
                 stage_a(q + A + 5 * S, P5);
             }
             if constexpr (D > 6) {
-                process(P6, win, 6);
+                process(P6, win, std::integral_constant<int, 6>{});
                 stage_a(q + A + 6 * S, P6);
             }
             if constexpr (D > 7) {
-                process(P7, win, 7);
+                process(P7, win, std::integral_constant<int, 7>{});
                 stage_a(q + A + 7 * S, P7);
             }
             if constexpr (D > 8) {
-                process(P8, win, 8);
+                process(P8, win, std::integral_constant<int, 8>{});
                 stage_a(q + A + 8 * S, P8);
             }
             if constexpr (D > 9) {
-                process(P9, win, 9);
+                process(P9, win, std::integral_constant<int, 9>{});
                 stage_a(q + A + 9 * S, P9);
             }
             win = nwin;
         }
-        if (pending > 0u) start(pending);
+        if (pending > 0u) start(pending, std::integral_constant<int, 1>{});
         if constexpr (MODE == BatchMode::kMultiply) {
-            if (started) finish();
+            if (started) finish(std::integral_constant<int, 0>{});
         }
     }
     if constexpr (MODE == BatchMode::kCount) {
@@ -1209,10 +1220,7 @@ __global__ __launch_bounds__(64 * kBW, NC == 1 ? kBW : kBW / 2) void spmm_f16_ba
         return;
     } else {
         if constexpr (EX) {
-            // the waves' answers through smem, not __syncthreads_or: with a
-            // second LDS object in the kernel the compiler takes the tile's
-            // reads not to alias the direct-to-LDS loads and leaves out the
-            // wait between them
+            // the waves' answers through smem (no second LDS object: see finish)
             const uint64_t bad = __builtin_amdgcn_ballot_w64(pk.nonfinite[lane] != 0u || inexact != 0.f);
             uint32_t* const ws = reinterpret_cast<uint32_t*>(smem);
             __syncthreads();
