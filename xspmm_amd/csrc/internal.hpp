@@ -401,6 +401,8 @@ bool spmm_band_f16_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N);
 bool spmm_band_f32_covers(int64_t K, int64_t Kb, int64_t Mb, int64_t N, const void* B, const void* C);
 // Estimated times (us) of its two launches for N columns.
 void spmm_band_f32_times(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, double* one, double* balanced);
+// Whether the estimates pick its balanced launch.
+bool spmm_band_f32_balances(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N);
 template <typename I>
 bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const float* bvals, const float* B, float* C, int64_t N, const I* row_map,

@@ -1789,7 +1789,7 @@ constexpr int64_t kF32BatchMinGroups = 512;
 //            runs 1.5 times as fast as two);
 //   kBatch:  0.13 (N <= 64) or 0.19 on a short grid, then with its workgroups;
 //   kTile:   with its workgroups and the columns of each;
-//   padding B costs 18 more.  kTile and kShared multiply whole blocks, as does
+//   padding B costs 18 more (its allocation included).  kTile and kShared multiply whole blocks, as does
 //   kBatch on a padded copy; kBatch on B itself skips zero columns, which an
 //   Inf in B shows, so it stays with the full grids of 512 workgroups or more.
 //   4096 x 4096 full, tile / batch / shared: N = 8 16 / 33 / 84, N = 64 40 / 33 /
@@ -1807,15 +1807,24 @@ constexpr int64_t kF32BatchMinGroups = 512;
 // whole: the tile kernel covers B (f32_short_wanted); share: kShared covers the
 // shape, whose 64-column chunks are one grid dimension (so are the tile kernel's
 // groups of tiles: neither reaches the last columns below 2^22).
+// Bands of more than 64 columns keep the kernel their rows were chosen for where
+// B's rows start on 16 bytes (tile is ahead only on small grids: 4096^2 80 %, N =
+// 128, 44 / 57).  Elsewhere the copy of B (6 us, with scratch at hand) and the
+// launch that the band kernel would take count too: its balanced launch 1.35 times
+// its estimate, and the tile kernel 1.15 times, so that it is taken only where it
+// is ahead.  192 bands of 1024^2 to 16384^2, 2 to 80 %, N = 65 .. 511, shared / tile:
+// 1024^2 80 % N = 127 49 / 8; 2048^2 80 % N = 511 103 / 49; 4096^2 50 % N = 129 70 /
+// 48, N = 257 77 / 79; 8192^2 5 % N = 65 17 / 22; 16384^2 50 % N = 127 276 / 527: the
+// choice is never the slower one by more than 1.23, and by 1 % on average.
 F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool aligned, bool whole,
                             bool share, bool contiguous)
 {
     const int64_t tiles = (N + 15) / 16;
     const bool full = nnzb == Mb * Kb;
-    // a band of more columns keeps the kernel its rows were chosen for (tile is
-    // ahead only on small grids: 4096^2 80 %, N = 128, 44 / 57)
-    if ((full || (contiguous && N <= 64)) && nnzb > 0 && whole && N < (int64_t(1) << 22) && Kb < (int64_t(1) << 20)) {
-        const double pad = aligned ? 0.0 : 18.0;
+    const bool wide_band = contiguous && !full && N > 64 && !aligned;
+    if ((full || wide_band || (contiguous && N <= 64)) && nnzb > 0 && whole && N < (int64_t(1) << 22) &&
+        Kb < (int64_t(1) << 20)) {
+        const double pad = aligned ? 0.0 : wide_band ? 6.0 : 18.0;
         const double blocks = (double)nnzb / (double)Mb;
         const double groups = (double)((Mb + 3) / 4) * (double)((N + 63) / 64);
         const double rows = (double)Mb * (double)((N + 127) / 128);
@@ -1825,7 +1834,11 @@ F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, boo
         } else {
             double one, balanced;
             spmm_band_f32_times(Mb, Kb, nnzb, (N + 63) / 64 * 64, &one, &balanced);
-            shared = std::min(groups <= 256.0 ? 0.65 * one : one, 1.05 * balanced);
+            if (groups <= 256.0) one *= 0.65;
+            if (!wide_band)
+                shared = std::min(one, 1.05 * balanced);
+            else
+                shared = spmm_band_f32_balances(Mb, Kb, nnzb, (N + 3) / 4 * 4) ? 1.35 * balanced : one;
         }
         constexpr double kNever = std::numeric_limits<double>::infinity();
         shared = share ? shared + 1.5 + pad : kNever;
@@ -1838,6 +1851,7 @@ F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, boo
         const double tile = gy > 65535 ? kNever
                                        : blocks * std::max(0.045, wgs * (ntw == 1 ? 1.9e-4 : ntw == 2 ? 3.3e-4 : 5.4e-4)) +
                                              (ntw == 4 ? 6.0 : ntw == 2 ? 5.0 : 2.0);
+        if (wide_band) return 1.15 * tile < shared ? F32Kernel::kTile : F32Kernel::kShared;
         if (shared < std::min(batch, tile)) return F32Kernel::kShared;
         return batch < tile ? F32Kernel::kBatch : F32Kernel::kTile;
     }

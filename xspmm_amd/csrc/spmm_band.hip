@@ -997,6 +997,16 @@ void spmm_band_f32_times(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, double
     *balanced = W + 25.0;
 }
 
+// Where the one-group-per-workgroup launch is predicted to take 10 % longer.
+// Measured rule: it picks the faster launch on every band of 4096^2 to
+// 16384^2 and N of 64 to 256 timed both ways.
+bool spmm_band_f32_balances(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N)
+{
+    double one, balanced;
+    spmm_band_f32_times(Mb, Kb, nnzb, N, &one, &balanced);
+    return one > 1.1 * balanced;
+}
+
 template <typename I>
 bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp, const I* bci,
                         const float* bvals, const float* B, float* C, int64_t N, const I* row_map,
@@ -1008,17 +1018,9 @@ bool bcsr_spmm_band_f32(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* b
     const int64_t chunks = (N + 63) / 64;
     const int64_t P = std::min<int64_t>(kPlanSlots, ((int64_t)band_device_cus() + 7) / 8 * 8);
     const size_t tile_bytes = (size_t)chunks * 2 * (size_t)P * kBandPart32 * sizeof(float);
-    // The balanced launch (on grids of at most kPlanGroups groups) where the
-    // one-group-per-workgroup launch is predicted to take 10 % longer.
-    // Measured rule: it picks the faster launch on every band of 4096^2 to
-    // 16384^2 and N of 64 to 256 timed both ways.
+    // the balanced launch, on grids of at most kPlanGroups groups
     const int mode = band_split_mode();
-    bool pays = false;
-    if (mode == 1) {
-        double one, balanced;
-        spmm_band_f32_times(Mb, Kb, nnzb, N, &one, &balanced);
-        pays = one > 1.1 * balanced;
-    }
+    const bool pays = mode == 1 && spmm_band_f32_balances(Mb, Kb, nnzb, N);
     if (mode > 0 && nnzb > 0 && (mode == 2 || pays) && G <= kPlanGroups && tile_bytes <= (size_t(512) << 20)) {
         Carve cv;
         const size_t o_S = cv.take((size_t)(G + 1) * sizeof(int64_t));
