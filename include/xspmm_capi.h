@@ -193,15 +193,27 @@ int xspmm_bcsr_spmm_band(int vtype, int itype, int64_t M, int64_t K, int64_t Mb,
  * that is the band kernel where it is the faster one (for fp32 not below
  * about 32 columns, nor on small grids).  scratch (NULL, or 256-byte aligned
  * device memory of scratch_bytes, kept until the call's work on `stream` is
- * done) holds a product's temporaries if they fit: 512 + K * N' * value bytes
- * + 4 * Mb do for every product, rounded up to 256 each, N' = N rounded up to
- * a multiple of 16 bytes.  What does not fit is allocated on the stream.
+ * done) holds the call's temporaries: xspmm_bcsr_spmm_scratch says how many bytes
+ * they are (0 for most).  What does not fit is allocated on the stream, and so is
+ * the plan of an fp32 band whose blocks are shared out over the CUs.  Where the
+ * device has no memory for a padded copy of B, the product takes a kernel without.
  * Asynchronous on `stream`.
  * Replaces the same call as xspmm_bcsr_spmm.
  */
 int xspmm_bcsr_spmm_auto(int vtype, int itype, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb,
                          const void* brp, const void* bci, const void* bvals, const void* B, float* C, int64_t N,
                          const int32_t* order, int band, void* scratch, int64_t scratch_bytes, void* stream);
+
+/*
+ * *bytes = the scratch that xspmm_bcsr_spmm_auto uses for a product of these sizes
+ * (a padded copy of B where its rows start off 16 bytes, its marks, an order on a
+ * long grid that is given none).  B and C are looked at for their alignment only
+ * (NULL: 16-byte aligned); ordered: whether the call is given an order.  Host only:
+ * nothing is launched.
+ * No counterpart in the reference.
+ */
+int xspmm_bcsr_spmm_scratch(int vtype, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const void* B,
+                            const float* C, int64_t N, int ordered, int band, int64_t* bytes);
 
 /*
  * CSR -> BCSR, phase 1: writes bcsr_row_ptr[Mb+1] (device) for r x c blocks,

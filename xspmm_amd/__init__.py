@@ -73,6 +73,8 @@ def load():
     L.xspmm_bcsr_spmm_band.argtypes = [i32, i32, i64, i64, i64, i64, i64, p, p, p, p, p, i64, p]
     L.xspmm_bcsr_spmm_auto.restype = i32
     L.xspmm_bcsr_spmm_auto.argtypes = [i32, i32, i64, i64, i64, i64, i64, p, p, p, p, p, i64, p, i32, p, i64, p]
+    L.xspmm_bcsr_spmm_scratch.restype = i32
+    L.xspmm_bcsr_spmm_scratch.argtypes = [i32, i64, i64, i64, i64, i64, p, p, i64, i32, i32, C.POINTER(i64)]
     L.xspmm_bcsr_dispatch_order_cols.restype = i32
     L.xspmm_bcsr_dispatch_order_cols.argtypes = [i32, i64, p, p, p, C.POINTER(C.c_int), p]
     L.xspmm_csr_to_bcsr_count.restype = i32
@@ -278,6 +280,8 @@ class BCSRMatrix:
     _band: object = field(default=None, repr=False, compare=False)
     _band_key: object = field(default=None, repr=False, compare=False)
     _nnz: int = field(default=0, repr=False, compare=False)
+    # The last answer of _scratch_bytes and what it was for.
+    _scratch: object = field(default=((), 0), repr=False, compare=False)
 
     @property
     def num_blocks(self) -> int:
@@ -306,6 +310,20 @@ class BCSRMatrix:
             self._order = order[:int(self.num_block_rows)] if written.value else None
             self._order_key = key
         return self._order
+
+    def _scratch_bytes(self, vt, N, b_at, c_at, ordered, band):
+        """Scratch that a product of N columns uses (xspmm_bcsr_spmm_scratch):
+        from sizes, types and alignment alone."""
+        sizes = (vt, self.num_rows, self.num_cols, self.num_block_rows, self.num_block_cols, self.num_blocks,
+                 b_at % 16, c_at % 16, N, ordered, band)
+        known, n = self._scratch
+        if known != sizes:
+            out = C.c_int64(0)
+            _check(load().xspmm_bcsr_spmm_scratch(vcode(vt), *sizes[1:6], b_at % 16, c_at % 16, N, int(ordered),
+                                                  int(band), C.byref(out)))
+            n = out.value
+            self._scratch = (sizes, n)
+        return n
 
     def band_rows(self) -> bool:
         """Whether Tier-1 multiplies this grid with a band kernel (decided on
@@ -378,22 +396,31 @@ def spmm(A: BCSRMatrix, B, C_out=None, N: int | None = None):
     key = A._layout_key()
     band = A._band if A._band_key == key else A._find_band(key)
     order = A._order if A._order_key == key else A._find_order(key)
-    # rows of B off 16 bytes: a product may take a padded copy of B (and, on a
-    # long grid, an order), from torch's allocator, which costs a tenth of the
-    # library's own stream-ordered allocation.  Freed on this stream when the
-    # call returns, so only later work of the same stream reuses it.
-    vec = 8 if vt is torch.float16 else 4
+    # rows of B off 16 bytes, or a full fp16 grid: what the product takes beside
+    # its operands (a padded copy of B, marks) comes from torch's allocator,
+    # which costs a tenth of the library's own stream-ordered allocation.
+    # Freed on this stream when the call returns, so only later work of the same
+    # stream reuses it.
+    b_at, c_at = B.data_ptr(), C_out.data_ptr()
     ws, ws_bytes = None, 0
     cur = torch.cuda.current_device()
-    if N % vec and dev.index == cur:
-        ws_bytes = 1024 + A.num_cols * (N + vec) * (16 // vec) + 4 * A.num_block_rows
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    if vt is torch.float16:
+        temps = N % 8 or ci.numel() == A.num_block_rows * A.num_block_cols
+    else:
+        temps = N % 4 or (b_at | c_at) % 16
+    if temps and dev.index == cur:
+        ws_bytes = A._scratch_bytes(vt, N, b_at, c_at, order is not None, bool(band))
+        if ws_bytes:
+            try:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:  # the library does without
+                ws_bytes = 0
     # (an empty tensor's address is not passed on)
     rc = L.xspmm_bcsr_spmm_auto(codes[vt] if vt in codes else vcode(vt),
                                 codes[rp.dtype] if rp.dtype in codes else icode(rp.dtype), A.num_rows, A.num_cols,
                                 A.num_block_rows, A.num_block_cols, ci.numel(), rp.data_ptr(),
-                                ci.data_ptr() or None, vals.data_ptr() or None, B.data_ptr() or None,
-                                C_out.data_ptr() or None, N,
+                                ci.data_ptr() or None, vals.data_ptr() or None, b_at or None,
+                                c_at or None, N,
                                 order.data_ptr() if order is not None else None, 1 if band else 0,
                                 ws.data_ptr() if ws is not None else None, ws_bytes,
                                 _raw_stream(cur))

@@ -225,6 +225,17 @@ int xspmm_bcsr_spmm_auto(int vtype, int itype, int64_t M, int64_t K, int64_t Mb,
     });
 }
 
+int xspmm_bcsr_spmm_scratch(int vtype, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const void* B,
+                            const float* C, int64_t N, int ordered, int band, int64_t* bytes)
+{
+    return guarded([&] {
+        require(bytes != nullptr, "bytes is null");
+        if (vtype != XSPMM_F16 && vtype != XSPMM_F32) throw std::invalid_argument("xSpMM: unknown value type.");
+        *bytes = (int64_t)bcsr_spmm_scratch(vtype == XSPMM_F16 ? 2 : 4, M, K, Mb, Kb, nnzb, B, C, N, ordered != 0,
+                                            band != 0);
+    });
+}
+
 int xspmm_csr_to_bcsr_count(int itype, int64_t M, int64_t K, int64_t nnz, const void* rp,
                             const void* ci, int64_t r_block, int64_t c_block,
                             void* bcsr_row_ptr, int64_t* nnzb_out, void* stream)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <new>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -44,6 +45,19 @@ public:
             XSPMM_HIP_CHECK(hipGetDevice(&dev));
             init_device_pool(dev);
             XSPMM_HIP_CHECK(hipMallocAsync(&p_, bytes, s));
+        }
+    }
+    // for callers that can do without: null when there is no memory for it
+    Scratch(size_t bytes, hipStream_t s, std::nothrow_t) : s_(s) {
+        int dev = 0;
+        XSPMM_HIP_CHECK(hipGetDevice(&dev));
+        init_device_pool(dev);
+        const hipError_t e = hipMallocAsync(&p_, bytes, s);
+        if (e == hipErrorOutOfMemory) {
+            p_ = nullptr;
+            (void)hipGetLastError();  // reported here
+        } else {
+            XSPMM_HIP_CHECK(e);
         }
     }
     ~Scratch() {
@@ -126,12 +140,16 @@ public:
         const size_t at = (used_ + 255) & ~size_t(255);
         return !base_ || spill_ || (at <= cap_ && bytes <= cap_ - at);
     }
-    void* take(size_t bytes) {
+    // or_null: null rather than an error when the device has no memory left
+    void* take(size_t bytes, bool or_null = false) {
         if (bytes == 0) return nullptr;
         const size_t at = (used_ + 255) & ~size_t(255);
         const bool room = base_ && at <= cap_ && bytes <= cap_ - at;
         if (!base_ || (spill_ && !room)) {
-            owned_.emplace_back(bytes, s_);
+            if (or_null)
+                owned_.emplace_back(bytes, s_, std::nothrow);
+            else
+                owned_.emplace_back(bytes, s_);
             return owned_.back().get();
         }
         if (!room)
@@ -264,19 +282,23 @@ void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
 // Tier-1 with everything kept on a matrix: its dispatch order (or null) and
 // whether its block-rows are contiguous runs (band; spmm_band_wanted).  The
 // kernel follows from the sizes: a contiguous grid takes a band kernel where
-// that is the faster one.  Temporaries come from scratch (bcsr_spmm_scratch
-// bytes always do; null or less: stream-ordered allocations), which the caller
-// keeps for the call's work on s.
+// that is the faster one.  Temporaries come from scratch, which the caller keeps
+// for the call's work on s; what does not fit is a stream-ordered allocation.
 template <typename T, typename I>
 void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp, const I* bci,
                     const T* bvals, const T* B, float* C, int64_t N, const int32_t* order, bool band, void* scratch,
                     size_t scratch_bytes, hipStream_t s);
-size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N);
+// Bytes of scratch that such a call uses: from the sizes, the alignment of B and C
+// (null: aligned) and the diagnostic switches; ordered: the call is given an order.
+// The fp32 band kernel's balanced launch allocates its plan beside them.
+size_t bcsr_spmm_scratch(int value_bytes, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const void* B,
+                         const void* C, int64_t N, bool ordered, bool band);
 // B with rows of Np columns (N rounded up to 16 bytes; B itself when its rows
 // start there already) and its marks (256 bytes, one set where a part of B holds
 // an Inf or NaN), made on the stream by pad_b_kernel, and room for order_rows
 // int32, all one piece of the arena (an allocation costs the host about 15 us).
-// T: uint16_t (fp16) or float.
+// bt is null where the device has no memory left for them: the caller takes a
+// kernel without.  T: uint16_t (fp16) or float.
 template <typename T>
 struct PaddedB {
     const T* bt = nullptr;

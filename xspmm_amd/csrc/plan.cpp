@@ -264,6 +264,7 @@ public:
         const I* rmap = clustered_ ? perm_.as<I>() : nullptr;
         TempArena arena(s);
         const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K_, N, 0, arena, s);
+        if (!pb.bt) return false;
         if (!spmm_f16_packed<I>(M_, K_, Mb_, poff_.as<int64_t>(), pa_.as<void>(), prow_.as<uint32_t>(), pb.bt, C,
                                 pb.Np, order, rmap, s, N, pb.marks))
             return false;

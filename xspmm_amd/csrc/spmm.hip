@@ -2061,7 +2061,8 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     p.Np = (N + V - 1) / V * V;
     const bool copy = p.Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
     const PadPieces at = pad_pieces(sizeof(T), K, p.Np, copy, order_rows);
-    char* const base = static_cast<char*>(arena.take(at.end));
+    char* const base = static_cast<char*>(arena.take(at.end, true));
+    if (!base) return p;
     const int64_t vecs = K * (p.Np / V);
     const dim3 wgs((unsigned)std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads)));
     const U* src = reinterpret_cast<const U*>(B);
@@ -2103,12 +2104,109 @@ bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
     return tiled <= per_block * (double)Kb * std::max(1.0, 0.35 + 0.49 * wgs) + 18.0;
 }
 
+// What a Tier-1 product runs and the temporaries it takes, from sizes, types and
+// alignment alone, never from the memory at hand: calls given the same pad_limit
+// run the same kernels (bcsr_spmm_launch), and bcsr_spmm_scratch says beforehand
+// what they will take.
+// pad_limit: bytes that a padded copy of B, its marks and an order may take.
+enum class F16Kernel { kTiled, kBatch, kGather, kPanel };
+struct F16Route {
+    F16Kernel kernel;
+    bool padded = false;     // on pad_b's copy, or with its marks (kTiled, kBatch)
+    bool own_order = false;  // kBatch: the launcher orders the rows
+    size_t bytes = 0;
+};
+size_t f16_panel_bytes(int64_t Kb, int64_t N)
+{
+    return (size_t)(Kb > 0 ? Kb : 1) * (size_t)((N + 15) / 16 * 16) * 16 * sizeof(uint16_t);
+}
+F16Route f16_route(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool have_order,
+                   size_t pad_limit)
+{
+    const Fp16Kernel choice = fp16_kernel_choice();
+    const bool batches = choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch;
+    // batch and gather paths: byte offsets into B, and a wave's A range,
+    // fit 32 bits; B row indices fit 24 bits
+    auto offsets32 = [&](int64_t n) {
+        return K * n * 2 <= (int64_t(1) << 31) && n < (int64_t(1) << 22) && Kb < (int64_t(1) << 20);
+    };
+    const int64_t Np = (N + 7) / 8 * 8;
+    // every block present: GEMM-tiled kernel (matrix-core bound); its tiles are
+    // one grid dimension and take N that the batches do not
+    const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, Np);
+    const bool tiled = full && (!offsets32(Np) || dense_f16_pays(Mb, Kb, N));
+    const bool ordered = spmm_order_wanted(Mb);
+    const size_t order_bytes = (size_t)Mb * sizeof(int32_t);
+    if (tiled && N % 8 == 0) return {F16Kernel::kTiled};
+    // more block-rows than resident workgroups (4 per CU on 256 CUs,
+    // times two): dispatch the longest rows first
+    if (batches && N % 8 == 0 && offsets32(N) && !full) {
+        const bool own = ordered && !have_order;
+        return {F16Kernel::kBatch, false, own, own ? order_bytes : 0};
+    }
+    // N % 8 != 0: rows of B off 16 bytes.  The kernels above, on a padded
+    // copy of B, instead of the panel kernel below, which repacks B just
+    // the same and whose waves then walk whole block-rows alone.  Faster
+    // on every matrix and N tried (1 .. 127): 16384^2 templates, N = 17,
+    // 342 -> 77 us; 50000^2 power-law graph, N = 1, 867 -> 104 us;
+    // 5003 x 4999 at 2 %, N = 31, 96 -> 29 us; 8192^2 with 5 % of the
+    // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
+    // range come here with any N: it multiplies every column of a block,
+    // and so must the batches where B holds an Inf or NaN.
+    // (Beyond the limit N % 8 != 0 repacks panels, unless those exceed it too.)
+    // An order counts whether or not the caller has one: it decides no kernel.
+    const size_t panel_bytes = f16_panel_bytes(Kb, N);
+    if (batches && (N % 8 != 0 || full) && offsets32(Np)) {
+        auto bytes = [&](bool order) { return pad_pieces(2, K, Np, N % 8 != 0, order ? Mb : 0).end; };
+        const bool rows = !tiled && ordered;
+        if (bytes(rows) <= pad_limit || (N % 8 != 0 && panel_bytes > pad_limit)) {
+            const bool own = rows && !have_order;
+            return {tiled ? F16Kernel::kTiled : F16Kernel::kBatch, true, own, bytes(own)};
+        }
+    }
+    if (full && N % 8 == 0) return {F16Kernel::kTiled};  // the marks and an order exceed the limit
+    if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32(N)) return {F16Kernel::kGather};
+    return {F16Kernel::kPanel, false, false, panel_bytes};
+}
+
+struct F32Route {
+    F32Kernel kernel = F32Kernel::kTile;
+    bool padded = false;     // N % 4 != 0, or B or C off 16 bytes: on pad_b's copy
+    bool own_order = false;
+    bool whole = false;      // kTile: B within a buffer resource (f32_short_wanted)
+    size_t bytes = 0;
+};
+// contiguous: every block-row is one run of block columns.
+F32Route f32_route(int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, const void* B, const void* C,
+                   bool contiguous, bool have_order, size_t pad_limit)
+{
+    F32Route r;
+    const bool aligned = spmm_f32_batch_covers(K, Kb, N, B, C);
+    const int64_t Np = (N + 3) / 4 * 4;
+    r.whole = f32_short_wanted(Kb, N);
+    const bool share = spmm_band_f32_covers(K, Kb, Mb, Np, nullptr, nullptr);
+    const char* forced = std::getenv("XSPMM_F32_KERNEL");
+    if ((aligned || spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr)) &&
+        !(forced && std::strcmp(forced, "tile") == 0))
+        r.kernel = forced && std::strcmp(forced, "batch") == 0
+                       ? F32Kernel::kBatch
+                       : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, r.whole, share, contiguous);
+    const bool copy = Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
+    auto pad_bytes = [&](bool order) { return pad_pieces(4, K, Np, copy, order ? Mb : 0).end; };
+    r.padded = r.kernel != F32Kernel::kTile && !aligned;
+    const bool ordered = spmm_order_wanted(Mb);
+    if (r.padded && pad_bytes(r.kernel == F32Kernel::kBatch && ordered) > pad_limit) {
+        r.kernel = F32Kernel::kTile;
+        r.padded = false;
+    }
+    r.own_order = r.kernel != F32Kernel::kShared && (r.kernel == F32Kernel::kBatch || r.whole) && !have_order && ordered;
+    r.bytes = r.padded ? pad_bytes(r.own_order) : r.own_order ? (size_t)Mb * sizeof(int32_t) : 0;
+    return r;
+}
+
 // The Tier-1 launcher: kernel choice as described at the top of this file;
-// temporaries (the dispatch order, repacked B panels) come from `arena`.
-// contiguous (fp32): every block-row is one run of block columns.
-// pad_limit: the temporaries a padded copy of B may take.  The choice depends on
-// sizes, types and alignment alone, never on the room an arena has left, so calls
-// given the same limit run the same kernels.
+// temporaries (the dispatch order, a padded copy of B, repacked B panels) come
+// from `arena`.  contiguous (fp32): every block-row is one run of block columns.
 template <typename T, typename I>
 bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                       const I* bci, const T* bvals, const T* B, float* C, int64_t N,
@@ -2128,28 +2226,15 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
     if constexpr (sizeof(T) == 2) {
         const uint16_t* v = reinterpret_cast<const uint16_t*>(bvals);
         const uint16_t* b = reinterpret_cast<const uint16_t*>(B);
-        // batch and gather paths: byte offsets into B, and a wave's A range,
-        // fit 32 bits; B row indices fit 24 bits
-        const Fp16Kernel choice = fp16_kernel_choice();
-        // every block present: GEMM-tiled kernel (matrix-core bound)
-        const bool full = choice == Fp16Kernel::kAuto && spmm_dense_f16_covers(M, K, Mb, Kb, nnzb, (N + 7) / 8 * 8);
-        // (its tiles are one grid dimension and take N that the batches do not)
-        const int64_t Np = (N + 7) / 8 * 8;
-        const bool batchable = K * Np * 2 <= (int64_t(1) << 31) && Np < (int64_t(1) << 22) && Kb < (int64_t(1) << 20);
-        const bool tiled = full && (!batchable || dense_f16_pays(Mb, Kb, N));
-        if (tiled && N % 8 == 0)
+        const F16Route r = f16_route(M, K, Mb, Kb, nnzb, N, order_in != nullptr, pad_limit);
+        if (r.kernel == F16Kernel::kTiled && !r.padded)
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
-        const bool offsets32 = K * N * 2 <= (int64_t(1) << 31) && N < (int64_t(1) << 22) &&
-                               Kb < (int64_t(1) << 20);
         const int64_t chunks = (N + 127) / 128;
         if (chunks > 65535) throw std::invalid_argument("xSpMM: N too large.");
         const dim3 ggrid((unsigned)Mb, (unsigned)chunks);
-        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && N % 8 == 0 &&
-            offsets32 && !full) {
-            // more block-rows than resident workgroups (4 per CU on 256 CUs,
-            // times two): dispatch the longest rows first
+        if (r.kernel == F16Kernel::kBatch && !r.padded) {
             const int32_t* order = order_in;
-            if (!order && spmm_order_wanted(Mb)) {
+            if (r.own_order) {
                 int32_t* buf = arena.take_as<int32_t>((size_t)Mb);
                 spmm_dispatch_order<I>(brp, Mb, buf, s);
                 order = buf;
@@ -2177,26 +2262,14 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             XSPMM_LAUNCH_CHECK();
             return true;
         }
-        // N % 8 != 0: rows of B off 16 bytes.  The kernels above, on a padded
-        // copy of B, instead of the panel kernel below, which repacks B just
-        // the same and whose waves then walk whole block-rows alone.  Faster
-        // on every matrix and N tried (1 .. 127): 16384^2 templates, N = 17,
-        // 342 -> 77 us; 50000^2 power-law graph, N = 1, 867 -> 104 us;
-        // 5003 x 4999 at 2 %, N = 31, 96 -> 29 us; 8192^2 with 5 % of the
-        // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
-        // range come here with any N: it multiplies every column of a block,
-        // and so must the batches where B holds an Inf or NaN.
-        // (Beyond the limit N % 8 != 0 repacks panels, unless those exceed it too.)
-        const size_t panel_bytes = (size_t)(Kb > 0 ? Kb : 1) * (size_t)(ntiles64 * 16) * 16 * sizeof(uint16_t);
-        // An order counts whether or not the caller has one: it decides no kernel.
-        const bool own_order = !tiled && !order_in && spmm_order_wanted(Mb);
-        const size_t pad_bytes = pad_pieces(2, K, Np, N % 8 != 0, !tiled && spmm_order_wanted(Mb) ? Mb : 0).end;
-        if ((choice == Fp16Kernel::kAuto || choice == Fp16Kernel::kBatch) && (N % 8 != 0 || full) && batchable &&
-            (pad_bytes <= pad_limit || (N % 8 != 0 && panel_bytes > pad_limit))) {
-            const PaddedB<uint16_t> pb = pad_b<uint16_t>(b, K, N, own_order ? Mb : 0, arena, s);
-            if (tiled) return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
+        const PaddedB<uint16_t> pb =
+            r.padded ? pad_b<uint16_t>(b, K, N, r.own_order ? Mb : 0, arena, s) : PaddedB<uint16_t>{};
+        if (pb.bt) {
+            const int64_t Np = pb.Np;
+            if (r.kernel == F16Kernel::kTiled)
+                return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, pb.bt, C, Np, s, row_map, N);
             const int32_t* order = order_in;
-            if (own_order) {
+            if (r.own_order) {
                 spmm_dispatch_order<I>(brp, Mb, pb.order, s);
                 order = pb.order;
             }
@@ -2219,10 +2292,10 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             XSPMM_LAUNCH_CHECK();
             return true;
         }
-        if (full && N % 8 == 0)  // the marks and an order exceed the limit
+        if (r.padded && N % 8 == 0)  // a full grid, no memory for the marks
             return bcsr_spmm_dense_f16<I>(M, K, Mb, Kb, nnzb, brp, bci, v, b, C, N, s, row_map);
         if (row_map) return false;  // the other fp16 kernels store rows in place
-        if (choice == Fp16Kernel::kGather && N % 2 == 0 && offsets32) {
+        if (r.kernel == F16Kernel::kGather) {
             if (N <= 64)
                 hipLaunchKernelGGL((spmm_f16_gather_kernel<I, 4, kGatherRows>), ggrid, dim3(256), 0, s, brp, bci,
                                    v, b, C, M, K, N, Kb);
@@ -2233,7 +2306,7 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             return true;
         }
         const int64_t Nw = ntiles64 * 16;
-        uint16_t* bt = static_cast<uint16_t*>(arena.take(panel_bytes));
+        uint16_t* bt = static_cast<uint16_t*>(arena.take(f16_panel_bytes(Kb, N)));
         if (Kb > 0) {
             const int64_t per_kb = Nw * 2;
             const dim3 pg((unsigned)((per_kb + 255) / 256), (unsigned)(Kb < 65535 ? Kb : 65535));
@@ -2258,45 +2331,27 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
     } else {
         const float* v = reinterpret_cast<const float*>(bvals);
         const float* b = reinterpret_cast<const float*>(B);
-        const bool aligned = spmm_f32_batch_covers(K, Kb, N, B, C);
-        const int64_t Np = (N + 3) / 4 * 4;
-        const bool whole = f32_short_wanted(Kb, N);
-        const bool share = spmm_band_f32_covers(K, Kb, Mb, Np, nullptr, nullptr);
-        const char* forced = std::getenv("XSPMM_F32_KERNEL");
-        F32Kernel kernel = F32Kernel::kTile;
-        if ((aligned || spmm_f32_batch_covers(K, Kb, Np, nullptr, nullptr)) &&
-            !(forced && std::strcmp(forced, "tile") == 0))
-            kernel = forced && std::strcmp(forced, "batch") == 0
-                         ? F32Kernel::kBatch
-                         : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, whole, share, contiguous);
-        if (kernel != F32Kernel::kTile && !aligned) {
-            const bool copy = Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
-            const int64_t order_rows = kernel == F32Kernel::kBatch && spmm_order_wanted(Mb) ? Mb : 0;
-            if (pad_pieces(4, K, Np, copy, order_rows).end > pad_limit) kernel = F32Kernel::kTile;
-        }
-        const bool order_here = kernel != F32Kernel::kShared && !order_in && spmm_order_wanted(Mb);
+        const F32Route r = f32_route(K, Mb, Kb, nnzb, N, B, C, contiguous, order_in != nullptr, pad_limit);
         auto shared = [&](const float* bb, int64_t n, int64_t nc) {
             return contiguous
                        ? bcsr_spmm_band_f32<I>(M, K, Mb, Kb, brp, bci, v, bb, C, n, row_map, nnzb, s, nc)
                        : bcsr_spmm_full_f32<I>(M, K, Mb, Kb, brp, bci, v, bb, C, n, row_map, s, nc);
         };
         auto order_with = [&](int32_t* buf) -> const int32_t* {
-            if (!order_here) return order_in;
+            if (!r.own_order) return order_in;
             spmm_dispatch_order<I>(brp, Mb, buf, s);
             return buf;
         };
-        auto order_rows = [&]() { return order_with(order_here ? arena.take_as<int32_t>((size_t)Mb) : nullptr); };
-        if (kernel != F32Kernel::kTile && aligned) {
-            if (kernel == F32Kernel::kShared) return shared(b, N, 0);
-            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, b, C, N, order_rows(), row_map, s);
+        if (r.kernel != F32Kernel::kTile && !r.padded) {
+            if (r.kernel == F32Kernel::kShared) return shared(b, N, 0);
+            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, b, C, N,
+                                   order_with(static_cast<int32_t*>(arena.take(r.bytes))), row_map, s);
             return true;
         }
-        if (kernel != F32Kernel::kTile) {
-            // N % 4 != 0, or B or C off 16 bytes: the same kernels on a padded
-            // copy of B
-            const PaddedB<float> pb = pad_b<float>(b, K, N, order_here ? Mb : 0, arena, s);
-            if (kernel == F32Kernel::kShared) return shared(pb.bt, Np, N);
-            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, Np, order_with(pb.order), row_map, s, N,
+        const PaddedB<float> pb = r.padded ? pad_b<float>(b, K, N, r.own_order ? Mb : 0, arena, s) : PaddedB<float>{};
+        if (pb.bt) {
+            if (r.kernel == F32Kernel::kShared) return shared(pb.bt, pb.Np, N);
+            bcsr_spmm_f32_batch<I>(M, K, Mb, Kb, brp, bci, v, pb.bt, C, pb.Np, order_with(pb.order), row_map, s, N,
                                    pb.marks);
             return true;
         }
@@ -2304,12 +2359,14 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
         const int64_t gy = (ntiles + ntw - 1) / ntw;
         if (gy > 65535) throw std::invalid_argument("xSpMM: N too large.");
         const dim3 fgrid((unsigned)Mb, (unsigned)gy);
-        if (whole) {
+        if (r.whole) {
             // blocks beyond the 256 MB last-level cache are read past it
             // (775 MB, N = 4: 150 -> 141 us; 100 MB, N = 16: 26 -> 30)
             const bool stream = nnzb > (int64_t(1) << 18);
-            const int32_t* order =
-                !order_here || arena.fits((size_t)Mb * sizeof(int32_t)) ? order_rows() : nullptr;
+            // (an allocation-free call's array may not hold an order: it decides nothing)
+            const int32_t* order = order_in;
+            if (r.own_order && !r.padded && arena.fits(r.bytes))
+                order = order_with(static_cast<int32_t*>(arena.take(r.bytes)));
             auto launch = [&](auto k) {
                 hipLaunchKernelGGL(k, fgrid, dim3(64 * kF32ShortWaves), 0, s, brp, bci, v, b, C, M, K, N, Kb,
                                    ntiles, order, row_map);
@@ -2413,6 +2470,14 @@ void bcsr_spmm_band(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
     bcsr_spmm<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, s, kNoAllocScratchBytes);
 }
 
+namespace {
+// whether a band's product may take the fp32 band kernel (on B or a padded copy)
+bool f32_contiguous(int64_t K, int64_t Kb, int64_t Mb, int64_t N, bool band)
+{
+    return band && spmm_band_f32_covers(K, Kb, Mb, (N + 3) / 4 * 4, nullptr, nullptr);
+}
+}  // namespace
+
 template <typename T, typename I>
 void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp, const I* bci,
                     const T* bvals, const T* B, float* C, int64_t N, const int32_t* order, bool band, void* scratch,
@@ -2429,23 +2494,26 @@ void bcsr_spmm_auto(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, 
             const int64_t Np = (N + 7) / 8 * 8;
             if (spmm_band_f16_covers(K, Kb, Mb, Np)) {
                 const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K, N, 0, arena, s);
-                if (bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, pb.bt, C, Np, nullptr, s, N)) return;
+                if (pb.bt && bcsr_spmm_band_f16<I>(M, K, Mb, Kb, brp, bci, bvals, pb.bt, C, Np, nullptr, s, N)) return;
             }
         }
     }
-    const bool contiguous = sizeof(T) == 4 && band && spmm_band_f32_covers(K, Kb, Mb, (N + 3) / 4 * 4, nullptr, nullptr);
+    const bool contiguous = sizeof(T) == 4 && f32_contiguous(K, Kb, Mb, N, band);
     (void)bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order, nullptr, arena, s, SIZE_MAX,
                                  contiguous);
 }
 
-size_t bcsr_spmm_scratch(int value_bytes, int64_t K, int64_t Mb, int64_t N)
+size_t bcsr_spmm_scratch(int value_bytes, int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const void* B,
+                         const void* C, int64_t N, bool ordered, bool band)
 {
-    const int64_t V = 16 / value_bytes;
-    Carve cv;  // as pad_b
-    cv.take(kPadMarks);
-    cv.take((size_t)(K > 0 ? K : 1) * (size_t)((N + V - 1) / V * V) * (size_t)value_bytes);
-    cv.take(spmm_order_wanted(Mb) ? (size_t)Mb * sizeof(int32_t) : 0);
-    return cv.end;
+    check_shape(M, K, Mb, Kb, nnzb, N);
+    if (M == 0 || N == 0 || Mb == 0) return 0;
+    if (value_bytes == 2) {
+        const int64_t Np = (N + 7) / 8 * 8;
+        if (band && spmm_band_f16_covers(K, Kb, Mb, Np)) return N % 8 ? pad_pieces(2, K, Np, true, 0).end : 0;
+        return f16_route(M, K, Mb, Kb, nnzb, N, ordered, SIZE_MAX).bytes;
+    }
+    return f32_route(K, Mb, Kb, nnzb, N, B, C, f32_contiguous(K, Kb, Mb, N, band), ordered, SIZE_MAX).bytes;
 }
 
 #define XSPMM_SPMM_BAND(T, I)                                                                          \
