@@ -1,0 +1,50 @@
+"""Prepared products against the pipeline, bit for bit, where the plan multiplies a
+padded copy of B or stores into a C off 16 bytes: real-valued operands, so that
+another kernel's order of sums would show."""
+from __future__ import annotations
+
+import pytest
+
+import xspmm_amd as X
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need an MI355X (torch.cuda.is_available() is False)")
+    X.load()
+    return torch
+
+
+def csr(torch, M, K, keys, dtype):
+    rp = torch.searchsorted(keys, torch.arange(M + 1, device="cuda:0") * K)
+    vals = torch.randn(keys.numel(), device="cuda:0").to(dtype)
+    return X.CSRMatrix(M, K, rp.int(), (keys % K).int(), vals)
+
+
+def full_blocks(torch, M, K, share):
+    Mb, Kb = M // 16, K // 16
+    b = (torch.rand(Mb * Kb, device="cuda:0") < share).nonzero().reshape(-1)
+    r = torch.arange(16, device="cuda:0")
+    keys = ((b // Kb * 16)[:, None, None] + r[None, :, None]) * K + (b % Kb * 16)[:, None, None] + r[None, None, :]
+    return keys.reshape(-1).sort().values
+
+
+@pytest.mark.parametrize("N", [64, 200])
+def test_f32_clustered_plan_with_c_off_16_bytes(torch, N):
+    """Blocks that the packed form would not shrink: the plan's product goes through
+    its workspace, as the pipeline's does, and keeps its kernel."""
+    M = K = 9216
+    A = csr(torch, M, K, full_blocks(torch, M, K, 0.02), torch.float32)
+    plan = X.SpMMPlan(A, optimize_pattern=True)
+    assert plan.packed_batches == -1
+    B = torch.randn((K, N), device="cuda:0")
+    want = X.spmm_pipeline(A, B, optimize_pattern=True)[0]
+    for off in (0, 1, 2):
+        guard = torch.full((M * N + 8,), -7.0, device="cuda:0")
+        C = plan.execute(B, guard[off:off + M * N].view(M, N))
+        assert torch.equal(C, want), off
+        assert bool((guard[off + M * N:] == -7.0).all())

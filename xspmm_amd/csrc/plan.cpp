@@ -239,8 +239,11 @@ public:
                                B, C, N, order, nullptr, s);
             return;
         }
-        if (bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(),
-                               bvals_.as<T>(), B, C, N, order, perm_.as<I>(), s))
+        // A C off 16 bytes decides the fp32 kernel of N % 4 == 0, and the pipeline's
+        // permuted product is never off them: it goes through the workspace
+        const bool direct = sizeof(T) == 2 || N % 4 != 0 || (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+        if (direct && bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(),
+                                         bvals_.as<T>(), B, C, N, order, perm_.as<I>(), s))
             return;
         const size_t need = (size_t)M_ * (size_t)N * sizeof(float);
         if (ws_.size() < need) {
