@@ -48,3 +48,26 @@ def test_f32_clustered_plan_with_c_off_16_bytes(torch, N):
         C = plan.execute(B, guard[off:off + M * N].view(M, N))
         assert torch.equal(C, want), off
         assert bool((guard[off + M * N:] == -7.0).all())
+
+
+@pytest.mark.parametrize("cluster", [False, True])
+@pytest.mark.parametrize("M,K,per_row,columns", [(4099, 5003, 48, (129, 257, 260, 391)), (20000, 20000, 12, (3, 67, 127))])
+def test_packed_f16_plan_on_padded_b_equals_the_pipeline(torch, monkeypatch, M, K, per_row, columns, cluster):
+    """fp16, N % 8 != 0, on both sides of the line from which a plan multiplies its
+    packed batches on the padded copy (3 * 2^16 products of a block with 128
+    columns: 73 thousand blocks from N = 257, 222 thousand from N = 1): the
+    pipeline's C and that of a plan without packed batches."""
+    keys = torch.unique((torch.arange(M, device="cuda:0")[:, None] * K +
+                         torch.randint(K, (M, per_row), device="cuda:0")).reshape(-1))
+    A = csr(torch, M, K, keys, torch.float16)
+    packed = X.SpMMPlan(A, optimize_pattern=cluster)
+    monkeypatch.setenv("XSPMM_PLAN_PACK", "off")
+    plain = X.SpMMPlan(A, optimize_pattern=cluster)
+    monkeypatch.delenv("XSPMM_PLAN_PACK")
+    assert packed.packed_batches > 0 and plain.packed_batches == -1
+    for N in columns:
+        print(M, cluster, N, packed.num_blocks, flush=True)
+        B = torch.randn((K, N), device="cuda:0").half()
+        C = packed.execute(B)
+        assert torch.equal(C, plain.execute(B)), N
+        assert torch.equal(C, X.spmm_pipeline(A, B, optimize_pattern=cluster)[0]), N
