@@ -42,6 +42,13 @@ def test_bytes(vt, M, K, N, nnzb, want):
     assert scratch(vt, M, K, N, nnzb) == want
 
 
+def test_wide_b():
+    """fp32: no copy of a B with more than seven rows to a block, however many columns."""
+    for K, nnzb, pads in ((500000, 63733, False), (500000, 236400, True), (2000000, 15996, False),
+                          (2000000, 956467, True), (100000, 15922, True), (111454, 15922, True), (111455, 15922, False)):
+        assert (scratch(X.F32, 4000, K, 257, nnzb) > 0) is pads, (K, nnzb)
+
+
 def test_alignment_and_order():
     # B off 16 bytes is copied, C only marked
     assert scratch(X.F32, 16384, 16384, 128, 10 ** 6, b=4) == copy(4, 16384, 128)

@@ -1803,7 +1803,11 @@ constexpr int64_t kF32BatchMinGroups = 512;
 // 1.7 columns 137 -> 141); wider ones the batches from 512 workgroups; on a
 // padded copy of B, the batches from 2^18 products of a block with a tile (N =
 // 17: 300980 blocks 123 -> 80, 97367 blocks 43 -> 58; N = 33: 97367 blocks 71 ->
-// 58, 14465 blocks 14 -> 24).
+// 58, 14465 blocks 14 -> 24) unless B has more than seven rows to a block: the copy
+// reads and writes all of B at 2.3 TB/s, the tile kernel reads what the blocks
+// touch (N = 257, tile / batch: K = 500000, 63733 blocks 297 / 497, 236400 blocks
+// 962 / 629; K = 2000000, 15996 blocks 76 / 1767, 956467 blocks 4131 / 2450; K =
+// 100000, 15922 blocks 81 / 75).
 // whole: the tile kernel covers B (f32_short_wanted); share: kShared covers the
 // shape, whose 64-column chunks are one grid dimension (so are the tile kernel's
 // groups of tiles: neither reaches the last columns below 2^22).
@@ -1816,7 +1820,7 @@ constexpr int64_t kF32BatchMinGroups = 512;
 // 1024^2 80 % N = 127 49 / 8; 2048^2 80 % N = 511 103 / 49; 4096^2 50 % N = 129 70 /
 // 48, N = 257 77 / 79; 8192^2 5 % N = 65 17 / 22; 16384^2 50 % N = 127 276 / 527: the
 // choice is never the slower one by more than 1.23, and by 1 % on average.
-F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool aligned, bool whole,
+F32Kernel f32_kernel_choice(int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, bool aligned, bool whole,
                             bool share, bool contiguous)
 {
     const int64_t tiles = (N + 15) / 16;
@@ -1859,7 +1863,7 @@ F32Kernel f32_kernel_choice(int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, boo
     if (aligned)
         return (N > 8 || !whole) && Mb * ((N + 127) / 128) >= kF32BatchMinGroups ? F32Kernel::kBatch
                                                                                  : F32Kernel::kTile;
-    return N > 16 && nnzb * tiles >= (int64_t(1) << 18) ? F32Kernel::kBatch : F32Kernel::kTile;
+    return N > 16 && nnzb * tiles >= (int64_t(1) << 18) && 7 * nnzb >= K ? F32Kernel::kBatch : F32Kernel::kTile;
 }
 
 void check_shape(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N)
@@ -2190,7 +2194,7 @@ F32Route f32_route(int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N, c
         !(forced && std::strcmp(forced, "tile") == 0))
         r.kernel = forced && std::strcmp(forced, "batch") == 0
                        ? F32Kernel::kBatch
-                       : f32_kernel_choice(Mb, Kb, nnzb, N, aligned, r.whole, share, contiguous);
+                       : f32_kernel_choice(K, Mb, Kb, nnzb, N, aligned, r.whole, share, contiguous);
     const bool copy = Np != N || (reinterpret_cast<uintptr_t>(B) & 15) != 0;
     auto pad_bytes = [&](bool order) { return pad_pieces(4, K, Np, copy, order ? Mb : 0).end; };
     r.padded = r.kernel != F32Kernel::kTile && !aligned;
