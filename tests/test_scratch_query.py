@@ -43,9 +43,9 @@ def test_bytes(vt, M, K, N, nnzb, want):
 
 
 def test_wide_b():
-    """fp32: no copy of a B with more than seven rows to a block, however many columns."""
-    for K, nnzb, pads in ((500000, 63733, False), (500000, 236400, True), (2000000, 15996, False),
-                          (2000000, 956467, True), (100000, 15922, True), (111454, 15922, True), (111455, 15922, False)):
+    """fp32: no copy of a B with more than nine rows to a block, however many columns."""
+    for K, nnzb, pads in ((500000, 15987, False), (500000, 236400, True), (2000000, 15996, False),
+                          (2000000, 956467, True), (100000, 15922, True), (143298, 15922, True), (143299, 15922, False)):
         assert (scratch(X.F32, 4000, K, 257, nnzb) > 0) is pads, (K, nnzb)
 
 

@@ -69,46 +69,78 @@ __device__ __forceinline__ half8_t load_h8(const uint16_t* p)
 // ---------------------------------------------------------------------------
 // B (K x N) -> Bp (K x Np, Np = N rounded up to a 16-byte row multiple, the
 // added columns zero), for products whose rows do not start on 16 bytes: the
-// kernels that read B rows 16 bytes at a time then cover every N.  Bound by
-// memory (one read and one write of B): 3.2 us at 4999 x 31.
+// kernels that read B rows 16 bytes at a time then cover every N.
+// Bound by memory on a large B: 16-byte loads from any 2-byte boundary, four in
+// flight in each of 1024 threads per CU (the marks allow one workgroup each) reach
+// the rate of a plain copy (1 GB: 4.2 TB/s, torch's copy 4.7; 100 MB: 5.1), where
+// 256 threads with one vector of single loads each reached 2.1 (1 GB 977 -> 481 us,
+// 100 MB 75 -> 40).  Bound by latency up to one vector per thread of 256 workgroups:
+// 4999 x 31 3.2 us (0.2 TB/s), 3.5 with the wide loads, whose last vector of a row
+// takes both paths.
 // marks[0 .. 64) (256 bytes, all written): byte i is set when workgroup i of
 // the (at most 256) met an Inf or NaN.  Without COPY only the marks are made
 // (B's rows start on 16 bytes already).
 // ---------------------------------------------------------------------------
 constexpr int kPadMarks = 256;
-constexpr int kPadThreads = 256;
-template <typename U, bool COPY>
-__global__ __launch_bounds__(kPadThreads) void pad_b_kernel(const U* __restrict__ B, U* __restrict__ Bp,
-                                                            int64_t K, int64_t N, int64_t Np,
-                                                            unsigned char* __restrict__ marks)
+template <typename U, bool COPY, bool LARGE>
+__global__ __launch_bounds__(1024) void pad_b_kernel(const U* __restrict__ B, U* __restrict__ Bp,
+                                                     int64_t K, int64_t N, int64_t Np,
+                                                     unsigned char* __restrict__ marks)
 {
     constexpr int V = 16 / (int)sizeof(U);
     constexpr U kExp = sizeof(U) == 2 ? (U)0x7c00u : (U)0x7f800000u;
+    constexpr int kThreads = LARGE ? 1024 : 256;
+    constexpr int kAhead = LARGE ? 4 : 1;  // vectors in flight per thread
+    typedef U vec_t __attribute__((ext_vector_type(V)));
     // K * Np * sizeof(U) <= 2^31: vector counts fit 32 bits
     const uint32_t per_row = (uint32_t)(Np / V);
     const uint32_t total = (uint32_t)K * per_row;
+    const uint32_t step = gridDim.x * kThreads;
     bool bad = false;
-    for (uint32_t t = blockIdx.x * kPadThreads + threadIdx.x; t < total; t += gridDim.x * kPadThreads) {
-        const uint32_t k = t / per_row;
-        const int64_t c = (int64_t)(t - k * per_row) * V;
-        const U* src = B + k * N + c;
-        typedef U vec_t __attribute__((ext_vector_type(V)));
-        vec_t v;
-        if constexpr (COPY) {
+    for (uint32_t t0 = blockIdx.x * kThreads + threadIdx.x; t0 < total; t0 += kAhead * step) {
+        vec_t v[kAhead];
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[e] = c + e < N ? src[e] : (U)0;
-            *reinterpret_cast<vec_t*>(Bp + (size_t)t * V) = v;
-        } else {
-            v = *reinterpret_cast<const vec_t*>(src);
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t t = t0 + (uint32_t)u * step;
+            v[u] = vec_t{};
+            if (u > 0 && t >= total) continue;
+            const uint32_t k = t / per_row;
+            const int64_t c = (int64_t)(t - k * per_row) * V;
+            const U* src = B + k * N + c;
+            if (!COPY || (LARGE && c + V <= N)) {
+                __builtin_memcpy(&v[u], src, 16);  // (from any U boundary)
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[u][e] = c + e < N ? src[e] : (U)0;
+            }
         }
 #pragma unroll
-        for (int e = 0; e < V; ++e) bad |= (v[e] & kExp) == kExp;
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t t = t0 + (uint32_t)u * step;
+            if constexpr (COPY)
+                if (u == 0 || t < total) *reinterpret_cast<vec_t*>(Bp + (size_t)t * V) = v[u];
+#pragma unroll
+            for (int e = 0; e < V; ++e) bad |= (v[u][e] & kExp) == kExp;
+        }
     }
     const int any = __syncthreads_or(bad ? 1 : 0);
     if (threadIdx.x == 0) marks[blockIdx.x] = any ? 1 : 0;
     // the bytes of workgroups that the grid does not have
     if (blockIdx.x == 0)
-        for (int i = (int)gridDim.x + threadIdx.x; i < kPadMarks; i += kPadThreads) marks[i] = 0;
+        for (int i = (int)gridDim.x + threadIdx.x; i < kPadMarks; i += kThreads) marks[i] = 0;
+}
+
+template <typename U, bool COPY>
+void launch_pad_b(const U* B, U* Bp, int64_t K, int64_t N, int64_t Np, unsigned char* marks, hipStream_t s)
+{
+    const int64_t vecs = K * (Np / (16 / (int64_t)sizeof(U)));
+    const bool large = vecs > kPadMarks * 256;
+    const dim3 wgs((unsigned)std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + 255) / 256)));
+    if (large)
+        hipLaunchKernelGGL((pad_b_kernel<U, COPY, true>), wgs, dim3(1024), 0, s, B, Bp, K, N, Np, marks);
+    else
+        hipLaunchKernelGGL((pad_b_kernel<U, COPY, false>), wgs, dim3(256), 0, s, B, Bp, K, N, Np, marks);
+    XSPMM_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------------------
@@ -1803,11 +1835,10 @@ constexpr int64_t kF32BatchMinGroups = 512;
 // 1.7 columns 137 -> 141); wider ones the batches from 512 workgroups; on a
 // padded copy of B, the batches from 2^18 products of a block with a tile (N =
 // 17: 300980 blocks 123 -> 80, 97367 blocks 43 -> 58; N = 33: 97367 blocks 71 ->
-// 58, 14465 blocks 14 -> 24) unless B has more than seven rows to a block: the copy
-// reads and writes all of B at 2.3 TB/s, the tile kernel reads what the blocks
-// touch (N = 257, tile / batch: K = 500000, 63733 blocks 297 / 497, 236400 blocks
-// 962 / 629; K = 2000000, 15996 blocks 76 / 1767, 956467 blocks 4131 / 2450; K =
-// 100000, 15922 blocks 81 / 75).
+// 58, 14465 blocks 14 -> 24) unless B has more than nine rows to a block: the copy
+// reads and writes all of B, the tile kernel what the blocks touch (N = 257, tile
+// / batch: K = 500000, 15987 blocks 87 / 217, 63733 blocks 300 / 258; K = 2000000,
+// 15996 blocks 77 / 842, 239141 blocks 1082 / 1040, 956467 blocks 4120 / 1535).
 // whole: the tile kernel covers B (f32_short_wanted); share: kShared covers the
 // shape, whose 64-column chunks are one grid dimension (so are the tile kernel's
 // groups of tiles: neither reaches the last columns below 2^22).
@@ -1863,7 +1894,7 @@ F32Kernel f32_kernel_choice(int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int
     if (aligned)
         return (N > 8 || !whole) && Mb * ((N + 127) / 128) >= kF32BatchMinGroups ? F32Kernel::kBatch
                                                                                  : F32Kernel::kTile;
-    return N > 16 && nnzb * tiles >= (int64_t(1) << 18) && 7 * nnzb >= K ? F32Kernel::kBatch : F32Kernel::kTile;
+    return N > 16 && nnzb * tiles >= (int64_t(1) << 18) && 9 * nnzb >= K ? F32Kernel::kBatch : F32Kernel::kTile;
 }
 
 void check_shape(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, int64_t N)
@@ -1975,10 +2006,8 @@ bool all_finite_f16(const void* values, int64_t n, hipStream_t s)
     const int64_t vecs = n / 8;
     if (n % 8 != 0 || vecs > (int64_t(1) << 27)) return false;
     Scratch marks(kPadMarks, s);
-    hipLaunchKernelGGL((pad_b_kernel<uint16_t, false>), dim3(kPadMarks), dim3(kPadThreads), 0, s,
-                       static_cast<const uint16_t*>(values), static_cast<uint16_t*>(nullptr), vecs, (int64_t)8,
-                       (int64_t)8, marks.as<unsigned char>());
-    XSPMM_LAUNCH_CHECK();
+    launch_pad_b<uint16_t, false>(static_cast<const uint16_t*>(values), nullptr, vecs, 8, 8,
+                                  marks.as<unsigned char>(), s);
     uint32_t host[kPadMarks / 4];
     XSPMM_HIP_CHECK(hipMemcpyAsync(host, marks.get(), kPadMarks, hipMemcpyDeviceToHost, s));
     XSPMM_HIP_CHECK(hipStreamSynchronize(s));
@@ -2067,16 +2096,13 @@ PaddedB<T> pad_b(const T* B, int64_t K, int64_t N, int64_t order_rows, TempArena
     const PadPieces at = pad_pieces(sizeof(T), K, p.Np, copy, order_rows);
     char* const base = static_cast<char*>(arena.take(at.end, true));
     if (!base) return p;
-    const int64_t vecs = K * (p.Np / V);
-    const dim3 wgs((unsigned)std::max<int64_t>(1, std::min<int64_t>(kPadMarks, (vecs + kPadThreads - 1) / kPadThreads)));
     const U* src = reinterpret_cast<const U*>(B);
     U* bt = copy ? reinterpret_cast<U*>(base + at.bt) : nullptr;
     unsigned char* marks = reinterpret_cast<unsigned char*>(base + at.marks);
     if (copy)
-        hipLaunchKernelGGL((pad_b_kernel<U, true>), wgs, dim3(kPadThreads), 0, s, src, bt, K, N, p.Np, marks);
+        launch_pad_b<U, true>(src, bt, K, N, p.Np, marks, s);
     else
-        hipLaunchKernelGGL((pad_b_kernel<U, false>), wgs, dim3(kPadThreads), 0, s, src, bt, K, N, p.Np, marks);
-    XSPMM_LAUNCH_CHECK();
+        launch_pad_b<U, false>(src, bt, K, N, p.Np, marks, s);
     p.bt = copy ? reinterpret_cast<const T*>(bt) : B;
     p.marks = reinterpret_cast<const uint32_t*>(marks);
     p.order = reinterpret_cast<int32_t*>(base + at.order);
