@@ -756,6 +756,21 @@ __device__ __forceinline__ void batch_tile_store(const float4_t (&acc)[NT], unsi
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave * 2048 + (4 * g + r) * 128 + 16 * j + li] = acc[j][r];
     __syncthreads();
+    if ((N & 3) != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0) {
+        // rows of C off 16 bytes: neighbouring lanes store neighbouring columns
+        for (int t = threadIdx.x; t < 256 * NT; t += 64 * kBW) {
+            const int row = t / (16 * NT);
+            const int c = t % (16 * NT);
+            const int64_t grow = br * 16 + row;
+            if (grow >= M || n0 + c >= N) continue;
+            const int o = row * 128 + c;
+            float v = red[o];
+#pragma unroll
+            for (int w = 1; w < kBW; ++w) v += red[w * 2048 + o];
+            C[(row_map ? (int64_t)row_map[grow] : grow) * N + n0 + c] = v;
+        }
+        return;
+    }
     // 256 items of 8 columns (16 rows x 128 columns)
     for (int t = threadIdx.x; t < 256; t += 64 * kBW) {
         const int row = t >> 4;
@@ -773,7 +788,7 @@ __device__ __forceinline__ void batch_tile_store(const float4_t (&acc)[NT], unsi
             }
             const int64_t crow = row_map ? (int64_t)row_map[grow] : grow;
             float* dst = C + crow * N + n0 + c0;
-            if (n0 + c0 + 8 <= N && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
+            if (n0 + c0 + 8 <= N) {
                 *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
                 *reinterpret_cast<float4*>(dst + 4) = make_float4(out[4], out[5], out[6], out[7]);
             } else {
