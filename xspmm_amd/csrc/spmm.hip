@@ -2136,7 +2136,10 @@ namespace {
 //   batch: per block column, 0.055 (N <= 16) to 0.108 (N > 64) while its
 //          workgroups (block-rows x 128 columns) fit one to a CU, about half
 //          of that for each further one; and 18 us for the pass over B and
-//          the host's allocation of its marks.
+//          the host's allocation of its marks where N % 8 == 0.  Elsewhere both
+//          take a padded copy of B (950 blocks, N = 511, 27 us tiled, 11 in batches);
+//          1.2 is for long rows, where the batches are slower than their estimate
+//          (7000 x 8192, N = 257, 194 tiled, 230 in batches, estimated 164 and 158).
 // E.g. 4096 x 4096, N = 8: 84 us tiled, 17 in batches; N = 512: 95 and 67;
 // N = 1024: 96 and 118; 14336 x 4096, N = 128: 93 and 67; N = 256: 93 and 123.
 bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
@@ -2146,7 +2149,8 @@ bool dense_f16_pays(int64_t Mb, int64_t Kb, int64_t N)
     const double tiled = 0.32 * (double)Kb * std::ceil(tiles / kCus);
     const double per_block = N <= 16 ? 0.055 : N <= 32 ? 0.063 : N <= 64 ? 0.075 : 0.108;
     const double wgs = (double)Mb * (double)((N + 127) / 128) / kCus;
-    return tiled <= per_block * (double)Kb * std::max(1.0, 0.35 + 0.49 * wgs) + 18.0;
+    const double batch = per_block * (double)Kb * std::max(1.0, 0.35 + 0.49 * wgs);
+    return tiled <= (N % 8 == 0 ? batch + 18.0 : 1.2 * batch);
 }
 
 // What a Tier-1 product runs and the temporaries it takes, from sizes, types and
