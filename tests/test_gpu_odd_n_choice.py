@@ -1,5 +1,6 @@
 """fp16 products with N % 8 != 0: which kernel a grid takes, told by the order of its
-sums or the scratch, and the stores of C rows off 16 bytes."""
+sums, and the stores of C rows off 16 bytes.  Short rows of many columns keep panels
+of B, in Tier-1, plans and the pipeline alike."""
 from __future__ import annotations
 
 import ctypes as C
@@ -30,6 +31,40 @@ def csr(torch, M, K, per_row, seed=0):
     D = torch.zeros(M * K, device="cuda:0", dtype=torch.float64)
     D[keys] = vals.double()
     return X.CSRMatrix(M, K, rp.int(), (keys % K).int(), vals), D.view(M, K)
+
+
+@pytest.mark.parametrize("cluster", [False, True])
+@pytest.mark.parametrize("M,K,per_row", [(8205, 300, 6), (8205, 700, 2), (40000, 300, 3)])
+@pytest.mark.parametrize("N", [33, 65, 67, 129, 391, 1023])
+def test_short_rows(torch, M, K, per_row, N, cluster):
+    A, D = csr(torch, M, K, per_row)
+    blocks = X.csr_to_bcsr(A)
+    assert blocks.num_blocks < (20 if K == 300 else 32) * blocks.num_block_rows
+    B = torch.randn((K, N), device="cuda:0").half()
+    guard = torch.full((M * N + 64,), -7.0, device="cuda:0")
+    got = X.spmm(blocks, B, guard[:M * N].view(M, N))
+    # |sum error| <= n eps sum |a b|, n terms of a row's blocks
+    bound = K * 2.0 ** -24 * (D.abs() @ B.abs().double())
+    assert bool(((got - D @ B.double()).abs() <= bound).all())
+    assert bool((guard[M * N:] == -7.0).all())
+    plan = X.SpMMPlan(A, optimize_pattern=cluster)
+    assert torch.equal(plan.execute(B), X.spmm_pipeline(A, B, optimize_pattern=cluster)[0])
+
+
+def test_scratch_tells_panels_from_a_copy(torch):
+    """Panels hold 16 columns to a tile and whole blocks of rows, a copy 8 and marks."""
+    out = C.c_int64(0)
+
+    def scratch(Mb, nnzb, N, K=8000):
+        assert X.load().xspmm_bcsr_spmm_scratch(X.F16, Mb * 16, K, Mb, K // 16, nnzb, 0, 0, N, 1, 0,
+                                                C.byref(out)) == X.OK
+        return out.value
+
+    for N, panels in ((33, False), (64, False), (65, True), (257, True)):
+        copy, panel = -(-(256 + 8000 * (-(-N // 8) * 8) * 2) // 256) * 256, 8000 * (-(-N // 16) * 16) * 2
+        if N % 8:
+            assert scratch(900, 20 * 900 - 1, N) == (panel if panels else copy)
+            assert scratch(900, 20 * 900, N) == copy
 
 
 @pytest.mark.parametrize("M,K", [(811, 303), (305, 1003)])

@@ -42,7 +42,8 @@ namespace {
 // the same copy (from 23 us).  From 3 * 2^16 products of a block with 128 columns
 // (us, BCSR / packed: 47343 blocks, N = 257 27 / 28; 100926 blocks, N = 127 27 /
 // 27, N = 257 55 / 32; 553925 blocks, N = 3 100 / 29, N = 127 146 / 64; 756731
-// blocks, N = 127 91 / 39, N = 257 263 / 101).  C is the same bit for bit.
+// blocks, N = 127 91 / 39, N = 257 263 / 101).  C is the same bit for bit (so rows
+// that the BCSR form multiplies with panels, f16_short_rows, stay out).
 bool packed_pad_wanted(int64_t nnzb, int64_t N)
 {
     return nnzb * ((N + 127) / 128) >= 3 * (int64_t(1) << 16);
@@ -225,7 +226,7 @@ public:
                                               reinterpret_cast<const uint16_t*>(B), C, N, order,
                                               clustered_ ? perm_.as<I>() : nullptr, s))
                 return;
-            if (pads_ && packed_pad_wanted(nnzb_, N) &&
+            if (pads_ && packed_pad_wanted(nnzb_, N) && !f16_short_rows(Mb_, nnzb_, N) &&
                 execute_padded(reinterpret_cast<const uint16_t*>(B), C, N, order, s))
                 return;
         } else {

@@ -2165,6 +2165,19 @@ struct F16Route {
     bool own_order = false;  // kBatch: the launcher orders the rows
     size_t bytes = 0;
 };
+}  // namespace
+
+// Measured on 1549 grids (300 x 300 to 14336 x 8192, blocks full, at 20, 3 and 1 %,
+// N = 3 .. 1023; us, batches / panels): 14336 x 300 with 6 % of the blocks, N = 1023,
+// 37 / 18; 7000 x 2000 with 2 %, N = 257, 15 / 10; 14336 x 300 at 1 % (17 blocks a
+// row), N = 129, 18 / 14; 14336 x 1000 at 1 % (58), N = 129, 18 / 23; 300 x 2000 at
+// 1 %, N = 33, 11 / 31.  (Rows of many full blocks on tall grids would take panels
+// too, 14336 x 4096 with 60 %, N = 257, 137 / 85, but sizes do not tell them from
+// sparse blocks, which must not: at 3 % 0.7 to 1.05 of the panels' time.)
+bool f16_short_rows(int64_t Mb, int64_t nnzb, int64_t N) { return N > 64 && nnzb < 20 * Mb; }
+
+namespace {
+
 size_t f16_panel_bytes(int64_t Kb, int64_t N)
 {
     return (size_t)(Kb > 0 ? Kb : 1) * (size_t)((N + 15) / 16 * 16) * 16 * sizeof(uint16_t);
@@ -2199,7 +2212,8 @@ F16Route f16_route(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, i
     // on every matrix and N tried (1 .. 127): 16384^2 templates, N = 17,
     // 342 -> 77 us; 50000^2 power-law graph, N = 1, 867 -> 104 us;
     // 5003 x 4999 at 2 %, N = 31, 96 -> 29 us; 8192^2 with 5 % of the
-    // blocks, N = 7, 24 -> 23 us.  Full grids below the tiled kernel's
+    // blocks, N = 7, 24 -> 23 us; but not where rows are short and columns many
+    // (f16_short_rows).  Full grids below the tiled kernel's
     // range come here with any N: it multiplies every column of a block,
     // and so must the batches where B holds an Inf or NaN.
     // (Beyond the limit N % 8 != 0 repacks panels, unless those exceed it too.)
@@ -2208,7 +2222,9 @@ F16Route f16_route(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, i
     if (batches && (N % 8 != 0 || full) && offsets32(Np)) {
         auto bytes = [&](bool order) { return pad_pieces(2, K, Np, N % 8 != 0, order ? Mb : 0).end; };
         const bool rows = !tiled && ordered;
-        if (bytes(rows) <= pad_limit || (N % 8 != 0 && panel_bytes > pad_limit)) {
+        const bool panels = N % 8 != 0 && panel_bytes <= pad_limit;
+        if (!(panels && f16_short_rows(Mb, nnzb, N)) &&
+            (bytes(rows) <= pad_limit || (N % 8 != 0 && !panels))) {
             const bool own = rows && !have_order;
             return {tiled ? F16Kernel::kTiled : F16Kernel::kBatch, true, own, bytes(own)};
         }
