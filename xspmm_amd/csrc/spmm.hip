@@ -2428,8 +2428,11 @@ bool bcsr_spmm_launch(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb
             // blocks beyond the 256 MB last-level cache are read past it
             // (775 MB, N = 4: 150 -> 141 us; 100 MB, N = 16: 26 -> 30)
             const bool stream = nnzb > (int64_t(1) << 18);
-            // (an allocation-free call's array may not hold an order: it decides nothing)
-            const int32_t* order = order_in;
+            // An order of at most 2048 block-rows (neighbours on one XCD) is for the
+            // batches, which gather B row by row; it only unbalances whole blocks
+            // (4311^2 triangular, N = 60, 25 us in the rows' own order, 44 in it).
+            // (An allocation-free call's array may not hold an order: it decides nothing.)
+            const int32_t* order = spmm_order_wanted(Mb) ? order_in : nullptr;
             if (r.own_order && !r.padded && arena.fits(r.bytes))
                 order = order_with(static_cast<int32_t*>(arena.take(r.bytes)));
             auto launch = [&](auto k) {
