@@ -60,11 +60,12 @@ def test_scratch_tells_panels_from_a_copy(torch):
                                                 C.byref(out)) == X.OK
         return out.value
 
-    for N, panels in ((33, False), (64, False), (65, True), (257, True)):
+    for N, panels in ((33, False), (64, False), (65, False), (129, True), (257, True)):
         copy, panel = -(-(256 + 8000 * (-(-N // 8) * 8) * 2) // 256) * 256, 8000 * (-(-N // 16) * 16) * 2
         if N % 8:
             assert scratch(900, 20 * 900 - 1, N) == (panel if panels else copy)
             assert scratch(900, 20 * 900, N) == copy
+            assert scratch(300, 20 * 300 - 1, N) == copy  # at most 900 workgroups
 
 
 @pytest.mark.parametrize("M,K", [(811, 303), (305, 1003)])

@@ -315,7 +315,7 @@ void bcsr_rows_exact(int64_t M, int64_t K, int64_t Mb, int64_t Kb, const I* brp,
                      const uint16_t* B, float* C, int64_t N, int64_t nc, const I* row_map, const uint32_t* nonfinite,
                      hipStream_t s);
 // Whether fp16 products of N % 8 != 0 columns keep panels of B rather than batches on
-// a padded copy: fewer than 20 blocks to a row and more than 64 columns.
+// a padded copy: fewer than 20 blocks to a row, more than 64 columns, tall grids.
 bool f16_short_rows(int64_t Mb, int64_t nnzb, int64_t N);
 // Whether none of n fp16 values is an Inf or NaN (false as well when n is not a
 // multiple of 8, or beyond 2^30; synchronizes s).

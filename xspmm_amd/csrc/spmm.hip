@@ -2167,14 +2167,18 @@ struct F16Route {
 };
 }  // namespace
 
-// Measured on 1549 grids (300 x 300 to 14336 x 8192, blocks full, at 20, 3 and 1 %,
+// Measured on 1549 products (300 x 300 to 14336 x 8192, blocks full, at 20, 3 and 1 %,
 // N = 3 .. 1023; us, batches / panels): 14336 x 300 with 6 % of the blocks, N = 1023,
 // 37 / 18; 7000 x 2000 with 2 %, N = 257, 15 / 10; 14336 x 300 at 1 % (17 blocks a
 // row), N = 129, 18 / 14; 14336 x 1000 at 1 % (58), N = 129, 18 / 23; 300 x 2000 at
-// 1 %, N = 33, 11 / 31.  (Rows of many full blocks on tall grids would take panels
+// 1 %, N = 33, 11 / 31; 1605 x 3095 with 10 %, N = 260, 13 / 15 (batches while their
+// workgroups, four to a CU, all run at once).  (Rows of many full blocks on tall grids would take panels
 // too, 14336 x 4096 with 60 %, N = 257, 137 / 85, but sizes do not tell them from
 // sparse blocks, which must not: at 3 % 0.7 to 1.05 of the panels' time.)
-bool f16_short_rows(int64_t Mb, int64_t nnzb, int64_t N) { return N > 64 && nnzb < 20 * Mb; }
+bool f16_short_rows(int64_t Mb, int64_t nnzb, int64_t N)
+{
+    return N > 64 && nnzb < 20 * Mb && Mb * ((N + 127) / 128) >= 1024;
+}
 
 namespace {
 
