@@ -348,9 +348,11 @@ int xspmm_plan_create(int vtype, int itype, int64_t M, int64_t K, int64_t nnz, c
  * C.  Asynchronous on `stream`.  On the fp16 path with N % 8 == 0 it is one
  * kernel launch with the un-permutation fused into the store, which streams
  * the plan's packed column batches when it has them (larger fp16 products with
- * other N: on a padded copy of B, allocated on `stream`); otherwise it uses a
- * device workspace kept by the plan (grown, with a synchronization, when N
- * exceeds every earlier N).  Calls on one plan must not overlap.
+ * other N: on a padded copy of B).  What a product takes beside its operands (a
+ * padded copy of B and its marks, panels of B, a product in permuted order) is
+ * device memory kept by the plan, grown, with a synchronization, when a call
+ * needs more than every earlier one; while `stream` is being captured, a call
+ * that needs more allocates on it instead.  Calls on one plan must not overlap.
  */
 int xspmm_plan_execute(xspmm_plan_t plan, const void* B, float* C, int64_t N, void* stream);
 

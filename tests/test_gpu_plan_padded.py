@@ -71,3 +71,41 @@ def test_packed_f16_plan_on_padded_b_equals_the_pipeline(torch, monkeypatch, M, 
         C = packed.execute(B)
         assert torch.equal(C, plain.execute(B)), N
         assert torch.equal(C, X.spmm_pipeline(A, B, optimize_pattern=cluster)[0]), N
+
+
+@pytest.mark.parametrize("cluster", [False, True])
+@pytest.mark.parametrize("values,M,K,per_row,N", [
+    ("f32", 4099, 5003, 48, 67), ("f32", 4099, 5003, 48, 5), ("f16", 4099, 5003, 48, 31), ("f16", 4099, 5003, 48, 257),
+    ("f16", 515, 97, 0, 8), ("f16", 515, 97, 0, 33), ("f32", 2050, 1601, 0, 257), ("f16", 17000, 300, 2, 129)])
+def test_execute_allocates_nothing_again(torch, values, M, K, per_row, N, cluster):
+    """The second product of N columns takes nothing from the library's pool (nor
+    from hipMalloc), and can be captured: each replay gives the eager C."""
+    import ctypes as C
+    hip, pool = C.CDLL("libamdhip64.so.7"), C.c_void_p()
+    assert hip.hipDeviceGetDefaultMemPool(C.byref(pool), torch.cuda.current_device()) == 0
+    used, high, zero = C.c_uint64(0), C.c_uint64(0), C.c_uint64(0)
+    cols = (torch.randint(K, (M, per_row), device="cuda:0") if per_row else
+            (torch.arange(0, K, 16, device="cuda:0") + torch.arange(M, device="cuda:0")[:, None] % 16).clamp(max=K - 1))
+    keys = torch.unique((torch.arange(M, device="cuda:0")[:, None] * K + cols).reshape(-1))
+    dtype = torch.float16 if values == "f16" else torch.float32
+    plan = X.SpMMPlan(csr(torch, M, K, keys, dtype), optimize_pattern=cluster)
+    B = torch.randn((K, N), device="cuda:0").to(dtype)
+    want, out = plan.execute(B), torch.empty((M, N), device="cuda:0")
+    torch.cuda.synchronize()
+    assert hip.hipMemPoolGetAttribute(pool, 0x7, C.byref(used)) == 0  # hipMemPoolAttrUsedMemCurrent
+    assert hip.hipMemPoolSetAttribute(pool, 0x8, C.byref(zero)) == 0  # hipMemPoolAttrUsedMemHigh
+    free = torch.cuda.mem_get_info()[0]
+    plan.execute(B, out)
+    torch.cuda.synchronize()
+    assert hip.hipMemPoolGetAttribute(pool, 0x8, C.byref(high)) == 0
+    assert high.value <= used.value and torch.cuda.mem_get_info()[0] == free
+    assert torch.equal(out, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.execute(B, out)
+    for i in range(3):
+        B.mul_(-1)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, plan.execute(B)), i

@@ -267,11 +267,13 @@ void bcsr_spmm(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const
 // spmm_order_wanted) and an optional output row map: product row r is stored
 // in C row row_map[r] (row_map a permutation of [0, M)).  Returns false and
 // launches nothing when row_map is given but the selected kernel stores rows
-// in place; the caller then un-permutes a temporary.
+// in place; the caller then un-permutes a temporary.  arena: where temporaries come
+// from (null: stream-ordered allocations).
 template <typename T, typename I>
 bool bcsr_spmm_ex(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                   const I* bci, const T* bvals, const T* B, float* C, int64_t N,
-                  const int32_t* order, const I* row_map, hipStream_t s, size_t pad_limit = SIZE_MAX);
+                  const int32_t* order, const I* row_map, hipStream_t s, size_t pad_limit = SIZE_MAX,
+                  TempArena* arena = nullptr);
 // Tier-1 with the band kernel of T (uint16_t: fp16, float: fp32) where its
 // shape conditions hold, else as the C entry of bcsr_spmm.  The band
 // kernels are only correct when every block-row is one contiguous run of

@@ -21,9 +21,10 @@
 //     plan (it only grows) and is un-permuted into C.
 // C equals the pipeline's C bit for bit: the same kernels accumulate in the
 // same order, only the row a result is stored to differs.  execute() does not
-// allocate once the workspace is large enough (never, on the fused path), but
-// for the padded copies of B, which are stream-ordered allocations.
-// Calls on one plan must not overlap (they share the workspace).
+// allocate once the plan's memory is large enough for N: the workspace, and the
+// temporaries of products that take any (a padded copy of B, its marks).  Where
+// it is too small and the stream is being captured, those are stream-ordered
+// allocations.  Calls on one plan must not overlap (they share that memory).
 #include <cstdlib>
 #include <cstring>
 #include <limits>
@@ -37,12 +38,12 @@ namespace detail {
 namespace {
 
 // Whether an fp16 product with N % 8 != 0 takes the packed batches, on a padded
-// copy of B: three launches and an allocation (25 us of host time: B's copy, the
-// batches, rows_exact_kernel for an Inf or NaN in B) against the BCSR kernels on
-// the same copy (from 23 us).  From 3 * 2^16 products of a block with 128 columns
-// (us, BCSR / packed: 47343 blocks, N = 257 27 / 28; 100926 blocks, N = 127 27 /
-// 27, N = 257 55 / 32; 553925 blocks, N = 3 100 / 29, N = 127 146 / 64; 756731
-// blocks, N = 127 91 / 39, N = 257 263 / 101).  C is the same bit for bit (so rows
+// copy of B: three launches (B's copy, the batches, rows_exact_kernel for an Inf or
+// NaN in B) against the BCSR kernels on the same copy, two.  From 3 * 2^16 products
+// of a block with 128 columns (us, BCSR / packed, each with an allocation of about
+// 15 us that the plan's memory has since replaced: 47343 blocks, N = 257 27 / 28;
+// 100926 blocks, N = 127 27 / 27, N = 257 55 / 32; 553925 blocks, N = 3 101 / 33,
+// N = 127 146 / 64; 756731 blocks, N = 127 91 / 39, N = 257 263 / 101).  C is the same bit for bit (so rows
 // that the BCSR form multiplies with panels, f16_short_rows, stay out).
 bool packed_pad_wanted(int64_t nnzb, int64_t N)
 {
@@ -75,6 +76,27 @@ public:
         p_ = nullptr;
         n_ = 0;
         if (bytes) XSPMM_HIP_CHECK(hipMalloc(&p_, bytes));
+        n_ = bytes;
+    }
+    // At least `bytes` for work on s, keeping nothing of the old contents; left
+    // as it is while s is captured or when the device has no memory.
+    void reserve(size_t bytes, hipStream_t s) {
+        if (n_ >= bytes) return;
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {
+            (void)hipGetLastError();  // another thread captures: nothing may synchronize
+            return;
+        }
+        if (capturing != hipStreamCaptureStatusNone) return;
+        XSPMM_HIP_CHECK(hipStreamSynchronize(s));  // the old memory may be in use
+        reset(0);
+        const hipError_t e = hipMalloc(&p_, bytes);
+        if (e == hipErrorOutOfMemory) {
+            p_ = nullptr;
+            (void)hipGetLastError();  // reported by n_
+            return;
+        }
+        XSPMM_HIP_CHECK(e);
         n_ = bytes;
     }
     size_t size() const { return n_; }
@@ -235,38 +257,54 @@ public:
                                               N, order, clustered_ ? perm_.as<I>() : nullptr, s))
                 return;
         }
+        reserve_temps(B, C, N, s);
         if (!clustered_) {
-            bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(), bvals_.as<T>(),
-                               B, C, N, order, nullptr, s);
+            blocks(B, C, N, nullptr, s);
             return;
         }
         // A C off 16 bytes decides the fp32 kernel of N % 4 == 0, and the pipeline's
         // permuted product is never off them: it goes through the workspace
         const bool direct = sizeof(T) == 2 || N % 4 != 0 || (reinterpret_cast<uintptr_t>(C) & 15) == 0;
-        if (direct && bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(),
-                                         bvals_.as<T>(), B, C, N, order, perm_.as<I>(), s))
-            return;
+        if (direct && blocks(B, C, N, perm_.as<I>(), s)) return;
         const size_t need = (size_t)M_ * (size_t)N * sizeof(float);
         if (ws_.size() < need) {
             XSPMM_HIP_CHECK(hipStreamSynchronize(s));  // the old workspace may be in use
             ws_.reset(need);
         }
-        bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(), bvals_.as<T>(), B,
-                           ws_.as<float>(), N, order, nullptr, s);
+        blocks(B, ws_.as<float>(), N, nullptr, s);
         unpermute_dense<I>(ws_.as<float>(), C, perm_.as<I>(), M_, N, s);
+    }
+
+    // The BCSR form's product; false: its kernel stores rows in place.
+    bool blocks(const T* B, float* C, int64_t N, const I* row_map, hipStream_t s)
+    {
+        TempArena arena(tmp_.as<void>(), tmp_.size(), s, true);
+        return bcsr_spmm_ex<T, I>(M_, K_, Mb_, Kb_, nnzb_, brp_.as<I>(), bci_.as<I>(), bvals_.as<T>(), B, C, N,
+                                  order_.size() ? order_.as<int32_t>() : nullptr, row_map, s, SIZE_MAX, &arena);
+    }
+    // Room in tmp_ for what that product takes beside its operands.
+    void reserve_temps(const T* B, const float* C, int64_t N, hipStream_t s)
+    {
+        // (none where rows start on 16 bytes: the plan has its order; full fp16
+        // grids may take marks)
+        const bool aligned = sizeof(T) == 2 ? N % 8 == 0 && nnzb_ != Mb_ * Kb_
+                                            : N % 4 == 0 && ((reinterpret_cast<uintptr_t>(B) |
+                                                              reinterpret_cast<uintptr_t>(C)) & 15) == 0;
+        if (aligned) return;
+        tmp_.reserve(bcsr_spmm_scratch(sizeof(T), M_, K_, Mb_, Kb_, nnzb_, B, C, N, order_.size() != 0, false), s);
     }
 
     // fp16, N % 8 != 0: the packed product on a padded copy of B.  Where B holds an
     // Inf or NaN, which only the whole blocks carry to every row it reaches, the
-    // second kernel makes the product.  The copy is a stream-ordered allocation,
-    // as in the BCSR form.
+    // second kernel makes the product.
     bool execute_padded(const uint16_t* B, float* C, int64_t N, const int32_t* order, hipStream_t s)
     {
         const int64_t Np = (N + 7) / 8 * 8;
         if (Np >= (int64_t(1) << 22) || K_ * Np * 2 > (int64_t(1) << 31)) return false;
         if ((reinterpret_cast<uintptr_t>(B) & 15) != 0) return false;  // refused by the BCSR form
         const I* rmap = clustered_ ? perm_.as<I>() : nullptr;
-        TempArena arena(s);
+        reserve_temps(reinterpret_cast<const T*>(B), C, N, s);
+        TempArena arena(tmp_.as<void>(), tmp_.size(), s, true);
         const PaddedB<uint16_t> pb = pad_b<uint16_t>(B, K_, N, 0, arena, s);
         if (!pb.bt) return false;
         if (!spmm_f16_packed<I>(M_, K_, Mb_, poff_.as<int64_t>(), pa_.as<void>(), prow_.as<uint32_t>(), pb.bt, C,
@@ -288,6 +326,7 @@ private:
     bool clustered_ = false, packed_ = false;
     bool pads_ = false;  // packed, and taken for padded copies of B too
     DeviceBuffer perm_, brp_, bci_, bvals_, order_, ws_;
+    DeviceBuffer tmp_;  // a padded copy of B, its marks: execute()'s temporaries
     DeviceBuffer poff_, pa_, prow_;  // packed column batches
 };
 

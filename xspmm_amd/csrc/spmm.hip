@@ -2520,11 +2520,11 @@ void bcsr_spmm(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const
 template <typename T, typename I>
 bool bcsr_spmm_ex(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, const I* brp,
                   const I* bci, const T* bvals, const T* B, float* C, int64_t N,
-                  const int32_t* order_in, const I* row_map, hipStream_t s, size_t pad_limit)
+                  const int32_t* order_in, const I* row_map, hipStream_t s, size_t pad_limit, TempArena* arena)
 {
-    TempArena arena(s);
+    TempArena own(s);
     return bcsr_spmm_launch<T, I>(M, K, Mb, Kb, nnzb, brp, bci, bvals, B, C, N, order_in, row_map,
-                                  arena, s, pad_limit);
+                                  arena ? *arena : own, s, pad_limit);
 }
 
 template <typename T, typename I>
@@ -2617,7 +2617,7 @@ void bcsr_spmm_noalloc(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnz
 #define XSPMM_SPMM_EX(T, I)                                                                      \
     template bool bcsr_spmm_ex<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*,      \
                                      const I*, const T*, const T*, float*, int64_t,              \
-                                     const int32_t*, const I*, hipStream_t, size_t);             \
+                                     const int32_t*, const I*, hipStream_t, size_t, TempArena*); \
     template void bcsr_spmm<T, I>(int64_t, int64_t, int64_t, int64_t, int64_t, const I*,         \
                                   const I*, const T*, const T*, float*, int64_t, hipStream_t,    \
                                    size_t);                                                      \
