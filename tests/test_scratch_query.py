@@ -3,6 +3,7 @@ its sizes (no GPU is asked)."""
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import pytest
 
@@ -59,7 +60,16 @@ def test_alignment_and_order():
 
 
 def test_errors():
-    L, out = X.load(), C.c_int64(0)
-    assert L.xspmm_bcsr_spmm_scratch(X.F16, 16, 16, 1, 1, 1, 0, 0, 8, 0, 0, None) == X.ERR_INVALID
-    assert L.xspmm_bcsr_spmm_scratch(7, 16, 16, 1, 1, 1, 0, 0, 8, 0, 0, C.byref(out)) == X.ERR_INVALID
-    assert L.xspmm_bcsr_spmm_scratch(X.F16, 17, 16, 1, 1, 1, 0, 0, 8, 0, 0, C.byref(out)) == X.ERR_INVALID
+    # in a thread of its own: the library keeps the last error per thread
+    L, codes = X.load(), []
+
+    def calls():
+        out = C.c_int64(0)
+        codes.append(L.xspmm_bcsr_spmm_scratch(X.F16, 16, 16, 1, 1, 1, 0, 0, 8, 0, 0, None))
+        codes.append(L.xspmm_bcsr_spmm_scratch(7, 16, 16, 1, 1, 1, 0, 0, 8, 0, 0, C.byref(out)))
+        codes.append(L.xspmm_bcsr_spmm_scratch(X.F16, 17, 16, 1, 1, 1, 0, 0, 8, 0, 0, C.byref(out)))
+
+    t = threading.Thread(target=calls)
+    t.start()
+    t.join()
+    assert codes == [X.ERR_INVALID] * 3

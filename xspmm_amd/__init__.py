@@ -319,8 +319,10 @@ class BCSRMatrix:
         known, n = self._scratch
         if known != sizes:
             out = C.c_int64(0)
-            _check(load().xspmm_bcsr_spmm_scratch(vcode(vt), *sizes[1:6], b_at % 16, c_at % 16, N, int(ordered),
-                                                  int(band), C.byref(out)))
+            rc = _lib.xspmm_bcsr_spmm_scratch(_TYPE_CODES[vt] if vt in _TYPE_CODES else vcode(vt),
+                                              *sizes[1:], C.byref(out))
+            if rc != OK:
+                _check(rc)
             n = out.value
             self._scratch = (sizes, n)
         return n
