@@ -18,7 +18,9 @@
 //   spmm_f16_gather_kernel  per-pair masked B-row gather (XSPMM_SPMM_KERNEL=gather);
 //   pack_b_panels + spmm_f16_kernel  B repacked into 16-row panels laid out
 //                           [block_col][n][k16], two blocks per K = 32 operand:
-//                           B beyond 2^31 bytes, or no room for a padded copy.
+//                           N % 8 != 0 where rows are short and columns many
+//                           (f16_short_rows), B beyond 2^31 bytes, or a padded copy
+//                           beyond its limit or the device's memory.
 // N % 8 != 0 (fp32: N % 4 != 0, or B or C off 16 bytes): the same kernels on a
 // copy of B with padded rows (pad_b_kernel).
 //
