@@ -78,8 +78,8 @@ def test_packed_f16_plan_on_padded_b_equals_the_pipeline(torch, monkeypatch, M, 
     ("f32", 4099, 5003, 48, 67), ("f32", 4099, 5003, 48, 5), ("f16", 4099, 5003, 48, 31), ("f16", 4099, 5003, 48, 257),
     ("f16", 515, 97, 0, 8), ("f16", 515, 97, 0, 33), ("f32", 2050, 1601, 0, 257), ("f16", 17000, 300, 2, 129)])
 def test_execute_allocates_nothing_again(torch, values, M, K, per_row, N, cluster):
-    """The second product of N columns takes nothing from the library's pool (nor
-    from hipMalloc), and can be captured: each replay gives the eager C."""
+    """The second product of N columns takes nothing from the library's pool, and can
+    be captured (which refuses hipMalloc): each replay gives the eager C."""
     import ctypes as C
     hip, pool = C.CDLL("libamdhip64.so.7"), C.c_void_p()
     assert hip.hipDeviceGetDefaultMemPool(C.byref(pool), torch.cuda.current_device()) == 0
@@ -94,11 +94,10 @@ def test_execute_allocates_nothing_again(torch, values, M, K, per_row, N, cluste
     torch.cuda.synchronize()
     assert hip.hipMemPoolGetAttribute(pool, 0x7, C.byref(used)) == 0  # hipMemPoolAttrUsedMemCurrent
     assert hip.hipMemPoolSetAttribute(pool, 0x8, C.byref(zero)) == 0  # hipMemPoolAttrUsedMemHigh
-    free = torch.cuda.mem_get_info()[0]
     plan.execute(B, out)
     torch.cuda.synchronize()
     assert hip.hipMemPoolGetAttribute(pool, 0x8, C.byref(high)) == 0
-    assert high.value <= used.value and torch.cuda.mem_get_info()[0] == free
+    assert high.value <= used.value
     assert torch.equal(out, want)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):

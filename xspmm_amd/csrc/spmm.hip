@@ -1828,7 +1828,7 @@ int f32_tiles_per_group(int64_t Mb, int64_t ntiles)
 enum class F32Kernel { kTile, kBatch, kShared };
 constexpr int64_t kF32BatchMinGroups = 512;
 
-// The choice, from measured times (us).
+// The choice, from times (us) measured on the whole chip's 256 CUs.
 // Full grids and grids of contiguous block-rows, whose blocks are mostly full
 // (512 x 8192 to 14336 x 4096 full, bands of 5 to 90 % of 2984^2 to 16384^2; N =
 // 4 .. 1024), per block of an average block-row:
