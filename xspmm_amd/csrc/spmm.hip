@@ -2174,9 +2174,10 @@ struct F16Route {
 // 37 / 18; 7000 x 2000 with 2 %, N = 257, 15 / 10; 14336 x 300 at 1 % (17 blocks a
 // row), N = 129, 18 / 14; 14336 x 1000 at 1 % (58), N = 129, 18 / 23; 300 x 2000 at
 // 1 %, N = 33, 11 / 31; 1605 x 3095 with 10 %, N = 260, 13 / 15 (batches while their
-// workgroups, four to a CU, all run at once).  (Rows of many full blocks on tall grids would take panels
-// too, 14336 x 4096 with 60 %, N = 257, 137 / 85, but sizes do not tell them from
-// sparse blocks, which must not: at 3 % 0.7 to 1.05 of the panels' time.)
+// workgroups, four to a CU, all run at once).  (Rows of many full blocks on tall
+// grids would take panels too, 14336 x 4096 with 60 %, N = 257, 137 / 85, but sizes
+// do not tell them from sparse blocks, which must not: at 3 % 0.7 to 1.05 of the
+// panels' time.)
 bool f16_short_rows(int64_t Mb, int64_t nnzb, int64_t N)
 {
     return N > 64 && nnzb < 20 * Mb && Mb * ((N + 127) / 128) >= 1024;
@@ -2229,7 +2230,7 @@ F16Route f16_route(int64_t M, int64_t K, int64_t Mb, int64_t Kb, int64_t nnzb, i
         auto bytes = [&](bool order) { return pad_pieces(2, K, Np, N % 8 != 0, order ? Mb : 0).end; };
         const bool rows = !tiled && ordered;
         const bool panels = N % 8 != 0 && panel_bytes <= pad_limit;
-        if (!(panels && f16_short_rows(Mb, nnzb, N)) &&
+        if (!(panels && choice == Fp16Kernel::kAuto && f16_short_rows(Mb, nnzb, N)) &&
             (bytes(rows) <= pad_limit || (N % 8 != 0 && !panels))) {
             const bool own = rows && !have_order;
             return {tiled ? F16Kernel::kTiled : F16Kernel::kBatch, true, own, bytes(own)};
